@@ -8,7 +8,7 @@ import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
-SOURCES = [os.path.join(CSRC, "emx_attn.hip")]
+SOURCES = [os.path.join(CSRC, f) for f in ("emx_attn.hip", "emx_mfma.hip")]
 DEPENDS = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hpp", ".hip"))]
 OUT = os.path.join(_HERE, "_lib", "libemx_attn.so")
 
@@ -16,7 +16,6 @@ HIPCC_FLAGS = [
     "-O3",
     "--offload-arch=gfx950",
     "-std=c++17",
-    "-shared",
     "-fPIC",
     # no packed-fp32 VALU ops anywhere in device code
     "-Xclang",
@@ -40,11 +39,19 @@ def build_native(verbose: bool = False) -> str:
     """Compile the HIP library; always recompiles.  Returns the .so path."""
     os.makedirs(os.path.dirname(OUT), exist_ok=True)
     tmp = OUT + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, *SOURCES, "-o", tmp]
-    res = subprocess.run(cmd, capture_output=True, text=True)
+    objs = [os.path.join(os.path.dirname(OUT), os.path.basename(src) + ".o") for src in SOURCES]
+    cmds = [[hipcc(), *HIPCC_FLAGS, "-c", src, "-o", obj] for src, obj in zip(SOURCES, objs)]
+    # one compiler per translation unit, side by side
+    procs = [subprocess.Popen(c, stdout=subprocess.DEVNULL, stderr=subprocess.PIPE, text=True) for c in cmds]
+    errs = [p.communicate()[1] for p in procs]
+    link = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp]
+    for cmd, p, err in zip(cmds, procs, errs):
+        if p.returncode != 0:
+            raise RuntimeError(f"hipcc failed ({p.returncode}):\n{' '.join(cmd)}\n{err[-4000:]}")
+    res = subprocess.run(link, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{' '.join(cmd)}\n{res.stderr[-4000:]}")
+        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{' '.join(link)}\n{res.stderr[-4000:]}")
     if verbose:
-        print(" ".join(cmd))
+        print("\n".join(" ".join(c) for c in [*cmds, link]))
     os.replace(tmp, OUT)
     return OUT

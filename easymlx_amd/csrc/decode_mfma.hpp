@@ -1,0 +1,553 @@
+// Single-token paged decode over token-major caches [nb, bs, Hkv, D]:
+// unquantized fp16 / bf16 and FP8 (E4M3, one fp32 scale per page), head_dim 64,
+// 128 or 256, pages of a multiple of 8 tokens, any GQA ratio.  MFMA, split-K, one
+// launch.
+//
+// Replaces the reference's per-(seq, q_head) serial key loop
+// (lib/python/easymlx/operations/kernels/unified_attention.py:467-609, head-256
+// :611-775, FP8 :776-1268) and its split-K form (page_attention.py:1718-2059).
+//
+// Work: a unit is (sequence, kv head, up to 16 query heads), an item 128 tokens
+// of one unit (32 per wave).  Items are ordered unit-major and workgroup w of NWG
+// takes the range [w I / NWG, (w + 1) I / NWG); a unit inside one range goes
+// straight to the output, a cut one leaves an fp32 partial per workgroup, merged
+// by the workgroup that arrives last (counter per unit, zero before and after).
+//
+// Per 32-token item of a wave (lane l: i = l % 16, jj = l / 16)
+//   QK^T : v_mfma 16x16x32, A row i of sub-tile t = token 16 t + i; a load
+//          instruction reads 64 contiguous bytes of each of its 16 rows.  B column
+//          i = query head i.  Lane (h, jj) gets the scores of tokens 16 t + 4 jj + r.
+//   PV   : the k slot 8 jj + e is token 16 (e / 4) + 4 jj + e % 4, the eight scores
+//          lane (h, jj) holds, so P needs no lane exchange.  Lane (i, jj) loads dims
+//          D/16 i .. of those eight tokens (whole rows per 16 lanes) and sub-tile b
+//          takes dim D/16 i + b, picked by byte permutes.
+// K of the next item is loaded as soon as QK^T has consumed this one's registers,
+// V after PV: one register image, always in flight.
+//
+// Bound by HBM.  Against decode_split and its merge (VALU dot products, single-element
+// loads, two launches), which ran these shapes before: batch 32, contexts of 512 to
+// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 75.7 us, FP8 (136 MB)
+// 330 -> 51 us; one context of 1024, D 64, fp16: 38.4 -> 14.1 us.
+#pragma once
+
+#include "mfma_common.hpp"
+
+namespace emx {
+
+constexpr int kDecodeMfmaNT = 128;  // tokens per workgroup item
+
+struct DecodeMfmaArgs {
+  DecodeArgs d;      // kc / vc: the caches; nt = kDecodeMfmaNT; ws_cnt, ws_o [slot][hc][D], ws_ml [slot][hc][2]
+  int hc, nhc;       // query heads per unit (<= 16) and units per kv head
+  uint32_t inv_bs;   // ceil(2^32 / bs)
+};
+
+template <class C, int D>
+struct DecodeMfmaCfg {
+  static constexpr int EB = sizeof(typename C::ET);   // bytes per cache element
+  static constexpr int KS = D / 32;                   // QK^T k-slices
+  static constexpr int KL = D * EB / 64;              // 16-byte K loads per row (per lane)
+  static constexpr int SB = D / 16;                   // PV sub-tiles; dims a lane holds
+  static constexpr int VW = SB * EB / 4;              // V words a lane holds per token
+  static constexpr int RD = D < 128 ? D : 128;        // dims combined per round
+  static constexpr int XS = RD + 4;                   // LDS stride of a head's combined dims
+};
+
+template <class C, int D>
+struct DecodeMfmaLoads {
+  using P = DecodeMfmaCfg<C, D>;
+  uint32_t k[2][P::KL * 4];
+  uint32_t v[8][P::VW];
+};
+
+// MFMA operand of K k-slice w from the loaded words of one row.  16-bit: load w
+// holds dims 32 w + 8 jj ..; FP8: load w / 2 holds dims 64 (w / 2) + 16 jj .., its
+// halves the slices w, w + 1 (the query operand follows the same order).
+template <class C, int D>
+__device__ __forceinline__ typename C::Op k_operand(const uint32_t* k, const int w) {
+  if constexpr (C::kFp8) {
+    const uint32_t d0 = k[2 * w], d1 = k[2 * w + 1];
+    return as_h8(e4m3x2_to_h16x2(__builtin_amdgcn_perm(0u, d0, 0x0C010C00u)),
+                 e4m3x2_to_h16x2(__builtin_amdgcn_perm(0u, d0, 0x0C030C02u)),
+                 e4m3x2_to_h16x2(__builtin_amdgcn_perm(0u, d1, 0x0C010C00u)),
+                 e4m3x2_to_h16x2(__builtin_amdgcn_perm(0u, d1, 0x0C030C02u)));
+  } else {
+    return __builtin_bit_cast(typename C::Op, u32x4{k[4 * w], k[4 * w + 1], k[4 * w + 2], k[4 * w + 3]});
+  }
+}
+
+// PV operand of sub-tile b: element b of each of the eight tokens.
+template <class C, int VW>
+__device__ __forceinline__ typename C::Op v_operand(const uint32_t (&v)[8][VW], const int b) {
+  uint32_t w[4];
+  if constexpr (C::kFp8) {
+    const uint32_t sel = 0x0C000C00u | (uint32_t)(b & 3) | ((uint32_t)(4 + (b & 3)) << 16);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      w[m] = e4m3x2_to_h16x2(__builtin_amdgcn_perm(v[2 * m + 1][b >> 2], v[2 * m][b >> 2], sel));
+  } else {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      w[m] = __builtin_amdgcn_perm(v[2 * m + 1][b >> 1], v[2 * m][b >> 1], b & 1 ? 0x07060302u : 0x05040100u);
+  }
+  return __builtin_bit_cast(typename C::Op, u32x4{w[0], w[1], w[2], w[3]});
+}
+
+// O / L to four adjacent outputs (zeros for L = 0, a row without a live key);
+// true when a value of O is not finite.
+template <class QT>
+__device__ __forceinline__ bool write4(const f32x4 O, const float L, QT* out) {
+  struct alignas(8) Four {
+    QT x[4];
+  } v;
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    bad |= not_finite(O[k]);
+    from_f32(L > 0.f ? O[k] / L : 0.f, &v.x[k]);
+  }
+  *reinterpret_cast<Four*>(out) = v;
+  return bad;
+}
+
+template <class C, int D>
+__device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const int bid, const int nblocks) {
+  using P = DecodeMfmaCfg<C, D>;
+  typedef typename C::Op Op;
+  typedef typename C::QT QT;
+  const DecodeArgs& a = A.d;
+  constexpr int NT = kDecodeMfmaNT;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, jj = lane >> 4;
+  auto uru = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+
+  // LDS, carved from the shared arena
+  constexpr int oCum = 0, oKvl = lds_next(oCum, 4 * (kMaxSeqs + 1)), oQrw = lds_next(oKvl, 4 * kMaxSeqs);
+  constexpr int oXo = lds_next(oQrw, 4 * kMaxSeqs), oXml = lds_next(oXo, 4 * 4 * 16 * P::XS);
+  constexpr int oFlag = lds_next(oXml, 4 * 4 * 16 * 2), oEnd = lds_next(oFlag, 16);
+  static_assert(oEnd <= kArenaBytes, "LDS arena too small");
+  int(&cum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oCum);
+  int(&kvl)[kMaxSeqs] = lds_at<int[kMaxSeqs]>(oKvl);
+  int(&qrw)[kMaxSeqs] = lds_at<int[kMaxSeqs]>(oQrw);
+  float* xo = &lds_at<float>(oXo);      // [wave][head][XS]
+  float* xml = &lds_at<float>(oXml);    // [wave][head][2]
+  int& flag = lds_at<int>(oFlag);
+  seq_table(a, cum, kvl, qrw);
+  const int S = a.S, HG = a.Hq / a.Hkv, Hu = a.Hkv * A.nhc;
+  {  // decoded sequences without a live token produce zeros (the reference's l == 0 case)
+    const int per_seq = a.Hq * D / 8;
+    for (int i = bid * 256 + tid; i < S * per_seq; i += nblocks * 256) {
+      const int si = i / per_seq;
+      if (kvl[si] >= 0 && cum[si + 1] == cum[si])
+        reinterpret_cast<u32x4*>(a.out)[(size_t)qrw[si] * per_seq + i % per_seq] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  const long long I = (long long)Hu * uru(cum[S]);
+  const int NW = (int)min((long long)nblocks, I);
+  if (bid >= NW) return;
+  const long long g0 = (long long)bid * I / NW, g1 = (long long)(bid + 1) * I / NW;
+
+  auto start_of = [&](int kl) { return a.window > 0 ? max(0, kl - a.window) : 0; };
+  // An item: item j of the n of unit y of sequence s; this wave's tokens start at tb.
+  struct Item {
+    int s, y, j, n, kl, st, tb;
+    bool has;  // inside the range
+  };
+  auto tb_of = [&](int st, int jx) { return (st / NT + jx) * NT + 32 * wv; };
+  Item it0;
+  {
+    int s = 0;
+    for (int c = 0; c < S; c += 64) {
+      const int si = c + lane;
+      s += __builtin_popcountll(__ballot(si < S && (long long)Hu * cum[si + 1] <= g0));
+    }
+    it0.s = uru(s);
+    it0.n = uru(cum[it0.s + 1]) - uru(cum[it0.s]);
+    const int r = (int)(g0 - (long long)Hu * uru(cum[it0.s]));
+    it0.y = uru(r / it0.n);
+    it0.j = uru(r % it0.n);
+    it0.kl = uru(kvl[it0.s]);
+    it0.st = start_of(it0.kl);
+    it0.tb = tb_of(it0.st, it0.j);
+    it0.has = true;
+  }
+  // the item after x, g being x's index; past the range x again with has = false
+  auto after = [&](const Item& x, const long long g) {
+    Item r = x;
+    r.has = g + 1 < g1;
+    if (!r.has) return r;
+    if (++r.j == r.n) {
+      r.j = 0;
+      if (++r.y == Hu) {
+        r.y = 0;
+        do {
+          ++r.s;
+        } while (uru(cum[r.s + 1]) == uru(cum[r.s]));
+        r.n = uru(cum[r.s + 1]) - uru(cum[r.s]);
+        r.kl = uru(kvl[r.s]);
+        r.st = start_of(r.kl);
+      }
+    }
+    r.tb = tb_of(r.st, r.j);
+    return r;
+  };
+
+  const size_t rowb = (size_t)a.Hkv * D * P::EB;  // bytes between a page's tokens
+  const char* kbase = reinterpret_cast<const char*>(a.kc);
+  const char* vbase = reinterpret_cast<const char*>(a.vc);
+
+  // Page lookups of one item: K rows of tokens 16 t + i, and the quads 16 t + 4 jj
+  // (V rows; FP8 page scales).  Positions past the end repeat the last live token.
+  struct Look {
+    int blk[4];  // [K t = 0, 1; quad t = 0, 1]
+  };
+  auto pos_of = [&](const Item& x, int n) { return min(x.tb + 16 * (n & 1) + (n < 2 ? col : 4 * jj), x.kl - 1); };
+  auto lookup = [&](Look& L, const Item& x) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      L.blk[n] = a.block_tables[(size_t)x.s * a.max_blocks + page_of(pos_of(x, n), A.inv_bs)];
+  };
+  auto ok_blk = [&](int b) { return (unsigned)b < (unsigned)a.nb; };
+  auto row_of = [&](const Look& L, int n, const Item& x) {
+    const int p = pos_of(x, n);
+    const int b = ok_blk(L.blk[n]) ? L.blk[n] : 0;
+    return ((size_t)b * a.bs + (p - page_of(p, A.inv_bs) * a.bs)) * rowb + (size_t)(x.y / A.nhc) * (D * P::EB);
+  };
+
+  // (an item past the range: every lane reads the cache's first row, one line; the loads are
+  // issued on every path, so that the wait before a use never drains the ones behind it)
+  DecodeMfmaLoads<C, D> ld;
+  float ks[2] = {1.f, 1.f}, vs[2] = {1.f, 1.f}, ks1[2], vs1[2];  // FP8 page scales: this item's, the next one's
+  auto issue_k = [&](const Look& L, const Item& x) {
+    if constexpr (C::kFp8) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int b = ok_blk(L.blk[2 + t]) ? L.blk[2 + t] : 0;
+        ks1[t] = a.kps[b];
+        vs1[t] = a.vps[b];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const char* p = kbase + (x.has ? row_of(L, t, x) + 16 * jj : 0);
+#pragma unroll
+      for (int w = 0; w < P::KL; ++w) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(p + (x.has ? 64 * w : 0));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) ld.k[t][4 * w + c] = v[c];
+      }
+    }
+  };
+  auto issue_v = [&](const Look& L, const Item& x) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      // the quad's tokens lie in one page (bs % 8 == 0); past the end they repeat the last live one
+      const size_t r0 = x.has ? row_of(L, 2 + t, x) + (size_t)col * (4 * P::VW) : 0;
+      const int left = x.has ? x.kl - 1 - pos_of(x, 2 + t) : 0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(vbase + r0 + (size_t)min(r, left) * rowb);
+        uint32_t(&dst)[P::VW] = ld.v[4 * t + r];
+        if constexpr (P::VW == 1) {
+          dst[0] = w[0];
+        } else if constexpr (P::VW == 2) {
+          const u32x2 v = *reinterpret_cast<const u32x2*>(w);
+          dst[0] = v[0];
+          dst[1] = v[1];
+        } else {
+#pragma unroll
+          for (int c = 0; c < P::VW / 4; ++c) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(w + 4 * c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst[4 * c + e] = v[e];
+          }
+        }
+      }
+    }
+  };
+
+  // query operand of a unit: column h = query head h (zero past the unit's heads)
+  Op qB[P::KS];
+  auto load_q = [&](int si, int yy) {
+    const int kh = yy / A.nhc, h0 = (yy % A.nhc) * A.hc;
+    const int nh = min(A.hc, HG - h0);
+    const QT* qp = reinterpret_cast<const QT*>(a.q) +
+                   ((size_t)qrw[si] * a.Hq + (size_t)kh * HG + h0 + (col < nh ? col : 0)) * D;
+#pragma unroll
+    for (int w = 0; w < P::KS; ++w) {
+      const int d = C::kFp8 ? 64 * (w >> 1) + 16 * jj + 8 * (w & 1) : 32 * w + 8 * jj;
+      const u32x4 x = *reinterpret_cast<const u32x4*>(qp + d);
+      qB[w] = __builtin_bit_cast(Op, col < nh ? x : u32x4{0u, 0u, 0u, 0u});
+    }
+  };
+
+  float m_run = -INFINITY, l_part = 0.f;
+  f32x4 acc[P::SB];
+  auto clear = [&]() {
+    m_run = -INFINITY;
+    l_part = 0.f;
+#pragma unroll
+    for (int b = 0; b < P::SB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+
+  // In flight, oldest first: K of this item, the lookups of the next, V of this item.
+  Item cur = it0, nxt = after(cur, g0);
+  Look lc, ln, l2;
+  lookup(lc, cur);
+  load_q(cur.s, cur.y);
+  issue_k(lc, cur);
+  lookup(ln, nxt);
+  issue_v(lc, cur);
+  long long seg0 = g0;  // first item of the unit that this workgroup holds
+
+  for (long long g = g0; g < g1; ++g) {
+    const int s = cur.s, y = cur.y, n_s = cur.n, tb = cur.tb, kv_len = cur.kl, start_k = cur.st;
+    const Item n2 = nxt.has ? after(nxt, g + 1) : nxt;
+    // ---- scores
+    float sc[8];
+    if constexpr (C::kFp8) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        ks[t] = ks1[t];
+        vs[t] = vs1[t];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < P::KS; ++w) c = mfma_op(k_operand<C, D>(ld.k[t], w), qB[w], c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[4 * t + r] = C::kFp8 ? c[r] * (ks[t] * 256.f) : c[r];
+    }
+    issue_k(ln, nxt);
+    lookup(l2, n2);
+    const bool unit_end = !nxt.has || nxt.s != s || nxt.y != y;
+
+    // ---- mask: outside [start_k, kv_len), or on a page with an invalid id
+    const bool okq = ok_blk(lc.blk[2]) && ok_blk(lc.blk[3]);
+    if (tb < start_k || tb + 32 > kv_len || !__all(okq)) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int p = tb + 16 * (e >> 2) + 4 * jj + (e & 3);
+        if (p < start_k || p >= kv_len || !ok_blk(lc.blk[2 + (e >> 2)])) sc[e] = -INFINITY;
+      }
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) tmax = fmaxf(tmax, sc[e]);
+    tmax = rows4_max(tmax) * a.scale_log2;
+    const float m_new = fmaxf(m_run, tmax);
+    if (__any(m_new != m_run)) {
+      const float alpha = m_run == m_new ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+      l_part *= alpha;
+#pragma unroll
+      for (int b = 0; b < P::SB; ++b) acc[b] *= alpha;
+      m_run = m_new;
+    }
+    const float m_sub = fmaxf(m_run, -3.0e38f) - kPBias;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      sc[e] = __builtin_amdgcn_exp2f(fmaf(sc[e], a.scale_log2, -m_sub));
+      l_part += sc[e];
+    }
+    float post = 1.f;
+    if constexpr (C::kFp8) {
+      // p * (value page scale), brought near 1 by a power of two taken out after the MFMA
+      const float vmax = rows4_max(fmaxf(vs[0], vs[1]));
+      const int ex = min(max((int)((__float_as_uint(vmax) >> 23) & 0xFFu) - 127, -100), 100);
+      const float down = __uint_as_float((uint32_t)(127 - ex) << 23);
+      post = __uint_as_float((uint32_t)(127 + ex + 8) << 23);  // the codes enter as value * 2^-8
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sc[e] *= vs[e >> 2] * down;
+    }
+    Op pB[C::kParts];
+    split_p(sc, pB);
+#pragma unroll
+    for (int b = 0; b < P::SB; ++b) {
+      const Op V = v_operand<C, P::VW>(ld.v, b);
+      f32x4 t = C::kFp8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[b];
+#pragma unroll
+      for (int k = 0; k < C::kParts; ++k) t = mfma_op(V, pB[k], t);
+      if constexpr (C::kFp8) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(t[r], post, acc[b][r]);
+      } else {
+        acc[b] = t;
+      }
+    }
+    issue_v(ln, nxt);
+
+    if (unit_end) {
+      // ---- the waves' states through LDS (rounds of RD dims), all threads combining
+      const int kvh = y / A.nhc, h0 = (y % A.nhc) * A.hc, nh = min(A.hc, HG - h0);
+      const int u = s * Hu + y;
+      const long long unit_first = (long long)Hu * uru(cum[s]) + (long long)y * n_s;
+      const bool whole = seg0 == unit_first && g + 1 == unit_first + n_s;
+      int slot = 0, np = 1;
+      if (!whole) {
+        const int wf = wave_of_item(unit_first, I, NW);
+        np = uru(wave_of_item(unit_first + n_s - 1, I, NW) - wf + 1);
+        slot = uru(wf + u);  // the unit's pieces sit in slots wf + u ..
+      }
+      float l = l_part + __shfl_xor(l_part, 16, 64);
+      l += __shfl_xor(l, 32, 64);
+      bool bad = false;
+      QT* out = reinterpret_cast<QT*>(a.out) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0) * D;
+      const __amdgpu_buffer_rsrc_t ro =
+          uniform_rsrc(a.ws_o + (size_t)slot * (A.hc * D), whole ? 0 : np * A.hc * D * 4);
+      const __amdgpu_buffer_rsrc_t rm = uniform_rsrc(a.ws_ml + (size_t)slot * (A.hc * 2), whole ? 0 : np * A.hc * 8);
+      const int me = whole ? 0 : uru(bid + u - slot);
+#pragma unroll
+      for (int rd = 0; rd < D / P::RD; ++rd) {
+        __syncthreads();  // (the previous combine has been read)
+        constexpr int BR = P::SB / (D / P::RD);  // sub-tiles of the round
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int b = 0; b < BR; b += 4) {
+            const f32x4 x = {acc[rd * BR + b][r], acc[rd * BR + b + 1][r], acc[rd * BR + b + 2][r],
+                             acc[rd * BR + b + 3][r]};
+            if (col < nh)
+              *reinterpret_cast<f32x4*>(xo + (wv * 16 + col) * P::XS + (4 * jj + r) * BR + b) = x;
+          }
+        if (rd == 0 && jj == 0 && col < nh) {
+          xml[(wv * 16 + col) * 2] = m_run;
+          xml[(wv * 16 + col) * 2 + 1] = l;
+        }
+        __syncthreads();
+        for (int e = tid; e < nh * (P::RD / 4); e += 256) {
+          const int h = e / (P::RD / 4), c = e % (P::RD / 4);
+          float M = -INFINITY;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) M = fmaxf(M, xml[(w * 16 + h) * 2]);
+          f32x4 O = {0.f, 0.f, 0.f, 0.f};
+          float L = 0.f;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const float mw = xml[(w * 16 + h) * 2];
+            const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+            O += *reinterpret_cast<const f32x4*>(xo + (w * 16 + h) * P::XS + 4 * c) * f;
+            L = fmaf(xml[(w * 16 + h) * 2 + 1], f, L);
+          }
+          // element 4 c + k of the round is dim SB * row + rd * BR + ..: contiguous in k
+          const int dim = (4 * c / BR) * P::SB + rd * BR + (4 * c) % BR;
+          if (whole) {
+            bad |= write4(O, L, out + (size_t)h * D + dim);
+          } else {
+            store_f32x4(O, ro, (h * D + dim) * 4, me * A.hc * D * 4);
+            if (rd == 0 && c == 0)
+              __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{M, L}), rm, h * 8, me * A.hc * 8,
+                                                    kCoherent);
+          }
+        }
+      }
+      bool done = whole;
+      if (!whole) {
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete before the workgroup is counted
+        __syncthreads();
+        if (tid == 0) {
+          const int old = __hip_atomic_fetch_add(a.ws_cnt + u, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (old == np - 1) __hip_atomic_store(a.ws_cnt + u, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          flag = old == np - 1;
+        }
+        __syncthreads();
+        done = flag != 0;
+        if (done) {
+          // the workgroup counted last merges the pieces (page_attention.py:2006-2059):
+          // NE float4 elements; with fewer than 256, groups of threads share the pieces
+          const int NE = nh * (D / 4);
+          const int ng = NE < 256 ? 256 / NE : 1;
+          for (int e0 = 0; e0 < NE; e0 += 256) {
+            const int e = NE < 256 ? tid % NE : e0 + tid;
+            const int grp = NE < 256 ? tid / NE : 0;
+            const bool act = e < NE && grp < ng;
+            const int h = act ? 4 * e / D : 0;
+            float M = -INFINITY, L = 0.f;
+            f32x4 O = {0.f, 0.f, 0.f, 0.f};
+            constexpr int NB = 4;  // pieces in flight per thread
+            if (act) {
+              for (int p0 = grp; p0 < np; p0 += NB * ng) {
+                f32x4 o[NB];
+                f32x2 ml[NB];
+#pragma unroll
+                for (int k = 0; k < NB; ++k) {
+                  const int p = min(p0 + k * ng, np - 1);
+                  // (the piece's offset in the per-lane part: groups read different pieces)
+                  o[k] = __builtin_bit_cast(
+                      f32x4, __builtin_amdgcn_raw_buffer_load_b128(ro, (p * A.hc * D + 4 * e) * 4, 0, kCoherent));
+                  ml[k] = __builtin_bit_cast(
+                      f32x2, __builtin_amdgcn_raw_buffer_load_b64(rm, (p * A.hc + h) * 8, 0, kCoherent));
+                }
+#pragma unroll
+                for (int k = 0; k < NB; ++k) {
+                  if (p0 + k * ng >= np || ml[k].x == -INFINITY) continue;
+                  const float Mn = fmaxf(M, ml[k].x);
+                  const float fo = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
+                  const float fp = __builtin_amdgcn_exp2f(ml[k].x - Mn);
+                  O = O * fo + o[k] * fp;
+                  L = L * fo + ml[k].y * fp;
+                  M = Mn;
+                }
+              }
+            }
+            if (ng > 1) {  // the groups' states through LDS (element-major: 6 floats each)
+              if (act) {
+                float* x = xo + (grp * NE + e) * 6;
+                x[0] = M;
+                x[1] = L;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[2 + k] = O[k];
+              }
+              __syncthreads();
+              if (act && grp == 0) {
+                for (int q = 1; q < ng; ++q) {
+                  const float* x = xo + (q * NE + e) * 6;
+                  if (x[0] == -INFINITY) continue;
+                  const float Mn = fmaxf(M, x[0]);
+                  const float fo = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
+                  const float fp = __builtin_amdgcn_exp2f(x[0] - Mn);
+#pragma unroll
+                  for (int k = 0; k < 4; ++k) O[k] = O[k] * fo + x[2 + k] * fp;
+                  L = L * fo + x[1] * fp;
+                  M = Mn;
+                }
+              }
+            }
+            if (act && grp == 0) {
+              bad |= write4(O, L, out + 4 * e);
+            }
+          }
+        }
+      }
+      // ---- a row that is not finite: again in fp32, key by key (attend_row)
+      if (__syncthreads_or(done && bad)) {
+        for (int h = wv; h < nh; h += 4) {
+          float lr, x[D / 64];
+          const QT* qp = reinterpret_cast<const QT*>(a.q) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0 + h) * D;
+          attend_row<C, D>(a, s, kvh, qp, start_k, kv_len, lr, x, lane);
+#pragma unroll
+          for (int i = 0; i < D / 64; ++i) from_f32(lr > 0.f ? x[i] / lr : 0.f, out + (size_t)h * D + lane + 64 * i);
+        }
+      }
+      clear();
+      seg0 = g + 1;
+      if (nxt.has) load_q(nxt.s, nxt.y);
+    }
+    cur = nxt;
+    nxt = n2;
+    lc = ln;
+    ln = l2;
+  }
+}
+
+// (D = 256 holds 64 words of V and 64 of K per lane: one workgroup per compute unit, no spills)
+template <class C, int D>
+__global__ __launch_bounds__(256, D == 256 ? 1 : 2) void decode_mfma(DecodeMfmaArgs a) {
+  decode_mfma_body<C, D>(a, blockIdx.x, gridDim.x);
+}
+
+}  // namespace emx

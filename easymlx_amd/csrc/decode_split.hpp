@@ -1,4 +1,6 @@
-// Split-K single-token decode for the shapes outside the MFMA decode kernels:
+// Split-K single-token decode for the shapes outside the MFMA decode kernels
+// (decode_q4 / decode_affine / decode_fp8, and decode_mfma for unquantized and FP8
+// caches of head_dim 64, 128 and 256):
 // any head_dim that is a multiple of 32 up to 256, pages of a multiple of 8
 // tokens, affine pages with group sizes that are multiples of 32, dense
 // fp16/bf16/fp32 caches and FP8 pages, fp16/bf16/fp32 queries.

@@ -24,6 +24,7 @@
 #include "slots.hpp"
 #include "probe.hpp"
 #include "pages.hpp"
+#include "mfma_launch.hpp"
 
 constexpr int kNoallocScratchFloats = 2 * emx::kFp8Parts;  // 2 KiB per stream slot
 constexpr int kNoallocSlots = 8;                            // streams with a slot of their own
@@ -388,6 +389,25 @@ int launch_generic_only(const emx::GenericArgs& ga, const KV& kv, hipStream_t st
   dim3 grid(ga.T, ga.Hkv, (hg + 15) / 16);
   hipLaunchKernelGGL((emx::paged_generic<QT, KV>), grid, dim3(64), 0, st, ga, kv);
   return check_launch("paged_generic");
+}
+
+// A call over a token-major cache (unquantized, FP8) with what `ga` holds.
+emx::TokenMajorCall token_major_call(emx::KvKind kind, const emx::GenericArgs& ga, const void* k, const void* v,
+                                     const float* kps, const float* vps) {
+  return emx::TokenMajorCall{kind, ga.q, ga.out, k, v, kps, vps, ga.block_tables, ga.kv_lens,
+                             ga.decode ? nullptr : ga.qsl, ga.T, ga.S, ga.Hq, ga.Hkv, ga.D, ga.bs, ga.nb,
+                             ga.max_blocks, ga.scale_log2, ga.window};
+}
+
+// Runs the call on the MFMA kernels where they take its shape and the workspace holds
+// their partials; false: nothing launched.
+bool run_token_major(const emx::TokenMajorCall& c, void* ws, size_t ws_bytes, hipStream_t st, int* rc) {
+  if (!ws || c.qsl || c.S != c.T || !emx::token_major_ok(c)) return false;
+  if (ws_bytes < kPartialsInt * sizeof(int) + emx::decode_mfma_partial_bytes(c.S, c.Hq, c.Hkv, c.D)) return false;
+  int* wi = static_cast<int*>(ws);
+  emx::launch_decode_mfma(c, wi, reinterpret_cast<float*>(wi + kPartialsInt), st);
+  *rc = check_launch("decode_mfma");
+  return true;
 }
 
 constexpr int kMaxDevices = 64;
@@ -1016,7 +1036,10 @@ size_t emx_paged_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads
   // the split-K decode of the other shapes keeps its chunks' partials after the same offset
   const size_t split = split_workspace_bytes(num_seqs, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq,
                                              page_size);
-  return std::max(fast, split ? kPartialsInt * sizeof(int) + split : 0);
+  // and so does the MFMA decode over token-major caches
+  const size_t mfma = page_size % 8 == 0 ? emx::decode_mfma_partial_bytes(num_seqs, num_q_heads, num_kv_heads, head_dim) : 0;
+  const size_t part = std::max(split, mfma);
+  return std::max(fast, part ? kPartialsInt * sizeof(int) + part : 0);
 }
 
 int emx_paged_attention_affine(const void* queries, int num_tokens, int num_q_heads, int head_dim,
@@ -1240,6 +1263,12 @@ int emx_paged_attention_dense(const void* queries, int num_tokens, int num_q_hea
   ga.scale_log2 = softmax_scale * emx::kLog2e;
   ga.window = sliding_window > 0 ? sliding_window : 0;
   ga.decode = single_token_decode ? 1 : 0;
+  if (dtype == EMX_DTYPE_F16 || dtype == EMX_DTYPE_BF16) {
+    const emx::KvKind kind = dtype == EMX_DTYPE_F16 ? emx::KvKind::f16 : emx::KvKind::bf16;
+    if (run_token_major(token_major_call(kind, ga, key_cache, value_cache, nullptr, nullptr), workspace,
+                        workspace_bytes, st, &rc))
+      return rc;
+  }
   switch (dtype) {
     case EMX_DTYPE_F16: {
       emx::DenseKV<emx::F16> kv{reinterpret_cast<const emx::h16*>(key_cache),
@@ -1584,6 +1613,10 @@ int emx_paged_attention_fp8(const void* queries, int num_tokens, int num_q_heads
   // other GQA ratios: the MFMA prefill kernel over every row (a decode row is a
   // tile of one query token)
   if (pf && query_start_loc) return launch_prefill(1);
+  if (dtype == EMX_DTYPE_F16 && run_token_major(token_major_call(emx::KvKind::fp8, ga, key_cache, value_cache, k_scale,
+                                                                 v_scale),
+                                                workspace, workspace_bytes, st, &rc))
+    return rc;
   const emx::Fp8KV kv{key_cache, value_cache, k_scale, v_scale, num_kv_heads, head_dim, page_size};
   switch (dtype) {
     case EMX_DTYPE_F16: return launch_generic<emx::h16>(ga, kv, st, workspace, workspace_bytes);

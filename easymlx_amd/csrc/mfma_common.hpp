@@ -1,0 +1,142 @@
+// Shared pieces of the MFMA attention kernels over token-major caches
+// [nb, bs, Hkv, D] (unquantized fp16 / bf16, FP8 E4M3): operand types, the
+// probability split, and the exact fallback for non-finite rows.
+#pragma once
+
+#include "common.hpp"
+#include "decode_affine.hpp"
+
+namespace emx {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef h16 h16x2 __attribute__((ext_vector_type(2)));
+
+// Cache kinds: the element type of the pages, and of the queries and outputs.
+struct KvF16 {
+  typedef h16 QT;       // queries, outputs
+  typedef h16x8 Op;     // one lane's MFMA operand
+  typedef h16 ET;       // cache element
+  static constexpr int kParts = 2;  // 16-bit parts of a probability
+  static constexpr bool kFp8 = false;
+};
+struct KvBF16 {
+  typedef uint16_t QT;
+  typedef bf16x8 Op;
+  typedef uint16_t ET;
+  static constexpr int kParts = 3;
+  static constexpr bool kFp8 = false;
+};
+struct KvFp8 {
+  typedef h16 QT;
+  typedef h16x8 Op;
+  typedef uint8_t ET;
+  static constexpr int kParts = 2;
+  static constexpr bool kFp8 = true;
+};
+
+__device__ __forceinline__ f32x4 mfma_op(const h16x8 a, const h16x8 b, const f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma_op(const bf16x8 a, const bf16x8 b, const f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Probabilities enter the matrix unit as a sum of 16-bit parts, so that the
+// products with V keep the fp32 probability: fp16 in two parts (11 + 11 bits of
+// the 24; the exponent offset kPBias lifts p out of fp16's sub-normals), bf16
+// in three (8 + 8 + 8, exact).
+constexpr float kPBias = 8.f;  // p = 2^(x - m + kPBias)
+
+__device__ __forceinline__ void split_p(const float (&x)[8], h16x8 (&p)[2]) {
+  typedef float f32x2v __attribute__((ext_vector_type(2)));
+  uint32_t hi[4], lo[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const h16x2 h = __builtin_convertvector(f32x2v{x[2 * i], x[2 * i + 1]}, h16x2);
+    const h16x2 l = __builtin_convertvector(f32x2v{x[2 * i] - (float)h[0], x[2 * i + 1] - (float)h[1]}, h16x2);
+    hi[i] = __builtin_bit_cast(uint32_t, h);
+    lo[i] = __builtin_bit_cast(uint32_t, l);
+  }
+  p[0] = as_h8(hi[0], hi[1], hi[2], hi[3]);
+  p[1] = as_h8(lo[0], lo[1], lo[2], lo[3]);
+}
+__device__ __forceinline__ void split_p(const float (&x)[8], bf16x8 (&p)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t a = __float_as_uint(x[2 * i]), b = __float_as_uint(x[2 * i + 1]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w[k][i] = __builtin_amdgcn_perm(b, a, 0x07060302u);  // the top halves
+      if (k < 2) {
+        a = __float_as_uint(__uint_as_float(a) - __uint_as_float(a & 0xFFFF0000u));
+        b = __float_as_uint(__uint_as_float(b) - __uint_as_float(b & 0xFFFF0000u));
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) p[k] = __builtin_bit_cast(bf16x8, u32x4{w[k][0], w[k][1], w[k][2], w[k][3]});
+}
+
+// page of position p for pages of bs tokens, inv = ceil(2^32 / bs) (bs >= 2):
+// exact while p * bs < 2^32, which the host checks for the whole table.
+__device__ __forceinline__ int page_of(const int p, const uint32_t inv) { return (int)__umulhi((uint32_t)p, inv); }
+
+template <class C>
+__device__ __forceinline__ float kv_elem(const void* base, const size_t i) {
+  if constexpr (C::kFp8)
+    return e4m3_to_f32(static_cast<const uint8_t*>(base)[i]);
+  else
+    return to_f32(static_cast<const typename C::ET*>(base)[i]);
+}
+
+// One query row against keys [k0, k1) in fp32 on one wave, a key at a time: the
+// rows whose MFMA result is not finite are computed again here.  On the matrix
+// unit a masked key still enters its tile's product with p = 0, and 0 * inf (an
+// infinity or NaN in a masked or stale value, or in the low part of a visible
+// one) would make NaN of what these arithmetic rules leave finite or infinite.
+// Lane L ends with dims L + 64 i; l is the sum of the probabilities.
+template <class C, int D>
+__device__ void attend_row(const DecodeArgs& a, const int s, const int kvh, const typename C::QT* q, const int k0,
+                           const int k1, float& l, float (&acc)[(D + 63) / 64], const int lane) {
+  constexpr int N = (D + 63) / 64;
+  float qv[N], m = -INFINITY;
+  l = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    qv[i] = to_f32(q[lane + 64 * i]);
+    acc[i] = 0.f;
+  }
+#pragma unroll 1
+  for (int k = k0; k < k1; ++k) {
+    const int blk = a.block_tables[(size_t)s * a.max_blocks + k / a.bs];
+    if ((unsigned)blk >= (unsigned)a.nb) continue;
+    const size_t row = (((size_t)blk * a.bs + k % a.bs) * a.Hkv + kvh) * D;
+    float x = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) x += qv[i] * kv_elem<C>(a.kc, row + lane + 64 * i);
+    x = wave_sum(x);
+    float vs = 1.f;
+    if constexpr (C::kFp8) {
+      x *= a.kps[blk];
+      vs = a.vps[blk];
+    }
+    x *= a.scale_log2;
+    const float mn = fmaxf(m, x);
+    float p = 0.f, al = 1.f;
+    if (mn != -INFINITY || x != x) {
+      p = exp2f(x - mn);
+      al = m == mn ? 1.f : exp2f(m - mn);
+    }
+    l = l * al + p;
+    m = mn;
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = acc[i] * al + p * (kv_elem<C>(a.vc, row + lane + 64 * i) * vs);
+  }
+}
+
+__device__ __forceinline__ bool not_finite(const float x) {
+  return (__float_as_uint(x) & 0x7F800000u) == 0x7F800000u;
+}
+
+}  // namespace emx

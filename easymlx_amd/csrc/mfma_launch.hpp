@@ -1,0 +1,38 @@
+// Launchers of the MFMA kernels over token-major caches (emx_mfma.hip, a translation
+// unit of its own), called by the C entry points in emx_attn.hip.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+namespace emx {
+
+enum class KvKind { f16, bf16, fp8 };
+
+// One attention call over a token-major cache, as the entry points receive it.
+struct TokenMajorCall {
+  KvKind kind;
+  const void* q;
+  void* out;
+  const void* k;
+  const void* v;
+  const float *kps, *vps;        // FP8: scale per page
+  const int32_t *block_tables, *kv_lens, *qsl;
+  int T, S, Hq, Hkv, D, bs, nb, max_blocks;
+  float scale_log2;
+  int window;
+};
+
+// Shapes the kernels take: head_dim 64, 128 or 256 (whole MFMA k-slices and a power of
+// two of dims per lane), pages of a multiple of 8 tokens (a quad of tokens in one page),
+// 16-byte aligned tensors, tables within the kernels' limits.  They were the faster side
+// at every size tried within these (decode_mfma.hpp has figures).
+bool token_major_ok(const TokenMajorCall& c);
+
+// Bytes the decode's partials take after the workspace's fixed region (0: shape not taken).
+size_t decode_mfma_partial_bytes(int S, int Hq, int Hkv, int D);
+// ws_cnt: the workspace's unit counters; partials: decode_mfma_partial_bytes bytes.
+void launch_decode_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, hipStream_t st);
+
+}  // namespace emx

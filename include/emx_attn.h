@@ -352,10 +352,11 @@ int emx_paged_attention_affine(const void* queries, int num_tokens, int num_q_he
  * Paged attention over an unquantized cache in the reference layout
  * key/value [num_blocks, page_size, Hkv, head_dim] (dtype = queries' dtype).
  * Single-token decode calls (head_dim a multiple of 32 up to 256, page_size a
- * multiple of 8) run split-K over chunks of keys when the workspace holds
+ * multiple of 8) run split-K over ranges of keys when the workspace holds
  * emx_paged_workspace_bytes(...) bytes (same rules as
- * emx_paged_attention_affine); otherwise, or with a null workspace, one
- * wave per (token, kv head) walks the keys.
+ * emx_paged_attention_affine): on the matrix units for fp16 / bf16 with
+ * head_dim 64, 128 or 256 and 16-byte aligned tensors.  Otherwise, or with a
+ * null workspace, one wave per (token, kv head) walks the keys.
  * Replaces: paged_attention(...) unified_attention.py:1377-1512 for fp16/bf16/fp32 caches
  *   (decode kernels :467-775, split-K precedent page_attention.py:1718-2059).
  */

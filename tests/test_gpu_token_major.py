@@ -1,0 +1,113 @@
+"""MFMA attention over token-major caches (unquantized fp16 / bf16, FP8) vs the float64 oracle.
+
+Bound of a result: half a unit in the last place of the 16-bit output (2^-11 / 2^-8 of the value, bf16
+rounding 8 bits) plus the fp32 arithmetic: scores are fp32 sums of up to 256 products, |s| <= ~16, so a
+probability is off by at most ~2^-18 of itself and an output by 2^-16 of the largest value it averages.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from easymlx_amd import paged_attention
+from oracle import fp8
+from oracle.paged_attention import paged_attention as oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "fp8": torch.float16}
+
+
+def batch(kind, qlens, kvl, hq, hkv, d, page, seed, invalid=()):
+    """Seeded inputs on the CPU: queries, stored caches (and scales), tables, and the exact cache values."""
+    rng = np.random.default_rng(seed)
+    pages = [-(-max(x, 1) // page) for x in kvl]
+    nb = sum(pages) + 1
+    tables = np.full((len(kvl), max(pages)), -1, np.int32)
+    perm, at = rng.permutation(nb).astype(np.int32), 0
+    for i, p in enumerate(pages):
+        tables[i, :p] = perm[at:at + p]
+        at += p
+    for i, c in invalid:
+        tables[i, c] = -1 if c % 2 else nb + 3
+    q = torch.from_numpy(rng.standard_normal((sum(qlens), hq, d), dtype=np.float32)).to(DTYPES[kind])
+    shape = (nb, page, hkv, d)
+    scales = None
+    if kind == "fp8":
+        codes = [rng.integers(0, 256, size=shape).astype(np.uint8) & 0xF7 for _ in range(2)]  # |x| <= 240, no NaN code
+        scales = [rng.uniform(0.003, 0.02, size=nb).astype(np.float32) for _ in range(2)]
+        cache = [torch.from_numpy(c) for c in codes]
+        exact = [fp8.e4m3_decode(c).astype(np.float64) * s[:, None, None, None].astype(np.float64)
+                 for c, s in zip(codes, scales)]
+    else:
+        cache = [torch.from_numpy(rng.standard_normal(shape, dtype=np.float32) * 1.5).to(DTYPES[kind])
+                 for _ in range(2)]
+        exact = [c.double().numpy() for c in cache]
+    return dict(q=q, cache=cache, scales=scales, exact=exact, tables=tables, kvl=np.asarray(kvl, np.int32),
+                qsl=np.concatenate([[0], np.cumsum(qlens)]).astype(np.int32))
+
+
+def run(b, dev, window=0, decode=True):
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    kw = dict(k_scale=t(b["scales"][0]), v_scale=t(b["scales"][1])) if b["scales"] is not None else {}
+    out = paged_attention(b["q"].to(dev), b["cache"][0].to(dev), b["cache"][1].to(dev), t(b["tables"]), t(b["kvl"]),
+                          t(b["qsl"]), sliding_window=window or None, single_token_decode=decode, **kw)
+    torch.cuda.synchronize()
+    return out.double().cpu().numpy()
+
+
+def expected(b, window=0):
+    return oracle_attention(b["q"].double().numpy(), b["exact"][0], b["exact"][1], b["tables"], b["kvl"], b["qsl"],
+                            sliding_window=window, compute_dtype=np.float64, out_dtype=np.float64)
+
+
+def check(b, got, exp):
+    ulp = 2.0 ** -8 if b["q"].dtype == torch.bfloat16 else 2.0 ** -11
+    bound = ulp * np.abs(exp) + 2.0 ** -16 * np.abs(b["exact"][1]).max() + 2.0 ** -24
+    err = np.abs(got - exp)
+    assert np.isfinite(got).all()
+    assert (err <= bound).all(), f"{int((err > bound).sum())} of {err.size}, worst {(err / bound).max():.2f} of the bound"
+
+
+# item (128), wave (32) and quad (4) edges, and contexts cut between workgroups
+CONTEXTS = [1, 3, 31, 32, 33, 127, 128, 129, 0, 300, 1000, 5]
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16", "fp8"])
+@pytest.mark.parametrize("d,page,hq,hkv", [(64, 16, 8, 2), (128, 16, 6, 2), (128, 24, 7, 1), (128, 8, 40, 2),
+                                           (256, 64, 4, 4), (256, 32, 16, 1)])
+def test_decode(cuda, kind, d, page, hq, hkv):
+    print(f"[token-major decode {kind} d{d} page{page} {hq}/{hkv}]", flush=True)
+    b = batch(kind, [1] * len(CONTEXTS), CONTEXTS, hq, hkv, d, page, seed=d + page + hq,
+              invalid=[(5, 1), (9, 0), (10, 2)] if page < 64 else [])
+    for window in (0, 1, 100):
+        check(b, run(b, cuda, window), expected(b, window))
+
+
+@pytest.mark.parametrize("kind", ["f16", "fp8"])
+def test_decode_one_long_row(cuda, kind):
+    """One sequence cut over every workgroup: a merge of many pieces, twice on the same workspace."""
+    print(f"[token-major long row {kind}]", flush=True)
+    b = batch(kind, [1], [40_003], 4, 1, 128, 16, seed=3)
+    exp = expected(b)
+    first = run(b, cuda)
+    check(b, first, exp)
+    assert np.array_equal(first, run(b, cuda))
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_decode_infinities(cuda, kind):
+    """An infinity or NaN outside the visible keys leaves a row as it is; a visible infinity stays one."""
+    print(f"[token-major infinities {kind}]", flush=True)
+    kvl, window = [200, 200, 70], 64
+    b = batch(kind, [1] * 3, kvl, 4, 2, 128, 16, seed=8)
+    exp = expected(b, window)
+    v = b["cache"][1]
+    at = lambda s, p: (int(b["tables"][s, p // 16]), p % 16)  # noqa: E731
+    v[at(0, 130)][0, 7] = float("inf")   # before the window, in a step the kernel reads
+    v[at(2, 75)][1, 9] = float("nan")    # stale, past kv_len in the last page
+    v[at(1, 190)][1, 3] = float("inf")   # visible to sequence 1, kv head 1
+    got = run(b, cuda, window)
+    assert np.isposinf(got[1, 2:, 3]).all()
+    got[1, 2:, 3] = exp[1, 2:, 3]
+    check(b, got, exp)
