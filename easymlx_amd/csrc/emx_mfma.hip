@@ -5,6 +5,7 @@
 
 #include "decode_mfma.hpp"
 #include "mfma_launch.hpp"
+#include "prefill_mfma.hpp"
 
 namespace emx {
 namespace {
@@ -74,6 +75,59 @@ void launch_decode_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, h
                           : c.kind == KvKind::bf16 ? pick_decode<KvBF16>(c.D)
                                                    : pick_decode<KvFp8>(c.D);
   hipLaunchKernelGGL(fn, dim3(kDecodeMfmaWGs), dim3(256), 0, st, decode_args(c, ws_cnt, partials));
+}
+
+namespace {
+
+// Query columns per wave: 16 CT.  More columns read each K and V operand from LDS fewer
+// times; at D = 256 the accumulator of 32 columns leaves one wave per SIMD.
+constexpr int ct_of(int D) { return D > 128 ? 1 : 2; }
+// Most query tiles per kv head: a sequence of q >= min_q query tokens has at most q / tokb + 1.
+long tile_items(int T, int S, int tokb, int min_q) { return (long)(T + tokb - 1) / tokb + std::min(S, T / min_q); }
+
+typedef void (*MixedFn)(PrefillMfmaArgs, DecodeMfmaArgs, int);
+
+template <class C>
+MixedFn pick_mixed(int D) {
+  return D == 64 ? mixed_mfma<C, 64, ct_of(64)> : D == 128 ? mixed_mfma<C, 128, ct_of(128)>
+                                                            : mixed_mfma<C, 256, ct_of(256)>;
+}
+
+}  // namespace
+
+bool mixed_mfma_ok(const TokenMajorCall& c) {
+  return token_major_ok(c) && c.qsl && c.Hq / c.Hkv <= 64 * ct_of(c.D) && (long long)c.nb * c.bs < (1LL << 31);
+}
+
+size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_counters) {
+  const int hg = Hq / Hkv;
+  if (!head_ok(D) || hg > 64 * ct_of(D)) return 0;
+  const long items = tile_items(T, S, 64 * ct_of(D) / hg, 2);
+  if (items * Hkv * 4 > max_counters) return 0;
+  return (size_t)items * Hkv * kPrefillParts * (4 * (ct_of(D) * (D / 16) + 1) * 1024);
+}
+
+void launch_mixed_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
+                       hipStream_t st) {
+  const MixedFn fn = c.kind == KvKind::f16    ? pick_mixed<KvF16>(c.D)
+                     : c.kind == KvKind::bf16 ? pick_mixed<KvBF16>(c.D)
+                                              : pick_mixed<KvFp8>(c.D);
+  const DecodeMfmaArgs d = decode_args(c, ws_cnt, partials);
+  PrefillMfmaArgs p{};
+  p.d = d.d;
+  p.inv_bs = d.inv_bs;
+  p.min_q = ws_cnt ? 2 : 1;
+  p.tokb = 64 * ct_of(c.D) / (c.Hq / c.Hkv);
+  const long items = tile_items(c.T, c.S, p.tokb, p.min_q);
+  p.nparts = part ? kPrefillParts : 1;
+  p.max_items = part ? (int)items : 0;
+  p.ws_cnt = ws_part_cnt;
+  p.ws_part = part;
+  // Decode workgroups by the decode rows' share of the step (at most S of the T rows):
+  // bytes per key of a decode row against matrix work per key of a query row.
+  const double share = 100.0 * (c.kind == KvKind::fp8 ? 0.5 : 1.0) * c.S / std::max(1, c.T - c.S) * c.Hkv / c.Hq;
+  const int ndec = ws_cnt ? std::clamp((int)(1024.0 * share), 64, kDecodeMfmaWGs) : 0;
+  hipLaunchKernelGGL(fn, dim3((unsigned)(items * c.Hkv * p.nparts + ndec)), dim3(256), 0, st, p, d, ndec);
 }
 
 }  // namespace emx

@@ -35,4 +35,12 @@ size_t decode_mfma_partial_bytes(int S, int Hq, int Hkv, int D);
 // ws_cnt: the workspace's unit counters; partials: decode_mfma_partial_bytes bytes.
 void launch_decode_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, hipStream_t st);
 
+// A ragged call (qsl given): rows of longer queries, and single-token rows beside them.
+// ws_cnt null (no workspace): every row as a query tile, nothing cut.  part null: tiles
+// are not cut; else mixed_mfma_part_bytes bytes (ws_part_cnt: their counters).
+bool mixed_mfma_ok(const TokenMajorCall& c);
+size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_counters);
+void launch_mixed_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
+                       hipStream_t st);
+
 }  // namespace emx

@@ -9,9 +9,8 @@
 // One wavefront per (token, kv_head, chunk of <=16 query heads): every K/V
 // element read is shared by the whole GQA group.  Keys are processed 64 at a
 // time (one per lane for QK^T, then one dim per lane for PV with the
-// probabilities staged in LDS).  This is the path for prefill rows, odd
-// shapes and unquantized caches; single-token decode over affine pages with
-// head_dim 128 uses decode_affine_d128.
+// probabilities staged in LDS).  This is the path of the shapes outside the
+// MFMA kernels: other head sizes and pages, fp32.
 #pragma once
 
 #include "common.hpp"

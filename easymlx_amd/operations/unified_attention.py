@@ -242,7 +242,7 @@ def paged_attention(
             raise ValueError("k_scale/v_scale must hold one scale per block: [num_blocks]")
         need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
         if need and not single_token_decode:  # room for the prefill key split
-            need += int(lib.emx_paged_prefill_workspace_bytes(total, S, hq, hkv, d))
+            need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
         if need and workspace is None:
             workspace = _workspace(dev, stream, need)
         ws_ptr = workspace.data_ptr() if workspace is not None else None
@@ -264,7 +264,11 @@ def paged_attention(
     key_cache = key_cache.contiguous()
     value_cache = value_cache.contiguous()
     nb, bs, hkv = int(key_cache.shape[0]), int(key_cache.shape[1]), int(key_cache.shape[2])
-    need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs)) if single_token_decode else 0
+    need = 0
+    if single_token_decode or queries.dtype != torch.float32:
+        need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
+        if need and not single_token_decode:  # room for the prefill key split
+            need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
     if need and workspace is None:
         workspace = _workspace(dev, stream, need)
     ws_ptr = workspace.data_ptr() if workspace is not None else None

@@ -330,6 +330,15 @@ size_t emx_paged_prefill_workspace_bytes(int num_tokens, int num_seqs, int num_q
                                          int head_dim);
 
 /*
+ * The same for ragged calls of emx_paged_attention_dense (fp16 / bf16) and
+ * emx_paged_attention_fp8 over every shape their MFMA kernels take (head_dim
+ * 64, 128 or 256, pages of a multiple of 8 tokens, any GQA ratio up to 128, 64
+ * at head_dim 256): at least emx_paged_prefill_workspace_bytes(...).
+ */
+size_t emx_paged_ragged_workspace_bytes(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads,
+                                        int head_dim);
+
+/*
  * Paged attention over affine pages; queries/out fp16 [num_tokens, Hq, head_dim].
  * block_tables int32 [num_seqs, max_blocks_per_seq]; kv_lens int32 [num_seqs];
  * query_start_loc int32 [num_seqs+1].  single_token_decode != 0 means token i

@@ -111,3 +111,52 @@ def test_decode_infinities(cuda, kind):
     assert np.isposinf(got[1, 2:, 3]).all()
     got[1, 2:, 3] = exp[1, 2:, 3]
     check(b, got, exp)
+
+
+# chunks around the tile and step edges, over cached prefixes, beside single-token and empty rows
+RAGGED = [(33, 40), (1, 129), (2, 2), (130, 700), (1, 1), (0, 5), (65, 65), (7, 3), (1, 600), (5, 0), (64, 1300)]
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16", "fp8"])
+@pytest.mark.parametrize("d,page,hq,hkv", [(64, 16, 8, 2), (128, 16, 6, 2), (128, 24, 7, 1), (128, 8, 40, 2),
+                                           (128, 128, 4, 4), (256, 64, 4, 4), (256, 32, 16, 1)])
+def test_ragged(cuda, kind, d, page, hq, hkv):
+    if kind == "fp8" and page == 128:
+        pytest.skip("prefill_affine_d128's shape (tests/test_gpu_fp8.py)")
+    print(f"[token-major ragged {kind} d{d} page{page} {hq}/{hkv}]", flush=True)
+    b = batch(kind, [q for q, _ in RAGGED], [k for _, k in RAGGED], hq, hkv, d, page, seed=d + page + hq,
+              invalid=[(3, 1), (3, 2), (8, 0), (10, 3)] if page < 64 else [])
+    for window in (0, 50):
+        check(b, run(b, cuda, window, decode=False), expected(b, window))
+
+
+def test_ragged_without_workspace(cuda):
+    """The C entry point with no workspace: single-token rows go as query tiles, no tile is cut."""
+    from easymlx_amd import _native
+
+    print("[token-major ragged, no workspace]", flush=True)
+    b = batch("f16", [q for q, _ in RAGGED], [k for _, k in RAGGED], 4, 2, 128, 16, seed=5)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+    q, k, v = b["q"].to(cuda), b["cache"][0].to(cuda), b["cache"][1].to(cuda)
+    bt, kvl, qsl = t(b["tables"]), t(b["kvl"]), t(b["qsl"])
+    out = torch.full_like(q, 7.0)
+    _native.check(_native.load().emx_paged_attention_dense(
+        q.data_ptr(), q.shape[0], 4, 128, _native.DTYPE_F16, k.data_ptr(), v.data_ptr(), k.shape[0], 16, 2,
+        bt.data_ptr(), bt.shape[0], bt.shape[1], kvl.data_ptr(), qsl.data_ptr(), 1 / np.sqrt(128), 0, 0, None, 0,
+        out.data_ptr(), _native.stream_ptr(cuda)))
+    torch.cuda.synchronize()
+    check(b, out.double().cpu().numpy(), expected(b))
+
+
+def test_ragged_infinities(cuda):
+    """A value a row does not see (a later token of the prompt, a stale one) leaves it as it is."""
+    print("[token-major ragged infinities]", flush=True)
+    b = batch("bf16", [40, 1], [60, 30], 4, 2, 128, 16, seed=9)
+    exp = expected(b)
+    at = lambda s, p: (int(b["tables"][s, p // 16]), p % 16)  # noqa: E731
+    b["cache"][1][at(0, 55)][0, 7] = float("inf")  # query rows 35 .. 39 see it, kv head 0
+    b["cache"][1][at(1, 31)][1, 3] = float("nan")
+    got = run(b, cuda, decode=False)
+    assert np.isposinf(got[35:40, :2, 7]).all()
+    got[35:40, :2, 7] = exp[35:40, :2, 7]
+    check(b, got, exp)
