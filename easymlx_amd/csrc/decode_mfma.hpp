@@ -1,6 +1,6 @@
-// Single-token paged decode over token-major caches [nb, bs, Hkv, D]:
-// unquantized fp16 / bf16 and FP8 (E4M3, one fp32 scale per page), head_dim 64,
-// 128 or 256, pages of a multiple of 8 tokens, any GQA ratio.  MFMA, split-K, one
+// Single-token paged decode, head_dim 64, 128 or 256, any GQA ratio, over token-major
+// caches [nb, bs, Hkv, D] (unquantized fp16 / bf16, FP8 E4M3 with one fp32 scale per
+// page; pages of a multiple of 8 tokens) and over affine pages.  MFMA, split-K, one
 // launch.
 //
 // Replaces the reference's per-(seq, q_head) serial key loop
@@ -8,7 +8,7 @@
 // :611-775, FP8 :776-1268) and its split-K form (page_attention.py:1718-2059).
 //
 // Work: a unit is (sequence, kv head, up to 16 query heads), an item 128 tokens
-// of one unit (32 per wave).  Items are ordered unit-major and workgroup w of NWG
+// of one unit (32 per wave; 256 and 64 over 4-bit pages).  Items are ordered unit-major and workgroup w of NWG
 // takes the range [w I / NWG, (w + 1) I / NWG); a unit inside one range goes
 // straight to the output, a cut one leaves an fp32 partial per workgroup, merged
 // by the workgroup that arrives last (counter per unit, zero before and after).
@@ -21,6 +21,11 @@
 //          lane (h, jj) holds, so P needs no lane exchange.  Lane (i, jj) loads dims
 //          D/16 i .. of those eight tokens (whole rows per 16 lanes) and sub-tile b
 //          takes dim D/16 i + b, picked by byte permutes.
+// Affine pages (as decode_affine.hpp, without its limits on head_dim and GQA): K rows are
+// taken in the order token TPL (i / 4) + 4 t + i % 4, so that lane (h, jj) ends with the
+// scores of TPL consecutive tokens, the tokens of the dim-major value words it loads; one
+// accumulator per quantization group, scale and bias applied in fp32 after the MFMA; the
+// value scale enters the probability before it is split, sum p * v_bias is kept in fp32.
 // K of the next item is loaded as soon as QK^T has consumed this one's registers,
 // V after PV: one register image, always in flight.
 //
@@ -34,30 +39,57 @@
 
 namespace emx {
 
-constexpr int kDecodeMfmaNT = 128;  // tokens per workgroup item
-
 struct DecodeMfmaArgs {
-  DecodeArgs d;      // kc / vc: the caches; nt = kDecodeMfmaNT; ws_cnt, ws_o [slot][hc][D], ws_ml [slot][hc][2]
+  DecodeArgs d;      // kc / vc: the caches; nt: DecodeMfmaCfg::NT; ws_cnt, ws_o [slot][hc][D], ws_ml [slot][hc][2]
   int hc, nhc;       // query heads per unit (<= 16) and units per kv head
   uint32_t inv_bs;   // ceil(2^32 / bs)
 };
 
+// Items longer than this many on average are cut freely; below, a unit that would be cut
+// costs its merge (a round trip through memory, the atomic and the partials: ~6 us, six
+// items' time) more than the balance gains, and ranges start at unit starts.
+constexpr int kDecodeMfmaMergeItems = 6;
+
 template <class C, int D>
 struct DecodeMfmaCfg {
-  static constexpr int EB = sizeof(typename C::ET);   // bytes per cache element
+  static constexpr int EB = sizeof(typename C::ET);   // bytes per cache element (token-major)
   static constexpr int KS = D / 32;                   // QK^T k-slices
+  static constexpr int SB = D / 16;                   // PV sub-tiles
+  static constexpr int NTW = 32;                      // tokens of a wave's item
+  static constexpr int NT = 4 * NTW;                  // tokens of an item
+  static constexpr int NA = NTW / 16;                 // QK^T sub-tiles
+  static constexpr int NV = NTW / 4;                  // scores per lane
   static constexpr int KL = D * EB / 64;              // 16-byte K loads per row (per lane)
-  static constexpr int SB = D / 16;                   // PV sub-tiles; dims a lane holds
-  static constexpr int VW = SB * EB / 4;              // V words a lane holds per token
+  static constexpr int KW = KL * 4;                   // K words a lane holds per sub-tile
+  static constexpr int VN = NTW / 4, VW = SB * EB / 4;  // tokens, words per token of V a lane holds
+  static constexpr int NL = 4;                        // page lookups per item
+  static constexpr int G = 1, SNI = 1, STAGE = 0;
   static constexpr int RD = D < 128 ? D : 128;        // dims combined per round
   static constexpr int XS = RD + 4;                   // LDS stride of a head's combined dims
+};
+template <int BITS, int GS, int D>
+struct DecodeMfmaCfg<KvAffine<BITS, GS>, D> {
+  static constexpr int KS = D / 32, SB = D / 16;
+  static constexpr int NTW = 256 / BITS, NT = 4 * NTW, NA = NTW / 16, NV = NTW / 4;
+  static constexpr int BD = GS < 64 ? GS : 64;        // dims of a K block: one quantization group
+  static constexpr int LD = BD / 4;                   // dims of a block a lane holds
+  static constexpr int BW = LD * BITS / 32;           // words of them
+  static constexpr int KW = (D / BD) * BW;
+  static constexpr int VN = SB, VW = 2;               // V: dims a lane holds, words of each (its NV tokens)
+  static constexpr int G = D / GS;
+  static constexpr int NP = 4 * G * NTW / 8;          // 16-byte scale pieces of an item
+  static constexpr int SNI = (NP + 63) / 64;
+  static constexpr int NL = 2 + SNI;
+  static constexpr int STAGE = 4 * G * NTW;           // halves of a wave's scale slot
+  static constexpr int RD = D < 128 ? D : 128, XS = RD + 4;
 };
 
 template <class C, int D>
 struct DecodeMfmaLoads {
   using P = DecodeMfmaCfg<C, D>;
-  uint32_t k[2][P::KL * 4];
-  uint32_t v[8][P::VW];
+  uint32_t k[P::NA][P::KW];
+  uint32_t v[P::VN][P::VW];
+  u32x4 s[P::SNI];  // affine: scale pieces
 };
 
 // MFMA operand of K k-slice w from the loaded words of one row.  16-bit: load w
@@ -116,7 +148,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   typedef typename C::Op Op;
   typedef typename C::QT QT;
   const DecodeArgs& a = A.d;
-  constexpr int NT = kDecodeMfmaNT;
+  constexpr int NT = P::NT;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -127,13 +159,15 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   constexpr int oCum = 0, oKvl = lds_next(oCum, 4 * (kMaxSeqs + 1)), oQrw = lds_next(oKvl, 4 * kMaxSeqs);
   constexpr int oXo = lds_next(oQrw, 4 * kMaxSeqs), oXml = lds_next(oXo, 4 * 4 * 16 * P::XS);
   constexpr int oFlag = lds_next(oXml, 4 * 4 * 16 * 2), oEnd = lds_next(oFlag, 16);
-  static_assert(oEnd <= kArenaBytes, "LDS arena too small");
+  constexpr int oStage = oXo;  // (an item's scales are read before its unit's combine, on every wave)
+  static_assert(oEnd <= kArenaBytes && 2 * 4 * P::STAGE <= oXml - oXo, "LDS arena too small");
   int(&cum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oCum);
   int(&kvl)[kMaxSeqs] = lds_at<int[kMaxSeqs]>(oKvl);
   int(&qrw)[kMaxSeqs] = lds_at<int[kMaxSeqs]>(oQrw);
   float* xo = &lds_at<float>(oXo);      // [wave][head][XS]
   float* xml = &lds_at<float>(oXml);    // [wave][head][2]
   int& flag = lds_at<int>(oFlag);
+  h16* stage = &lds_at<h16>(oStage) + wv * P::STAGE;  // affine: this wave's [array][group][token] scales
   seq_table(a, cum, kvl, qrw);
   const int S = a.S, HG = a.Hq / a.Hkv, Hu = a.Hkv * A.nhc;
   {  // decoded sequences without a live token produce zeros (the reference's l == 0 case)
@@ -147,7 +181,35 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   const long long I = (long long)Hu * uru(cum[S]);
   const int NW = (int)min((long long)nblocks, I);
   if (bid >= NW) return;
-  const long long g0 = (long long)bid * I / NW, g1 = (long long)(bid + 1) * I / NW;
+  // The sequence of item g; the most items a unit has.
+  auto seq_of = [&](const long long g) {
+    int s = 0;
+    for (int c = 0; c < S; c += 64) {
+      const int si = c + lane;
+      s += __builtin_popcountll(__ballot(si < S && (long long)Hu * cum[si + 1] <= g));
+    }
+    return uru(s);
+  };
+  int nmax = 0;
+  for (int c = 0; c < S; c += 64) {
+    const int si = c + lane;
+    nmax = max(nmax, si < S ? cum[si + 1] - cum[si] : 0);
+  }
+  nmax = uru((int)wave_max((float)nmax));
+  const bool cut = (long long)(nmax - kDecodeMfmaMergeItems) * NW > I;
+  long long g0 = (long long)bid * I / NW, g1 = (long long)(bid + 1) * I / NW;
+  if (!cut) {  // whole units: those whose first item lies in the range
+    auto unit_ceil = [&](const long long g) {
+      if (g >= I) return I;
+      const int s = seq_of(g);
+      const long long b = (long long)Hu * uru(cum[s]);
+      const int n = uru(cum[s + 1]) - uru(cum[s]);
+      return b + (long long)uru(((int)(g - b) + n - 1) / n) * n;
+    };
+    g0 = unit_ceil(g0);
+    g1 = unit_ceil(g1);
+    if (g0 >= g1) return;
+  }
 
   auto start_of = [&](int kl) { return a.window > 0 ? max(0, kl - a.window) : 0; };
   // An item: item j of the n of unit y of sequence s; this wave's tokens start at tb.
@@ -155,15 +217,10 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     int s, y, j, n, kl, st, tb;
     bool has;  // inside the range
   };
-  auto tb_of = [&](int st, int jx) { return (st / NT + jx) * NT + 32 * wv; };
+  auto tb_of = [&](int st, int jx) { return (st / NT + jx) * NT + P::NTW * wv; };
   Item it0;
   {
-    int s = 0;
-    for (int c = 0; c < S; c += 64) {
-      const int si = c + lane;
-      s += __builtin_popcountll(__ballot(si < S && (long long)Hu * cum[si + 1] <= g0));
-    }
-    it0.s = uru(s);
+    it0.s = seq_of(g0);
     it0.n = uru(cum[it0.s + 1]) - uru(cum[it0.s]);
     const int r = (int)(g0 - (long long)Hu * uru(cum[it0.s]));
     it0.y = uru(r / it0.n);
@@ -194,74 +251,149 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     return r;
   };
 
-  const size_t rowb = (size_t)a.Hkv * D * P::EB;  // bytes between a page's tokens
   const char* kbase = reinterpret_cast<const char*>(a.kc);
   const char* vbase = reinterpret_cast<const char*>(a.vc);
+  auto ok_blk = [&](int b) { return (unsigned)b < (unsigned)a.nb; };
 
-  // Page lookups of one item: K rows of tokens 16 t + i, and the quads 16 t + 4 jj
-  // (V rows; FP8 page scales).  Positions past the end repeat the last live token.
+  // Page lookups of one item.  Token-major: K rows of tokens 16 t + i (n = 0, 1) and the
+  // quads 16 t + 4 jj (n = 2, 3: V rows, FP8 page scales), positions past the end
+  // repeating the last live token.  Affine: the NV tokens of the lane's K rows (n = 0), of its
+  // value words (n = 1), the 8 tokens of its scale pieces (n = 2 ..); a group past the end
+  // repeats the last live one.
   struct Look {
-    int blk[4];  // [K t = 0, 1; quad t = 0, 1]
+    int blk[P::NL];
   };
-  auto pos_of = [&](const Item& x, int n) { return min(x.tb + 16 * (n & 1) + (n < 2 ? col : 4 * jj), x.kl - 1); };
+  // affine: scale piece i of the lane: segment (array, group), 8 tokens (lanes past the last repeat it)
+  auto piece_of = [&](int i) {
+    if constexpr (C::kAffine) return min(64 * i + lane, P::NP - 1);
+    return 0;
+  };
+  auto pos_of = [&](const Item& x, int n) {
+    if constexpr (C::kAffine) {
+      if (n < 2) return min(x.tb + P::NV * (n == 0 ? col >> 2 : jj), (x.kl - 1) & ~(P::NV - 1));
+      return min(x.tb + 8 * (piece_of(n - 2) % (P::NTW / 8)), (x.kl - 1) & ~7);
+    } else {
+      return min(x.tb + 16 * (n & 1) + (n < 2 ? col : 4 * jj), x.kl - 1);
+    }
+  };
   auto lookup = [&](Look& L, const Item& x) {
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
+    for (int n = 0; n < P::NL; ++n)
       L.blk[n] = a.block_tables[(size_t)x.s * a.max_blocks + page_of(pos_of(x, n), A.inv_bs)];
   };
-  auto ok_blk = [&](int b) { return (unsigned)b < (unsigned)a.nb; };
-  auto row_of = [&](const Look& L, int n, const Item& x) {
-    const int p = pos_of(x, n);
-    const int b = ok_blk(L.blk[n]) ? L.blk[n] : 0;
-    return ((size_t)b * a.bs + (p - page_of(p, A.inv_bs) * a.bs)) * rowb + (size_t)(x.y / A.nhc) * (D * P::EB);
-  };
 
-  // (an item past the range: every lane reads the cache's first row, one line; the loads are
+  // (an item past the range: every lane reads the cache's first bytes, one line; the loads are
   // issued on every path, so that the wait before a use never drains the ones behind it)
   DecodeMfmaLoads<C, D> ld;
   float ks[2] = {1.f, 1.f}, vs[2] = {1.f, 1.f}, ks1[2], vs1[2];  // FP8 page scales: this item's, the next one's
+  // token-major: byte offset of the row of lookup n
+  const size_t rowb = (size_t)a.Hkv * D * (C::kAffine ? 1 : sizeof(typename C::ET));
+  auto row_of = [&](const Look& L, int n, const Item& x) {
+    const int p = pos_of(x, n);
+    const int b = ok_blk(L.blk[n]) ? L.blk[n] : 0;
+    return ((size_t)b * a.bs + (p - page_of(p, A.inv_bs) * a.bs)) * rowb +
+           (size_t)(x.y / A.nhc) * (D * sizeof(typename C::ET));
+  };
+  // affine: page-head and offset of lookup n's first token
+  auto ph_of = [&](const Look& L, int n, const Item& x, int& off) {
+    const int p = pos_of(x, n);
+    off = p - page_of(p, A.inv_bs) * a.bs;
+    return (size_t)(ok_blk(L.blk[n]) ? L.blk[n] : 0) * a.Hkv + x.y / A.nhc;
+  };
   auto issue_k = [&](const Look& L, const Item& x) {
-    if constexpr (C::kFp8) {
+    if constexpr (C::kAffine) {
+      constexpr int B = C::kBits;
+#pragma unroll
+      for (int i = 0; i < P::SNI; ++i) {
+        const int seg = piece_of(i) / (P::NTW / 8), arr = seg / P::G, g = seg % P::G;
+        int off;
+        const size_t ph = ph_of(L, 2 + i, x, off);
+        const h16 *b_ks = a.ks, *b_kb = a.kb, *b_vs = a.vs, *b_vb = a.vb;
+        asm("" : "+s"(b_ks), "+s"(b_kb), "+s"(b_vs), "+s"(b_vb));  // picked from registers, not by a vector load
+        const h16* base = arr == 0 ? b_ks : arr == 1 ? b_kb : arr == 2 ? b_vs : b_vb;
+        typedef const __attribute__((address_space(1))) u32x4* gu32x4;
+        ld.s[i] = *(gu32x4)(base + (x.has ? (ph * P::G + g) * a.bs + off : 0));
+      }
+      int off;
+      const size_t ph = ph_of(L, 0, x, off);
+      // K rows of tokens 4 t + i % 4 of the lane's group; a block's BD dims over the four lane groups
+      const char* p = kbase + (x.has ? (ph * a.bs + off + (col & 3)) * (D * B / 8) + jj * (P::BW * 4) : 0);
+#pragma unroll
+      for (int t = 0; t < P::NA; ++t)
+#pragma unroll
+        for (int bl = 0; bl < D / P::BD; ++bl) {
+          const char* q = p + (x.has ? 4 * t * (D * B / 8) + bl * (P::BD * B / 8) : 0);
+          uint32_t* dst = &ld.k[t][bl * P::BW];
+          if constexpr (P::BW == 4) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(q);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) dst[c] = v[c];
+          } else if constexpr (P::BW == 2) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(q);
+            dst[0] = v[0];
+            dst[1] = v[1];
+          } else {
+            dst[0] = *reinterpret_cast<const uint32_t*>(q);
+          }
+        }
+    } else {
+      if constexpr (C::kFp8) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int b = ok_blk(L.blk[2 + t]) ? L.blk[2 + t] : 0;
+          ks1[t] = a.kps[b];
+          vs1[t] = a.vps[b];
+        }
+      }
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const int b = ok_blk(L.blk[2 + t]) ? L.blk[2 + t] : 0;
-        ks1[t] = a.kps[b];
-        vs1[t] = a.vps[b];
-      }
-    }
+        const char* p = kbase + (x.has ? row_of(L, t, x) + 16 * jj : 0);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const char* p = kbase + (x.has ? row_of(L, t, x) + 16 * jj : 0);
+        for (int w = 0; w < P::KL; ++w) {
+          const u32x4 v = *reinterpret_cast<const u32x4*>(p + (x.has ? 64 * w : 0));
 #pragma unroll
-      for (int w = 0; w < P::KL; ++w) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p + (x.has ? 64 * w : 0));
-#pragma unroll
-        for (int c = 0; c < 4; ++c) ld.k[t][4 * w + c] = v[c];
+          for (int c = 0; c < 4; ++c) ld.k[t][4 * w + c] = v[c];
+        }
       }
     }
   };
   auto issue_v = [&](const Look& L, const Item& x) {
+    if constexpr (C::kAffine) {
+      // two words per dim 16 b + i: the lane's NV tokens (one page: bs % NV == 0)
+      constexpr int B = C::kBits;
+      int off;
+      const size_t ph = ph_of(L, 1, x, off);
+      const int T = min(a.bs, P::NTW);  // tokens of a value tile
+      const size_t w0 = x.has ? v_word_index<B>(ph, off, col, D, a.bs) : 0;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      // the quad's tokens lie in one page (bs % 8 == 0); past the end they repeat the last live one
-      const size_t r0 = x.has ? row_of(L, 2 + t, x) + (size_t)col * (4 * P::VW) : 0;
-      const int left = x.has ? x.kl - 1 - pos_of(x, 2 + t) : 0;
+      for (int b = 0; b < P::SB; ++b) {
+        const u32x2 v = *reinterpret_cast<const u32x2*>(a.vc + w0 + (x.has ? 16 * b * (T * B / 32) : 0));
+        ld.v[b][0] = v[0];
+        ld.v[b][1] = v[1];
+      }
+    } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t* w = reinterpret_cast<const uint32_t*>(vbase + r0 + (size_t)min(r, left) * rowb);
-        uint32_t(&dst)[P::VW] = ld.v[4 * t + r];
-        if constexpr (P::VW == 1) {
-          dst[0] = w[0];
-        } else if constexpr (P::VW == 2) {
-          const u32x2 v = *reinterpret_cast<const u32x2*>(w);
-          dst[0] = v[0];
-          dst[1] = v[1];
-        } else {
+      for (int t = 0; t < 2; ++t) {
+        // the quad's tokens lie in one page (bs % 8 == 0); past the end they repeat the last live one
+        const size_t r0 = x.has ? row_of(L, 2 + t, x) + (size_t)col * (4 * P::VW) : 0;
+        const int left = x.has ? x.kl - 1 - pos_of(x, 2 + t) : 0;
 #pragma unroll
-          for (int c = 0; c < P::VW / 4; ++c) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(w + 4 * c);
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t* w = reinterpret_cast<const uint32_t*>(vbase + r0 + (size_t)min(r, left) * rowb);
+          uint32_t(&dst)[P::VW] = ld.v[4 * t + r];
+          if constexpr (P::VW == 1) {
+            dst[0] = w[0];
+          } else if constexpr (P::VW == 2) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(w);
+            dst[0] = v[0];
+            dst[1] = v[1];
+          } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) dst[4 * c + e] = v[e];
+            for (int c = 0; c < P::VW / 4; ++c) {
+              const u32x4 v = *reinterpret_cast<const u32x4*>(w + 4 * c);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) dst[4 * c + e] = v[e];
+            }
           }
         }
       }
@@ -270,24 +402,51 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
 
   // query operand of a unit: column h = query head h (zero past the unit's heads)
   Op qB[P::KS];
+  float qsum[P::G] = {};  // affine: the query's sum over each quantization group
   auto load_q = [&](int si, int yy) {
     const int kh = yy / A.nhc, h0 = (yy % A.nhc) * A.hc;
     const int nh = min(A.hc, HG - h0);
     const QT* qp = reinterpret_cast<const QT*>(a.q) +
                    ((size_t)qrw[si] * a.Hq + (size_t)kh * HG + h0 + (col < nh ? col : 0)) * D;
+    if constexpr (C::kAffine) {
+#pragma unroll
+      for (int g = 0; g < P::G; ++g) qsum[g] = 0.f;
+    }
 #pragma unroll
     for (int w = 0; w < P::KS; ++w) {
-      const int d = C::kFp8 ? 64 * (w >> 1) + 16 * jj + 8 * (w & 1) : 32 * w + 8 * jj;
+      int d;
+      if constexpr (C::kAffine)
+        d = P::BD * (w / (P::LD / 8)) + P::LD * jj + 8 * (w % (P::LD / 8));
+      else
+        d = C::kFp8 ? 64 * (w >> 1) + 16 * jj + 8 * (w & 1) : 32 * w + 8 * jj;
       const u32x4 x = *reinterpret_cast<const u32x4*>(qp + d);
-      qB[w] = __builtin_bit_cast(Op, col < nh ? x : u32x4{0u, 0u, 0u, 0u});
+      const Op v = __builtin_bit_cast(Op, col < nh ? x : u32x4{0u, 0u, 0u, 0u});
+      if constexpr (C::kAffine) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          qB[w][i] = v[slot_perm<C::kBits>(i)];  // the unpacked codes' order
+          qsum[32 * w / C::kGS] += (float)v[i];
+        }
+      } else {
+        qB[w] = v;
+      }
+    }
+    if constexpr (C::kAffine) {
+#pragma unroll
+      for (int g = 0; g < P::G; ++g) qsum[g] = rows4_sum(qsum[g]);
     }
   };
 
   float m_run = -INFINITY, l_part = 0.f;
   f32x4 acc[P::SB];
+  float pb[P::G];  // affine: sum p * v_bias per group
+  int vexp = 0;    // affine: acc holds the sum / 2^vexp
   auto clear = [&]() {
     m_run = -INFINITY;
     l_part = 0.f;
+    vexp = -60;
+#pragma unroll
+    for (int g = 0; g < P::G; ++g) pb[g] = 0.f;
 #pragma unroll
     for (int b = 0; b < P::SB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
@@ -306,39 +465,102 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   for (long long g = g0; g < g1; ++g) {
     const int s = cur.s, y = cur.y, n_s = cur.n, tb = cur.tb, kv_len = cur.kl, start_k = cur.st;
     const Item n2 = nxt.has ? after(nxt, g + 1) : nxt;
-    // ---- scores
-    float sc[8];
-    if constexpr (C::kFp8) {
+    // ---- scores: lane (h, jj), element 4 t + r
+    constexpr int NV = P::NV;
+    float sc[NV];
+    bool okp = ok_blk(lc.blk[1]);
+#pragma unroll
+    for (int n = 2; n < P::NL; ++n) okp = okp && ok_blk(lc.blk[n]);
+    const bool full = tb >= start_k && tb + P::NTW <= kv_len && __all(okp);
+    if constexpr (C::kAffine) {
+      // ---- this item's scales to the wave's LDS slot; those of tokens outside
+      // [start_k, kv_len) or on an invalid page (which may hold anything) as zeros
+      int vmax = 0;  // largest |v_scale|, as fp16 bits
+#pragma unroll
+      for (int i = 0; i < P::SNI; ++i) {
+        const int pc = piece_of(i), p0 = tb + 8 * (pc % (P::NTW / 8));
+        u32x4 x = ld.s[i];
+        if (!full) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const bool ok0 = p0 + 2 * e >= start_k && p0 + 2 * e < kv_len && ok_blk(lc.blk[2 + i]);
+            const bool ok1 = p0 + 2 * e + 1 >= start_k && p0 + 2 * e + 1 < kv_len && ok_blk(lc.blk[2 + i]);
+            x[e] &= (ok0 ? 0x0000FFFFu : 0u) | (ok1 ? 0xFFFF0000u : 0u);
+          }
+        }
+        if (pc / (P::NTW / 8) / P::G == 2) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) vmax = max(vmax, (int)max(x[e] & 0x7FFFu, (x[e] >> 16) & 0x7FFFu));
+        }
+        if (64 * i + lane < P::NP) *reinterpret_cast<u32x4*>(stage + 8 * pc) = x;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // the accumulator's exponent follows the value scales', so that p * v_scale keeps to the
+      // middle of fp16's range (exact powers of two; 6 binades of slack below)
+      const int ex = ((int)wave_max((float)vmax) >> 10) - 15;
+      if (ex > vexp || ex < vexp - 6) {
+        const float f = __uint_as_float((uint32_t)(127 + vexp - ex) << 23);
+#pragma unroll
+        for (int b = 0; b < P::SB; ++b) acc[b] *= f;
+        vexp = ex;
+      }
+#pragma unroll
+      for (int t = 0; t < P::NA; ++t) {
+        f32x4 c[P::G];
+#pragma unroll
+        for (int g = 0; g < P::G; ++g) c[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < P::KS; ++w) {
+          const uint32_t* k = &ld.k[t][w * C::kBits / 4];
+          c[32 * w / C::kGS] = mfma_op(C::kBits == 4 ? unpack4(k[0]) : unpack8(k[0], k[1]), qB[w], c[32 * w / C::kGS]);
+        }
+        typedef h16 h16x4v __attribute__((ext_vector_type(4)));
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int g = 0; g < P::G; ++g) {
+          const h16x4v ks4 = *reinterpret_cast<const h16x4v*>(stage + g * P::NTW + NV * jj + 4 * t);
+          const h16x4v kb4 = *reinterpret_cast<const h16x4v*>(stage + (P::G + g) * P::NTW + NV * jj + 4 * t);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            v[r] = fmaf(c[g][r] * kTwo24, (float)ks4[r], fmaf((float)kb4[r], qsum[g], v[r]));
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[4 * t + r] = v[r];
+      }
+    } else {
+      if constexpr (C::kFp8) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          ks[t] = ks1[t];
+          vs[t] = vs1[t];
+        }
+      }
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        ks[t] = ks1[t];
-        vs[t] = vs1[t];
+        f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < P::KS; ++w) c = mfma_op(k_operand<C, D>(ld.k[t], w), qB[w], c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[4 * t + r] = C::kFp8 ? c[r] * (ks[t] * 256.f) : c[r];
       }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      f32x4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < P::KS; ++w) c = mfma_op(k_operand<C, D>(ld.k[t], w), qB[w], c);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sc[4 * t + r] = C::kFp8 ? c[r] * (ks[t] * 256.f) : c[r];
     }
     issue_k(ln, nxt);
     lookup(l2, n2);
     const bool unit_end = !nxt.has || nxt.s != s || nxt.y != y;
 
     // ---- mask: outside [start_k, kv_len), or on a page with an invalid id
-    const bool okq = ok_blk(lc.blk[2]) && ok_blk(lc.blk[3]);
-    if (tb < start_k || tb + 32 > kv_len || !__all(okq)) {
+    if (!full) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int p = tb + 16 * (e >> 2) + 4 * jj + (e & 3);
-        if (p < start_k || p >= kv_len || !ok_blk(lc.blk[2 + (e >> 2)])) sc[e] = -INFINITY;
+      for (int e = 0; e < NV; ++e) {
+        const int p = tb + (C::kAffine ? NV * jj + e : 16 * (e >> 2) + 4 * jj + (e & 3));
+        if (p < start_k || p >= kv_len || !ok_blk(lc.blk[C::kAffine ? 1 : 2 + (e >> 2)])) sc[e] = -INFINITY;
       }
     }
     float tmax = -INFINITY;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) tmax = fmaxf(tmax, sc[e]);
+    for (int e = 0; e < NV; ++e) tmax = fmaxf(tmax, sc[e]);
     tmax = rows4_max(tmax) * a.scale_log2;
     const float m_new = fmaxf(m_run, tmax);
     if (__any(m_new != m_run)) {
@@ -346,37 +568,64 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       l_part *= alpha;
 #pragma unroll
       for (int b = 0; b < P::SB; ++b) acc[b] *= alpha;
+#pragma unroll
+      for (int g = 0; g < P::G; ++g) pb[g] *= alpha;
       m_run = m_new;
     }
     const float m_sub = fmaxf(m_run, -3.0e38f) - kPBias;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < NV; ++e) {
       sc[e] = __builtin_amdgcn_exp2f(fmaf(sc[e], a.scale_log2, -m_sub));
       l_part += sc[e];
     }
-    float post = 1.f;
-    if constexpr (C::kFp8) {
-      // p * (value page scale), brought near 1 by a power of two taken out after the MFMA
-      const float vmax = rows4_max(fmaxf(vs[0], vs[1]));
-      const int ex = min(max((int)((__float_as_uint(vmax) >> 23) & 0xFFu) - 127, -100), 100);
-      const float down = __uint_as_float((uint32_t)(127 - ex) << 23);
-      post = __uint_as_float((uint32_t)(127 + ex + 8) << 23);  // the codes enter as value * 2^-8
+    if constexpr (C::kAffine) {
+      const float down = __uint_as_float((uint32_t)(127 - vexp) << 23);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sc[e] *= vs[e >> 2] * down;
-    }
-    Op pB[C::kParts];
-    split_p(sc, pB);
+      for (int w = 0; w < NV / 8; ++w)
 #pragma unroll
-    for (int b = 0; b < P::SB; ++b) {
-      const Op V = v_operand<C, P::VW>(ld.v, b);
-      f32x4 t = C::kFp8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[b];
+        for (int g = 0; g < P::G; ++g) {
+          const h16x8 vs8 = *reinterpret_cast<const h16x8*>(stage + (2 * P::G + g) * P::NTW + NV * jj + 8 * w);
+          const h16x8 vb8 = *reinterpret_cast<const h16x8*>(stage + (3 * P::G + g) * P::NTW + NV * jj + 8 * w);
+          float x[8];
 #pragma unroll
-      for (int k = 0; k < C::kParts; ++k) t = mfma_op(V, pB[k], t);
+          for (int i = 0; i < 8; ++i) {
+            x[i] = sc[8 * w + i] * ((float)vs8[i] * down);
+            pb[g] = fmaf(sc[8 * w + i], (float)vb8[i], pb[g]);
+          }
+          Op pB[C::kParts];
+          split_p(x, pB);
+#pragma unroll
+          for (int b = g * (C::kGS / 16); b < (g + 1) * (C::kGS / 16); ++b) {
+            const Op V = C::kBits == 4 ? unpack4(ld.v[b][w]) : unpack8(ld.v[b][0], ld.v[b][1]);
+#pragma unroll
+            for (int k = 0; k < C::kParts; ++k) acc[b] = mfma_op(V, pB[k], acc[b]);
+          }
+        }
+    } else {
+      float post = 1.f;
       if constexpr (C::kFp8) {
+        // p * (value page scale), brought near 1 by a power of two taken out after the MFMA
+        const float vmax = rows4_max(fmaxf(vs[0], vs[1]));
+        const int ex = min(max((int)((__float_as_uint(vmax) >> 23) & 0xFFu) - 127, -100), 100);
+        const float down = __uint_as_float((uint32_t)(127 - ex) << 23);
+        post = __uint_as_float((uint32_t)(127 + ex + 8) << 23);  // the codes enter as value * 2^-8
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(t[r], post, acc[b][r]);
-      } else {
-        acc[b] = t;
+        for (int e = 0; e < 8; ++e) sc[e] *= vs[e >> 2] * down;
+      }
+      Op pB[C::kParts];
+      split_p(sc, pB);
+#pragma unroll
+      for (int b = 0; b < P::SB; ++b) {
+        const Op V = v_operand<C, P::VW>(ld.v, b);
+        f32x4 t = C::kFp8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[b];
+#pragma unroll
+        for (int k = 0; k < C::kParts; ++k) t = mfma_op(V, pB[k], t);
+        if constexpr (C::kFp8) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[b][r] = fmaf(t[r], post, acc[b][r]);
+        } else {
+          acc[b] = t;
+        }
       }
     }
     issue_v(ln, nxt);
@@ -395,6 +644,15 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       }
       float l = l_part + __shfl_xor(l_part, 16, 64);
       l += __shfl_xor(l, 32, 64);
+      if constexpr (C::kAffine) {  // codes entered as code * 2^-24; the bias term joins its group's dims
+        const float f = __uint_as_float((uint32_t)(127 + vexp + 24) << 23);
+#pragma unroll
+        for (int g = 0; g < P::G; ++g) {
+          const float bias = rows4_sum(pb[g]);
+#pragma unroll
+          for (int b = g * (C::kGS / 16); b < (g + 1) * (C::kGS / 16); ++b) acc[b] = acc[b] * f + bias;
+        }
+      }
       bool bad = false;
       QT* out = reinterpret_cast<QT*>(a.out) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0) * D;
       const __amdgpu_buffer_rsrc_t ro =
@@ -405,15 +663,22 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       for (int rd = 0; rd < D / P::RD; ++rd) {
         __syncthreads();  // (the previous combine has been read)
         constexpr int BR = P::SB / (D / P::RD);  // sub-tiles of the round
+        float* xw = xo + (wv * 16 + col) * P::XS;
+        if constexpr (C::kAffine) {  // sub-tile b, row 4 jj + r: dim 16 b + 4 jj + r
+          if (col < nh) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int b = 0; b < BR; b += 4) {
-            const f32x4 x = {acc[rd * BR + b][r], acc[rd * BR + b + 1][r], acc[rd * BR + b + 2][r],
-                             acc[rd * BR + b + 3][r]};
-            if (col < nh)
-              *reinterpret_cast<f32x4*>(xo + (wv * 16 + col) * P::XS + (4 * jj + r) * BR + b) = x;
+            for (int b = 0; b < BR; ++b) *reinterpret_cast<f32x4*>(xw + 16 * b + 4 * jj) = acc[rd * BR + b];
           }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int b = 0; b < BR; b += 4) {
+              const f32x4 x = {acc[rd * BR + b][r], acc[rd * BR + b + 1][r], acc[rd * BR + b + 2][r],
+                               acc[rd * BR + b + 3][r]};
+              if (col < nh) *reinterpret_cast<f32x4*>(xw + (4 * jj + r) * BR + b) = x;
+            }
+        }
         if (rd == 0 && jj == 0 && col < nh) {
           xml[(wv * 16 + col) * 2] = m_run;
           xml[(wv * 16 + col) * 2 + 1] = l;
@@ -434,7 +699,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
             L = fmaf(xml[(w * 16 + h) * 2 + 1], f, L);
           }
           // element 4 c + k of the round is dim SB * row + rd * BR + ..: contiguous in k
-          const int dim = (4 * c / BR) * P::SB + rd * BR + (4 * c) % BR;
+          const int dim = C::kAffine ? rd * P::RD + 4 * c : (4 * c / BR) * P::SB + rd * BR + (4 * c) % BR;
           if (whole) {
             bad |= write4(O, L, out + (size_t)h * D + dim);
           } else {

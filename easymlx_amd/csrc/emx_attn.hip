@@ -391,29 +391,45 @@ int launch_generic_only(const emx::GenericArgs& ga, const KV& kv, hipStream_t st
   return check_launch("paged_generic");
 }
 
-// A call over a token-major cache (unquantized, FP8) with what `ga` holds.
-emx::TokenMajorCall token_major_call(emx::KvKind kind, const emx::GenericArgs& ga, const void* k, const void* v,
-                                     const float* kps, const float* vps) {
-  return emx::TokenMajorCall{kind, ga.q, ga.out, k, v, kps, vps, ga.block_tables, ga.kv_lens,
-                             ga.decode ? nullptr : ga.qsl, ga.T, ga.S, ga.Hq, ga.Hkv, ga.D, ga.bs, ga.nb,
-                             ga.max_blocks, ga.scale_log2, ga.window};
+// What `ga` holds, over the given cache, as a call of the MFMA kernels.
+emx::MfmaCall mfma_call(emx::KvKind kind, const emx::GenericArgs& ga, const void* k, const void* v) {
+  emx::MfmaCall c{};
+  c.kind = kind;
+  c.q = ga.q;
+  c.out = ga.out;
+  c.k = k;
+  c.v = v;
+  c.block_tables = ga.block_tables;
+  c.kv_lens = ga.kv_lens;
+  c.qsl = ga.decode ? nullptr : ga.qsl;
+  c.T = ga.T;
+  c.S = ga.S;
+  c.Hq = ga.Hq;
+  c.Hkv = ga.Hkv;
+  c.D = ga.D;
+  c.bs = ga.bs;
+  c.nb = ga.nb;
+  c.max_blocks = ga.max_blocks;
+  c.scale_log2 = ga.scale_log2;
+  c.window = ga.window;
+  return c;
 }
 
 // Runs the call on the MFMA kernels where they take its shape; false: nothing launched.
 // Single-token calls need the workspace for their partials; ragged calls use it for the
 // single-token rows and, when it is larger, for cut tiles.
-bool run_token_major(const emx::TokenMajorCall& c, void* ws, size_t ws_bytes, hipStream_t st, int* rc) {
+bool run_mfma(const emx::MfmaCall& c, void* ws, size_t ws_bytes, hipStream_t st, int* rc) {
   const size_t need = emx_paged_workspace_bytes(c.S, c.Hq, c.Hkv, c.D, c.max_blocks, c.bs);
   const bool have = ws && need > 0 && ws_bytes >= need;
   int* wi = static_cast<int*>(ws);
   float* partials = have ? reinterpret_cast<float*>(wi + kPartialsInt) : nullptr;
   if (!c.qsl) {
-    if (!have || c.S != c.T || !emx::token_major_ok(c)) return false;
+    if (!have || c.S != c.T || !emx::mfma_ok(c)) return false;
     emx::launch_decode_mfma(c, wi, partials, st);
     *rc = check_launch("decode_mfma");
     return true;
   }
-  if (!emx::mixed_mfma_ok(c)) return false;
+  if (c.kind == emx::KvKind::affine || !emx::mixed_mfma_ok(c)) return false;
   const size_t part = emx::mixed_mfma_part_bytes(c.T, c.S, c.Hq, c.Hkv, c.D, emx::kPrefillCounters);
   const size_t base = (need + 255) & ~(size_t)255;
   const bool cut = have && part > 0 && ws_bytes >= base + part;
@@ -1229,6 +1245,16 @@ int emx_paged_attention_affine(const void* queries, int num_tokens, int num_q_he
   ga.scale_log2 = scale_log2;
   ga.window = window;
   ga.decode = single_token_decode ? 1 : 0;
+  {
+    emx::MfmaCall c = mfma_call(emx::KvKind::affine, ga, k_codes, v_codes);
+    c.ks = k_scales;
+    c.kb = k_biases;
+    c.vs = v_scales;
+    c.vb = v_biases;
+    c.bits = bits;
+    c.gs = group_size;
+    if (run_mfma(c, workspace, workspace_bytes, st, &rc)) return rc;
+  }
   if (bits == 4) {
     emx::AffineKV<4> kv{k_codes,
                         reinterpret_cast<const emx::h16*>(k_scales),
@@ -1288,9 +1314,7 @@ int emx_paged_attention_dense(const void* queries, int num_tokens, int num_q_hea
   ga.decode = single_token_decode ? 1 : 0;
   if (dtype == EMX_DTYPE_F16 || dtype == EMX_DTYPE_BF16) {
     const emx::KvKind kind = dtype == EMX_DTYPE_F16 ? emx::KvKind::f16 : emx::KvKind::bf16;
-    if (run_token_major(token_major_call(kind, ga, key_cache, value_cache, nullptr, nullptr), workspace,
-                        workspace_bytes, st, &rc))
-      return rc;
+    if (run_mfma(mfma_call(kind, ga, key_cache, value_cache), workspace, workspace_bytes, st, &rc)) return rc;
   }
   switch (dtype) {
     case EMX_DTYPE_F16: {
@@ -1638,10 +1662,12 @@ int emx_paged_attention_fp8(const void* queries, int num_tokens, int num_q_heads
   // other GQA ratios: the MFMA prefill kernel over every row (a decode row is a
   // tile of one query token)
   if (pf && query_start_loc) return launch_prefill(1);
-  if (dtype == EMX_DTYPE_F16 && run_token_major(token_major_call(emx::KvKind::fp8, ga, key_cache, value_cache, k_scale,
-                                                                 v_scale),
-                                                workspace, workspace_bytes, st, &rc))
-    return rc;
+  if (dtype == EMX_DTYPE_F16) {
+    emx::MfmaCall c = mfma_call(emx::KvKind::fp8, ga, key_cache, value_cache);
+    c.kps = k_scale;
+    c.vps = v_scale;
+    if (run_mfma(c, workspace, workspace_bytes, st, &rc)) return rc;
+  }
   const emx::Fp8KV kv{key_cache, value_cache, k_scale, v_scale, num_kv_heads, head_dim, page_size};
   switch (dtype) {
     case EMX_DTYPE_F16: return launch_generic<emx::h16>(ga, kv, st, workspace, workspace_bytes);

@@ -23,12 +23,32 @@ template <class C>
 DecodeMfmaFn pick_decode(int D) {
   return D == 64 ? decode_mfma<C, 64> : D == 128 ? decode_mfma<C, 128> : decode_mfma<C, 256>;
 }
+template <int BITS>
+DecodeMfmaFn pick_decode_affine(int D, int gs) {
+  if (gs == 64) return pick_decode<KvAffine<BITS, 64>>(D);
+  return D == 128 ? decode_mfma<KvAffine<BITS, 128>, 128> : decode_mfma<KvAffine<BITS, 128>, 256>;
+}
+DecodeMfmaFn decode_fn(const MfmaCall& c) {
+  switch (c.kind) {
+    case KvKind::f16: return pick_decode<KvF16>(c.D);
+    case KvKind::bf16: return pick_decode<KvBF16>(c.D);
+    case KvKind::fp8: return pick_decode<KvFp8>(c.D);
+    case KvKind::affine: break;
+  }
+  return c.bits == 4 ? pick_decode_affine<4>(c.D, c.gs) : pick_decode_affine<8>(c.D, c.gs);
+}
 
 }  // namespace
 
-bool token_major_ok(const TokenMajorCall& c) {
+bool mfma_ok(const MfmaCall& c) {
   // page_of() is exact for power-of-two pages, and for the others while position * bs < 2^32
   const bool pages = c.bs % 8 == 0 && ((c.bs & (c.bs - 1)) == 0 || (long long)c.max_blocks * c.bs * c.bs < (1LL << 32));
+  if (c.kind == KvKind::affine) {
+    const int tile = 256 / c.bits;
+    if ((c.gs != 64 && c.gs != 128) || c.D % c.gs || c.bs % (tile / 4) || (c.bs % tile && (c.bs & (c.bs - 1))) ||
+        !aligned16(c.ks) || !aligned16(c.kb) || !aligned16(c.vs) || !aligned16(c.vb))
+      return false;
+  }
   return head_ok(c.D) && pages && (long long)c.max_blocks * c.bs < (1LL << 31) && c.S <= kMaxSeqs &&
          (long)c.S * c.Hkv * head_chunks(c.Hq, c.Hkv) <= kMaxUnits && aligned16(c.q) && aligned16(c.out) &&
          aligned16(c.k) && aligned16(c.v);
@@ -40,7 +60,7 @@ size_t decode_mfma_partial_bytes(int S, int Hq, int Hkv, int D) {
   return slots * head_chunk(Hq, Hkv) * (D + 2) * sizeof(float);
 }
 
-static DecodeMfmaArgs decode_args(const TokenMajorCall& c, int* ws_cnt, float* partials) {
+static DecodeMfmaArgs decode_args(const MfmaCall& c, int* ws_cnt, float* partials) {
   DecodeMfmaArgs A{};
   DecodeArgs& a = A.d;
   a.q = static_cast<const h16*>(c.q);
@@ -60,7 +80,11 @@ static DecodeMfmaArgs decode_args(const TokenMajorCall& c, int* ws_cnt, float* p
   a.max_blocks = c.max_blocks;
   a.scale_log2 = c.scale_log2;
   a.window = c.window;
-  a.nt = kDecodeMfmaNT;
+  a.ks = static_cast<const h16*>(c.ks);
+  a.kb = static_cast<const h16*>(c.kb);
+  a.vs = static_cast<const h16*>(c.vs);
+  a.vb = static_cast<const h16*>(c.vb);
+  a.nt = c.kind == KvKind::affine ? 4 * (256 / c.bits) : 128;  // DecodeMfmaCfg::NT
   A.hc = head_chunk(c.Hq, c.Hkv);
   A.nhc = head_chunks(c.Hq, c.Hkv);
   A.inv_bs = (uint32_t)(((1ULL << 32) + c.bs - 1) / c.bs);
@@ -70,11 +94,8 @@ static DecodeMfmaArgs decode_args(const TokenMajorCall& c, int* ws_cnt, float* p
   return A;
 }
 
-void launch_decode_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, hipStream_t st) {
-  const DecodeMfmaFn fn = c.kind == KvKind::f16    ? pick_decode<KvF16>(c.D)
-                          : c.kind == KvKind::bf16 ? pick_decode<KvBF16>(c.D)
-                                                   : pick_decode<KvFp8>(c.D);
-  hipLaunchKernelGGL(fn, dim3(kDecodeMfmaWGs), dim3(256), 0, st, decode_args(c, ws_cnt, partials));
+void launch_decode_mfma(const MfmaCall& c, int* ws_cnt, float* partials, hipStream_t st) {
+  hipLaunchKernelGGL(decode_fn(c), dim3(kDecodeMfmaWGs), dim3(256), 0, st, decode_args(c, ws_cnt, partials));
 }
 
 namespace {
@@ -95,8 +116,8 @@ MixedFn pick_mixed(int D) {
 
 }  // namespace
 
-bool mixed_mfma_ok(const TokenMajorCall& c) {
-  return token_major_ok(c) && c.qsl && c.Hq / c.Hkv <= 64 * ct_of(c.D) && (long long)c.nb * c.bs < (1LL << 31);
+bool mixed_mfma_ok(const MfmaCall& c) {
+  return mfma_ok(c) && c.qsl && c.Hq / c.Hkv <= 64 * ct_of(c.D) && (long long)c.nb * c.bs < (1LL << 31);
 }
 
 size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_counters) {
@@ -107,7 +128,7 @@ size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_count
   return (size_t)items * Hkv * kPrefillParts * (4 * (ct_of(D) * (D / 16) + 1) * 1024);
 }
 
-void launch_mixed_mfma(const TokenMajorCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
+void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
                        hipStream_t st) {
   const MixedFn fn = c.kind == KvKind::f16    ? pick_mixed<KvF16>(c.D)
                      : c.kind == KvKind::bf16 ? pick_mixed<KvBF16>(c.D)

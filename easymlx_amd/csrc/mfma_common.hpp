@@ -1,10 +1,11 @@
-// Shared pieces of the MFMA attention kernels over token-major caches
-// [nb, bs, Hkv, D] (unquantized fp16 / bf16, FP8 E4M3): operand types, the
-// probability split, and the exact fallback for non-finite rows.
+// Shared pieces of the MFMA attention kernels over any cache (decode_mfma.hpp,
+// prefill_mfma.hpp): operand types, the probability split, and the exact fallback for
+// non-finite rows.
 #pragma once
 
 #include "common.hpp"
 #include "decode_affine.hpp"
+#include "paged_generic.hpp"
 
 namespace emx {
 
@@ -17,22 +18,47 @@ struct KvF16 {
   typedef h16x8 Op;     // one lane's MFMA operand
   typedef h16 ET;       // cache element
   static constexpr int kParts = 2;  // 16-bit parts of a probability
-  static constexpr bool kFp8 = false;
+  static constexpr bool kFp8 = false, kAffine = false;
 };
 struct KvBF16 {
   typedef uint16_t QT;
   typedef bf16x8 Op;
   typedef uint16_t ET;
   static constexpr int kParts = 3;
-  static constexpr bool kFp8 = false;
+  static constexpr bool kFp8 = false, kAffine = false;
 };
 struct KvFp8 {
   typedef h16 QT;
   typedef h16x8 Op;
   typedef uint8_t ET;
   static constexpr int kParts = 2;
-  static constexpr bool kFp8 = true;
+  static constexpr bool kFp8 = true, kAffine = false;
 };
+// Affine pages: codes enter the MFMA as exact fp16 sub-normals (code * 2^-24).
+template <int BITS, int GS>
+struct KvAffine {
+  typedef h16 QT;
+  typedef h16x8 Op;
+  typedef uint8_t ET;
+  static constexpr int kParts = 2;
+  static constexpr bool kFp8 = false, kAffine = true;
+  static constexpr int kBits = BITS, kGS = GS;
+};
+
+// The element loader of a call's cache (paged_generic.hpp).
+template <class C>
+__device__ __forceinline__ auto kv_loader(const DecodeArgs& a, const int D) {
+  if constexpr (C::kAffine)
+    return AffineKV<C::kBits>{a.kc, a.ks, a.kb, a.vc, a.vs, a.vb, a.Hkv, D, a.bs, C::kGS};
+  else if constexpr (C::kFp8)
+    return Fp8KV{reinterpret_cast<const uint8_t*>(a.kc), reinterpret_cast<const uint8_t*>(a.vc), a.kps, a.vps, a.Hkv,
+                 D, a.bs};
+  else if constexpr (__is_same(typename C::QT, h16))
+    return DenseKV<F16>{reinterpret_cast<const h16*>(a.kc), reinterpret_cast<const h16*>(a.vc), a.Hkv, D, a.bs};
+  else
+    return DenseKV<BF16>{reinterpret_cast<const uint16_t*>(a.kc), reinterpret_cast<const uint16_t*>(a.vc), a.Hkv, D,
+                         a.bs};
+}
 
 __device__ __forceinline__ f32x4 mfma_op(const h16x8 a, const h16x8 b, const f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -82,14 +108,6 @@ __device__ __forceinline__ void split_p(const float (&x)[8], bf16x8 (&p)[3]) {
 // exact while p * bs < 2^32, which the host checks for the whole table.
 __device__ __forceinline__ int page_of(const int p, const uint32_t inv) { return (int)__umulhi((uint32_t)p, inv); }
 
-template <class C>
-__device__ __forceinline__ float kv_elem(const void* base, const size_t i) {
-  if constexpr (C::kFp8)
-    return e4m3_to_f32(static_cast<const uint8_t*>(base)[i]);
-  else
-    return to_f32(static_cast<const typename C::ET*>(base)[i]);
-}
-
 // One query row against keys [k0, k1) in fp32 on one wave, a key at a time: the
 // rows whose MFMA result is not finite are computed again here.  On the matrix
 // unit a masked key still enters its tile's product with p = 0, and 0 * inf (an
@@ -100,6 +118,7 @@ template <class C, int D>
 __device__ void attend_row(const DecodeArgs& a, const int s, const int kvh, const typename C::QT* q, const int k0,
                            const int k1, float& l, float (&acc)[(D + 63) / 64], const int lane) {
   constexpr int N = (D + 63) / 64;
+  const auto kv = kv_loader<C>(a, D);
   float qv[N], m = -INFINITY;
   l = 0.f;
 #pragma unroll
@@ -111,17 +130,10 @@ __device__ void attend_row(const DecodeArgs& a, const int s, const int kvh, cons
   for (int k = k0; k < k1; ++k) {
     const int blk = a.block_tables[(size_t)s * a.max_blocks + k / a.bs];
     if ((unsigned)blk >= (unsigned)a.nb) continue;
-    const size_t row = (((size_t)blk * a.bs + k % a.bs) * a.Hkv + kvh) * D;
     float x = 0.f;
 #pragma unroll
-    for (int i = 0; i < N; ++i) x += qv[i] * kv_elem<C>(a.kc, row + lane + 64 * i);
-    x = wave_sum(x);
-    float vs = 1.f;
-    if constexpr (C::kFp8) {
-      x *= a.kps[blk];
-      vs = a.vps[blk];
-    }
-    x *= a.scale_log2;
+    for (int i = 0; i < N; ++i) x += qv[i] * kv.key(blk, k % a.bs, kvh, lane + 64 * i);
+    x = wave_sum(x) * a.scale_log2;
     const float mn = fmaxf(m, x);
     float p = 0.f, al = 1.f;
     if (mn != -INFINITY || x != x) {
@@ -131,7 +143,7 @@ __device__ void attend_row(const DecodeArgs& a, const int s, const int kvh, cons
     l = l * al + p;
     m = mn;
 #pragma unroll
-    for (int i = 0; i < N; ++i) acc[i] = acc[i] * al + p * (kv_elem<C>(a.vc, row + lane + 64 * i) * vs);
+    for (int i = 0; i < N; ++i) acc[i] = acc[i] * al + p * kv.val(blk, k % a.bs, kvh, lane + 64 * i);
   }
 }
 

@@ -1,4 +1,4 @@
-"""MFMA attention over token-major caches (unquantized fp16 / bf16, FP8) vs the float64 oracle.
+"""MFMA attention over every cache type (unquantized fp16 / bf16, FP8, affine pages) vs the float64 oracle.
 
 Bound of a result: half a unit in the last place of the 16-bit output (2^-11 / 2^-8 of the value, bf16
 rounding 8 bits) plus the fp32 arithmetic: scores are fp32 sums of up to 256 products, |s| <= ~16, so a
@@ -10,15 +10,16 @@ import pytest
 import torch
 
 from easymlx_amd import paged_attention
+from easymlx_amd.caching import layout
 from oracle import fp8
 from oracle.paged_attention import paged_attention as oracle_attention
 
 pytestmark = pytest.mark.gpu
 
-DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "fp8": torch.float16}
+DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "fp8": torch.float16, "q4": torch.float16, "q8": torch.float16}
 
 
-def batch(kind, qlens, kvl, hq, hkv, d, page, seed, invalid=()):
+def batch(kind, qlens, kvl, hq, hkv, d, page, seed, invalid=(), gs=64):
     """Seeded inputs on the CPU: queries, stored caches (and scales), tables, and the exact cache values."""
     rng = np.random.default_rng(seed)
     pages = [-(-max(x, 1) // page) for x in kvl]
@@ -39,6 +40,18 @@ def batch(kind, qlens, kvl, hq, hkv, d, page, seed, invalid=()):
         cache = [torch.from_numpy(c) for c in codes]
         exact = [fp8.e4m3_decode(c).astype(np.float64) * s[:, None, None, None].astype(np.float64)
                  for c, s in zip(codes, scales)]
+    elif kind in ("q4", "q8"):
+        bits = int(kind[1])
+        cache, exact, scales = [], [], {"bits": bits, "group_size": gs}
+        for name, pack in (("k", layout.key_pages_from_logical), ("v", lambda w: layout.value_pages_from_logical(w, bits))):
+            codes = rng.integers(0, 1 << bits, size=shape)
+            sc = (rng.uniform(0.5, 2.0, size=shape[:3] + (d // gs,)) * rng.choice([-1, 1], size=shape[:3] + (d // gs,))
+                  * 6.0 / (1 << bits)).astype(np.float16)
+            bi = (-sc.astype(np.float32) * (1 << (bits - 1)) + rng.standard_normal(sc.shape) * 0.3).astype(np.float16)
+            exact.append(codes * np.repeat(sc.astype(np.float64), gs, -1) + np.repeat(bi.astype(np.float64), gs, -1))
+            cache.append(torch.from_numpy(pack(layout._pack(codes, bits)).view(np.int32)))
+            scales[name + "_scales"] = torch.from_numpy(layout.params_pages_from_logical(sc))
+            scales[name + "_biases"] = torch.from_numpy(layout.params_pages_from_logical(bi))
     else:
         cache = [torch.from_numpy(rng.standard_normal(shape, dtype=np.float32) * 1.5).to(DTYPES[kind])
                  for _ in range(2)]
@@ -49,7 +62,11 @@ def batch(kind, qlens, kvl, hq, hkv, d, page, seed, invalid=()):
 
 def run(b, dev, window=0, decode=True):
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
-    kw = dict(k_scale=t(b["scales"][0]), v_scale=t(b["scales"][1])) if b["scales"] is not None else {}
+    sc = b["scales"]
+    if isinstance(sc, dict):
+        kw = {k: x.to(dev) if isinstance(x, torch.Tensor) else x for k, x in sc.items()}
+    else:
+        kw = dict(k_scale=t(sc[0]), v_scale=t(sc[1])) if sc is not None else {}
     out = paged_attention(b["q"].to(dev), b["cache"][0].to(dev), b["cache"][1].to(dev), t(b["tables"]), t(b["kvl"]),
                           t(b["qsl"]), sliding_window=window or None, single_token_decode=decode, **kw)
     torch.cuda.synchronize()
@@ -84,6 +101,20 @@ def test_decode(cuda, kind, d, page, hq, hkv):
         check(b, run(b, cuda, window), expected(b, window))
 
 
+# shapes the 128-wide affine decode kernels do not take: other head sizes, GQA ratios that are not
+# powers of two (or above 16), pages between theirs
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("d,page,hq,hkv,gs", [(64, 16, 8, 2, 64), (64, 128, 4, 4, 64), (128, 16, 6, 2, 64),
+                                              (128, 32, 40, 2, 128), (128, 192, 7, 1, 64), (256, 64, 4, 4, 64),
+                                              (256, 16, 16, 1, 128), (256, 128, 9, 3, 64)])
+def test_decode_affine(cuda, kind, d, page, hq, hkv, gs):
+    print(f"[affine decode {kind} d{d} page{page} {hq}/{hkv} g{gs}]", flush=True)
+    b = batch(kind, [1] * len(CONTEXTS), CONTEXTS, hq, hkv, d, page, seed=d + page + hq, gs=gs,
+              invalid=[(5, 1), (9, 0), (10, 2)] if page < 64 else [])
+    for window in (0, 1, 100):
+        check(b, run(b, cuda, window), expected(b, window))
+
+
 @pytest.mark.parametrize("kind", ["f16", "fp8"])
 def test_decode_one_long_row(cuda, kind):
     """One sequence cut over every workgroup: a merge of many pieces, twice on the same workspace."""
@@ -93,6 +124,32 @@ def test_decode_one_long_row(cuda, kind):
     first = run(b, cuda)
     check(b, first, exp)
     assert np.array_equal(first, run(b, cuda))
+
+
+def test_decode_affine_stale_scales(cuda):
+    """Scales of tokens past kv_len may hold anything; an infinite scale of a live token gives infinities."""
+    print("[affine decode stale scales]", flush=True)
+    b = batch("q8", [1, 1], [70, 41], 6, 2, 128, 16, seed=4)
+    exp = expected(b)
+    at = lambda s, p: (int(b["tables"][s, p // 16]), p % 16)  # noqa: E731
+    blk, off = at(0, 75)
+    for n in ("k_scales", "k_biases", "v_scales", "v_biases"):
+        b["scales"][n][blk, :, :, off] = float("nan")
+    blk, off = at(1, 40)
+    b["scales"]["v_biases"][blk, 1, 0, off] = float("inf")  # kv head 1, dims 0 .. 63
+    got = run(b, cuda)
+    assert np.isposinf(got[1, 3:, :64]).all()
+    got[1, 3:, :64] = exp[1, 3:, :64]
+    check(b, got, exp)
+
+
+def test_decode_short_contexts_whole_units(cuda):
+    """More units than workgroups, contexts too short to cut: ranges start at unit starts."""
+    print("[decode whole units]", flush=True)
+    kvl = [int(x) for x in np.random.default_rng(1).integers(1, 400, size=150)]
+    for kind in ("bf16", "q4"):
+        b = batch(kind, [1] * 150, kvl, 6, 6, 64, 16, seed=12)
+        check(b, run(b, cuda), expected(b))
 
 
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
