@@ -31,8 +31,9 @@
 //
 // Bound by HBM.  Against decode_split and its merge (VALU dot products, single-element
 // loads, two launches), which ran these shapes before: batch 32, contexts of 512 to
-// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 75.7 us, FP8 (136 MB)
-// 330 -> 51 us; one context of 1024, D 64, fp16: 38.4 -> 14.1 us.
+// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 71.3 us, FP8 (136 MB)
+// 330 -> 44 us; one context of 1024, D 64, fp16: 38.4 -> 14.2 us; 8-bit pages, D 256, 13
+// contexts of 200 to 5000 (64 MB): 141 -> 40 us.
 #pragma once
 
 #include "mfma_common.hpp"
@@ -142,6 +143,50 @@ __device__ __forceinline__ bool write4(const f32x4 O, const float L, QT* out) {
   return bad;
 }
 
+// Per-sequence tables in LDS: cum[s] = items (of NT tokens, per unit) of the decoded
+// sequences before s, kvl[s] = clamped kv_len (-1: not a single-token row), qrw[s] = query row.
+// (seq_table of decode_affine.hpp with a constant item size: its two divisions by a run-time
+// one and the serial 64-bit range arithmetic were a third of a short call.)
+template <int NT>
+__device__ __forceinline__ void decode_mfma_table(const DecodeArgs& a, int* cum, int* kvl, int* qrw, int* wsum) {
+  const int ch = (a.S + 255) / 256, s0 = threadIdx.x * ch;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int tsum = 0;
+  for (int i = 0; i < ch; ++i) {
+    const int s = s0 + i;
+    if (s >= a.S) break;
+    const int kl = max(min(a.kv_lens[s], a.max_blocks * a.bs), 0);
+    const int q0 = a.qsl ? a.qsl[s] : s, q1 = a.qsl ? a.qsl[s + 1] : s + 1;
+    const bool dec = q1 - q0 == 1;
+    const int st = a.window > 0 ? max(0, kl - a.window) : 0;
+    const int n = dec && kl > 0 ? (kl - 1) / NT - st / NT + 1 : 0;
+    kvl[s] = dec ? kl : -1;
+    qrw[s] = q0;
+    cum[s] = n;  // the count for now
+    tsum += n;
+  }
+  int x = tsum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) wsum[wv] = x;
+  __syncthreads();
+  int run = x - tsum;
+#pragma unroll
+  for (int w = 0; w < 3; ++w) run += w < wv ? wsum[w] : 0;
+  for (int i = 0; i < ch; ++i) {
+    const int s = s0 + i;
+    if (s >= a.S) break;
+    const int n = cum[s];
+    cum[s] = run;
+    run += n;
+  }
+  if (threadIdx.x == 255) cum[a.S] = run;
+  __syncthreads();
+}
+
 template <class C, int D>
 __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const int bid, const int nblocks) {
   using P = DecodeMfmaCfg<C, D>;
@@ -168,7 +213,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   float* xml = &lds_at<float>(oXml);    // [wave][head][2]
   int& flag = lds_at<int>(oFlag);
   h16* stage = &lds_at<h16>(oStage) + wv * P::STAGE;  // affine: this wave's [array][group][token] scales
-  seq_table(a, cum, kvl, qrw);
+  decode_mfma_table<NT>(a, cum, kvl, qrw, reinterpret_cast<int*>(xml));
   const int S = a.S, HG = a.Hq / a.Hkv, Hu = a.Hkv * A.nhc;
   {  // decoded sequences without a live token produce zeros (the reference's l == 0 case)
     const int per_seq = a.Hq * D / 8;
@@ -178,15 +223,22 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
         reinterpret_cast<u32x4*>(a.out)[(size_t)qrw[si] * per_seq + i % per_seq] = u32x4{0u, 0u, 0u, 0u};
     }
   }
-  const long long I = (long long)Hu * uru(cum[S]);
-  const int NW = (int)min((long long)nblocks, I);
+  // (the host keeps the number of items below 2^31)
+  const int I = Hu * uru(cum[S]);
+  const int NW = min(nblocks, I);
   if (bid >= NW) return;
+  const int per = (unsigned)I / (unsigned)NW, extra = I - per * NW;  // the first `extra` ranges hold one item more
+  auto first_of = [&](int w) { return w * per + min(w, extra); };
+  auto wg_of = [&](int g) {  // the workgroup whose range holds item g
+    const int big = extra * (per + 1);
+    return g < big ? (int)((unsigned)g / (unsigned)(per + 1)) : extra + (int)((unsigned)(g - big) / (unsigned)per);
+  };
   // The sequence of item g; the most items a unit has.
-  auto seq_of = [&](const long long g) {
+  auto seq_of = [&](const int g) {
     int s = 0;
     for (int c = 0; c < S; c += 64) {
       const int si = c + lane;
-      s += __builtin_popcountll(__ballot(si < S && (long long)Hu * cum[si + 1] <= g));
+      s += __builtin_popcountll(__ballot(si < S && Hu * cum[si + 1] <= g));
     }
     return uru(s);
   };
@@ -196,15 +248,14 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     nmax = max(nmax, si < S ? cum[si + 1] - cum[si] : 0);
   }
   nmax = uru((int)wave_max((float)nmax));
-  const bool cut = (long long)(nmax - kDecodeMfmaMergeItems) * NW > I;
-  long long g0 = (long long)bid * I / NW, g1 = (long long)(bid + 1) * I / NW;
+  const bool cut = nmax > per + kDecodeMfmaMergeItems;
+  int g0 = first_of(bid), g1 = first_of(bid + 1);
   if (!cut) {  // whole units: those whose first item lies in the range
-    auto unit_ceil = [&](const long long g) {
+    auto unit_ceil = [&](const int g) {
       if (g >= I) return I;
       const int s = seq_of(g);
-      const long long b = (long long)Hu * uru(cum[s]);
-      const int n = uru(cum[s + 1]) - uru(cum[s]);
-      return b + (long long)uru(((int)(g - b) + n - 1) / n) * n;
+      const int b = Hu * uru(cum[s]), n = uru(cum[s + 1]) - uru(cum[s]);
+      return b + uru((int)((unsigned)(g - b + n - 1) / (unsigned)n)) * n;
     };
     g0 = unit_ceil(g0);
     g1 = unit_ceil(g1);
@@ -222,16 +273,16 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   {
     it0.s = seq_of(g0);
     it0.n = uru(cum[it0.s + 1]) - uru(cum[it0.s]);
-    const int r = (int)(g0 - (long long)Hu * uru(cum[it0.s]));
-    it0.y = uru(r / it0.n);
-    it0.j = uru(r % it0.n);
+    const int r = g0 - Hu * uru(cum[it0.s]);
+    it0.y = uru((int)((unsigned)r / (unsigned)it0.n));
+    it0.j = r - it0.y * it0.n;
     it0.kl = uru(kvl[it0.s]);
     it0.st = start_of(it0.kl);
     it0.tb = tb_of(it0.st, it0.j);
     it0.has = true;
   }
   // the item after x, g being x's index; past the range x again with has = false
-  auto after = [&](const Item& x, const long long g) {
+  auto after = [&](const Item& x, const int g) {
     Item r = x;
     r.has = g + 1 < g1;
     if (!r.has) return r;
@@ -457,12 +508,17 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   Look lc, ln, l2;
   lookup(lc, cur);
   load_q(cur.s, cur.y);
+  // (kept in this order: one path with another order would make every wait the longest one)
+  __builtin_amdgcn_sched_barrier(0);
   issue_k(lc, cur);
+  __builtin_amdgcn_sched_barrier(0);
   lookup(ln, nxt);
+  __builtin_amdgcn_sched_barrier(0);
   issue_v(lc, cur);
-  long long seg0 = g0;  // first item of the unit that this workgroup holds
+  __builtin_amdgcn_sched_barrier(0);
+  int seg0 = g0;  // first item of the unit that this workgroup holds
 
-  for (long long g = g0; g < g1; ++g) {
+  for (int g = g0; g < g1; ++g) {
     const int s = cur.s, y = cur.y, n_s = cur.n, tb = cur.tb, kv_len = cur.kl, start_k = cur.st;
     const Item n2 = nxt.has ? after(nxt, g + 1) : nxt;
     // ---- scores: lane (h, jj), element 4 t + r
@@ -514,7 +570,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
 #pragma unroll
         for (int w = 0; w < P::KS; ++w) {
           const uint32_t* k = &ld.k[t][w * C::kBits / 4];
-          c[32 * w / C::kGS] = mfma_op(C::kBits == 4 ? unpack4(k[0]) : unpack8(k[0], k[1]), qB[w], c[32 * w / C::kGS]);
+          c[32 * w / C::kGS] = mfma_op(C::kBits == 4 ? unpack4_high(k[0]) : unpack8(k[0], k[1]), qB[w], c[32 * w / C::kGS]);
         }
         typedef h16 h16x4v __attribute__((ext_vector_type(4)));
         float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -524,7 +580,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
           const h16x4v kb4 = *reinterpret_cast<const h16x4v*>(stage + (P::G + g) * P::NTW + NV * jj + 4 * t);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            v[r] = fmaf(c[g][r] * kTwo24, (float)ks4[r], fmaf((float)kb4[r], qsum[g], v[r]));
+            v[r] = fmaf(c[g][r] * (float)(1 << C::kCodeExp), (float)ks4[r], fmaf((float)kb4[r], qsum[g], v[r]));
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) sc[4 * t + r] = v[r];
@@ -546,8 +602,11 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
         for (int r = 0; r < 4; ++r) sc[4 * t + r] = C::kFp8 ? c[r] * (ks[t] * 256.f) : c[r];
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
     issue_k(ln, nxt);
+    __builtin_amdgcn_sched_barrier(0);
     lookup(l2, n2);
+    __builtin_amdgcn_sched_barrier(0);
     const bool unit_end = !nxt.has || nxt.s != s || nxt.y != y;
 
     // ---- mask: outside [start_k, kv_len), or on a page with an invalid id
@@ -596,7 +655,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
           split_p(x, pB);
 #pragma unroll
           for (int b = g * (C::kGS / 16); b < (g + 1) * (C::kGS / 16); ++b) {
-            const Op V = C::kBits == 4 ? unpack4(ld.v[b][w]) : unpack8(ld.v[b][0], ld.v[b][1]);
+            const Op V = C::kBits == 4 ? unpack4_high(ld.v[b][w]) : unpack8(ld.v[b][0], ld.v[b][1]);
 #pragma unroll
             for (int k = 0; k < C::kParts; ++k) acc[b] = mfma_op(V, pB[k], acc[b]);
           }
@@ -634,18 +693,18 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       // ---- the waves' states through LDS (rounds of RD dims), all threads combining
       const int kvh = y / A.nhc, h0 = (y % A.nhc) * A.hc, nh = min(A.hc, HG - h0);
       const int u = s * Hu + y;
-      const long long unit_first = (long long)Hu * uru(cum[s]) + (long long)y * n_s;
+      const int unit_first = Hu * uru(cum[s]) + y * n_s;
       const bool whole = seg0 == unit_first && g + 1 == unit_first + n_s;
       int slot = 0, np = 1;
       if (!whole) {
-        const int wf = wave_of_item(unit_first, I, NW);
-        np = uru(wave_of_item(unit_first + n_s - 1, I, NW) - wf + 1);
+        const int wf = uru(wg_of(unit_first));
+        np = uru(wg_of(unit_first + n_s - 1)) - wf + 1;
         slot = uru(wf + u);  // the unit's pieces sit in slots wf + u ..
       }
       float l = l_part + __shfl_xor(l_part, 16, 64);
       l += __shfl_xor(l, 32, 64);
-      if constexpr (C::kAffine) {  // codes entered as code * 2^-24; the bias term joins its group's dims
-        const float f = __uint_as_float((uint32_t)(127 + vexp + 24) << 23);
+      if constexpr (C::kAffine) {  // codes entered as code * 2^-kCodeExp; the bias term joins its group's dims
+        const float f = __uint_as_float((uint32_t)(127 + vexp + C::kCodeExp) << 23);
 #pragma unroll
         for (int g = 0; g < P::G; ++g) {
           const float bias = rows4_sum(pb[g]);
@@ -801,6 +860,14 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       clear();
       seg0 = g + 1;
       if (nxt.has) load_q(nxt.s, nxt.y);
+      // waited for here: a query load outstanding on this path only would make every item's first
+      // product wait for all loads in flight
+#pragma unroll
+      for (int w = 0; w < P::KS; ++w) {
+        u32x4 x = __builtin_bit_cast(u32x4, qB[w]);
+        asm volatile("" : "+v"(x));
+        qB[w] = __builtin_bit_cast(Op, x);
+      }
     }
     cur = nxt;
     nxt = n2;

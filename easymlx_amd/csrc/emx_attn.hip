@@ -429,7 +429,7 @@ bool run_mfma(const emx::MfmaCall& c, void* ws, size_t ws_bytes, hipStream_t st,
     *rc = check_launch("decode_mfma");
     return true;
   }
-  if (c.kind == emx::KvKind::affine || !emx::mixed_mfma_ok(c)) return false;
+  if (!emx::mixed_mfma_ok(c)) return false;
   const size_t part = emx::mixed_mfma_part_bytes(c.T, c.S, c.Hq, c.Hkv, c.D, emx::kPrefillCounters);
   const size_t base = (need + 255) & ~(size_t)255;
   const bool cut = have && part > 0 && ws_bytes >= base + part;

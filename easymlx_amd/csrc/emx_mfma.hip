@@ -10,7 +10,8 @@
 namespace emx {
 namespace {
 
-constexpr int kDecodeMfmaWGs = 512;  // persistent grid: two workgroups per compute unit
+constexpr int kDecodeMfmaWGs = 512;  // persistent grid: two workgroups per compute unit ..
+int decode_wgs(int D) { return D == 256 ? kDecodeMfmaWGs / 2 : kDecodeMfmaWGs; }  // .. or the one that fits
 
 bool head_ok(int D) { return D == 64 || D == 128 || D == 256; }
 int head_chunk(int Hq, int Hkv) { return std::min(Hq / Hkv, 16); }
@@ -49,8 +50,9 @@ bool mfma_ok(const MfmaCall& c) {
         !aligned16(c.ks) || !aligned16(c.kb) || !aligned16(c.vs) || !aligned16(c.vb))
       return false;
   }
+  const long long units = (long long)c.S * c.Hkv * head_chunks(c.Hq, c.Hkv);
   return head_ok(c.D) && pages && (long long)c.max_blocks * c.bs < (1LL << 31) && c.S <= kMaxSeqs &&
-         (long)c.S * c.Hkv * head_chunks(c.Hq, c.Hkv) <= kMaxUnits && aligned16(c.q) && aligned16(c.out) &&
+         units <= kMaxUnits && units * ((long long)c.max_blocks * c.bs / 128 + 2) < (1LL << 31) && aligned16(c.q) && aligned16(c.out) &&
          aligned16(c.k) && aligned16(c.v);
 }
 
@@ -95,7 +97,7 @@ static DecodeMfmaArgs decode_args(const MfmaCall& c, int* ws_cnt, float* partial
 }
 
 void launch_decode_mfma(const MfmaCall& c, int* ws_cnt, float* partials, hipStream_t st) {
-  hipLaunchKernelGGL(decode_fn(c), dim3(kDecodeMfmaWGs), dim3(256), 0, st, decode_args(c, ws_cnt, partials));
+  hipLaunchKernelGGL(decode_fn(c), dim3(decode_wgs(c.D)), dim3(256), 0, st, decode_args(c, ws_cnt, partials));
 }
 
 namespace {
@@ -113,11 +115,26 @@ MixedFn pick_mixed(int D) {
   return D == 64 ? mixed_mfma<C, 64, ct_of(64)> : D == 128 ? mixed_mfma<C, 128, ct_of(128)>
                                                             : mixed_mfma<C, 256, ct_of(256)>;
 }
+template <int BITS>
+MixedFn pick_mixed_affine(int D, int gs) {
+  if (gs == 64) return pick_mixed<KvAffine<BITS, 64>>(D);
+  return D == 128 ? mixed_mfma<KvAffine<BITS, 128>, 128, ct_of(128)>
+                  : mixed_mfma<KvAffine<BITS, 128>, 256, ct_of(256)>;
+}
+MixedFn mixed_fn(const MfmaCall& c) {
+  switch (c.kind) {
+    case KvKind::f16: return pick_mixed<KvF16>(c.D);
+    case KvKind::bf16: return pick_mixed<KvBF16>(c.D);
+    case KvKind::fp8: return pick_mixed<KvFp8>(c.D);
+    case KvKind::affine: break;
+  }
+  return c.bits == 4 ? pick_mixed_affine<4>(c.D, c.gs) : pick_mixed_affine<8>(c.D, c.gs);
+}
 
 }  // namespace
 
 bool mixed_mfma_ok(const MfmaCall& c) {
-  return mfma_ok(c) && c.qsl && c.Hq / c.Hkv <= 64 * ct_of(c.D) && (long long)c.nb * c.bs < (1LL << 31);
+  return mfma_ok(c) && c.qsl && c.Hq / c.Hkv <= 64 * ct_of(c.D) && (long long)c.nb * c.bs * (c.kind == KvKind::affine ? c.Hkv : 1) < (1LL << 31);
 }
 
 size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_counters) {
@@ -130,9 +147,6 @@ size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_count
 
 void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
                        hipStream_t st) {
-  const MixedFn fn = c.kind == KvKind::f16    ? pick_mixed<KvF16>(c.D)
-                     : c.kind == KvKind::bf16 ? pick_mixed<KvBF16>(c.D)
-                                              : pick_mixed<KvFp8>(c.D);
   const DecodeMfmaArgs d = decode_args(c, ws_cnt, partials);
   PrefillMfmaArgs p{};
   p.d = d.d;
@@ -146,9 +160,10 @@ void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_
   p.ws_part = part;
   // Decode workgroups by the decode rows' share of the step (at most S of the T rows):
   // bytes per key of a decode row against matrix work per key of a query row.
-  const double share = 100.0 * (c.kind == KvKind::fp8 ? 0.5 : 1.0) * c.S / std::max(1, c.T - c.S) * c.Hkv / c.Hq;
-  const int ndec = ws_cnt ? std::clamp((int)(1024.0 * share), 64, kDecodeMfmaWGs) : 0;
-  hipLaunchKernelGGL(fn, dim3((unsigned)(items * c.Hkv * p.nparts + ndec)), dim3(256), 0, st, p, d, ndec);
+  const double bytes = c.kind == KvKind::affine ? c.bits / 16.0 : c.kind == KvKind::fp8 ? 0.5 : 1.0;
+  const double share = 100.0 * bytes * c.S / std::max(1, c.T - c.S) * c.Hkv / c.Hq;
+  const int ndec = ws_cnt ? std::clamp((int)(1024.0 * share), 64, kDecodeMfmaWGs) & ~7 : 0;
+  hipLaunchKernelGGL(mixed_fn(c), dim3((unsigned)(items * c.Hkv * p.nparts + ndec)), dim3(256), 0, st, p, d, ndec);
 }
 
 }  // namespace emx

@@ -34,7 +34,11 @@ struct KvFp8 {
   static constexpr int kParts = 2;
   static constexpr bool kFp8 = true, kAffine = false;
 };
-// Affine pages: codes enter the MFMA as exact fp16 sub-normals (code * 2^-24).
+// Affine pages: codes enter the MFMA as exact fp16 sub-normals, at 4 bits as code * 2^-18
+// and at 8 bits as code * 2^-24.  The matrix unit aligns a sub-normal's products as if it
+// had the smallest normal exponent, so what the code leaves of the 10 mantissa bits is lost
+// from the sum's precision: 4-bit codes at 2^-24 put scores off by up to 3e-5 where the fp32
+// bias and scale terms leave 3e-6.
 template <int BITS, int GS>
 struct KvAffine {
   typedef h16 QT;
@@ -43,7 +47,13 @@ struct KvAffine {
   static constexpr int kParts = 2;
   static constexpr bool kFp8 = false, kAffine = true;
   static constexpr int kBits = BITS, kGS = GS;
+  static constexpr int kCodeExp = BITS == 4 ? 18 : 24;
 };
+
+// One word of 4-bit codes -> code * 2^-18, in unpack4's element order.
+__device__ __forceinline__ h16x8 unpack4_high(const uint32_t w) {
+  return as_h8((w << 6) & 0x03C003C0u, (w << 2) & 0x03C003C0u, (w >> 2) & 0x03C003C0u, (w >> 6) & 0x03C003C0u);
+}
 
 // The element loader of a call's cache (paged_generic.hpp).
 template <class C>

@@ -1,7 +1,7 @@
-// Ragged / causal paged attention (sequences with more than one query token) over
-// token-major caches [nb, bs, Hkv, D]: unquantized fp16 / bf16 and FP8 (E4M3, one
-// fp32 scale per page), head_dim 64, 128 or 256, pages of a multiple of 8 tokens, any
-// GQA ratio up to 128.  MFMA.
+// Ragged / causal paged attention (sequences with more than one query token), head_dim
+// 64, 128 or 256, any GQA ratio up to 128, over token-major caches [nb, bs, Hkv, D]
+// (unquantized fp16 / bf16, FP8 E4M3 with one fp32 scale per page; pages of a multiple of
+// 8 tokens) and over affine pages.  MFMA.
 //
 // Replaces the ragged / causal Metal kernel of the reference
 // (lib/python/easymlx/operations/kernels/unified_attention.py:290-465, causal limit
@@ -20,14 +20,22 @@
 //   O^T += V^T P^T : A = V^T by the transposing LDS read (ds_read_b64_tr_b16: 4 tokens of
 //   16 dims per 16 lanes), B = the probabilities of the lane's own keys in two fp16 or
 //   three bf16 parts.
+// Affine pages: K codes go to LDS as exact fp16 sub-normals and accumulate per
+// quantization group, the (key, group) scale applied in fp32 and the bias term on the matrix
+// unit (as in prefill_affine.hpp); value codes stay exact too, dim-major, the value scale
+// entering the probability before it is split and sum p * v_bias kept in fp32 (the 128-wide
+// prefill_affine rounds scale * code + bias to fp16 instead).  Keys sit in LDS in the order
+// in which a lane's scores are then eight consecutive keys, those of its value operand.
 // Tiles of many keys are cut into up to kPrefillParts parts, merged in part order by the
 // wave that arrives last (as in prefill_affine.hpp).
 //
 // Bound by the matrix and vector units together (the probability parts double the PV
 // products of fp16, triple those of bf16).  It took over from paged_generic, one wave per
 // (token, kv head) on the VALU: four 512-token chunks beside 28 decode rows, bf16, D 128,
-// pages of 16: 20.7 ms -> 130 us; a 1531-token prompt, fp16, D 256, window 700: 9.7 ms ->
-// 53 us.
+// pages of 16: 20.8 ms -> 128 us; a 1531-token prompt, fp16, D 256, window 700: 9.6 ms ->
+// 53 us; three 203-token chunks beside 9 rows, 4-bit pages of 16: 5.47 ms -> 55 us.  Over 4-bit
+// pages of 128 tokens prefill_affine (value codes dequantized to fp16 once per workgroup)
+// remains the faster kernel where it applies.
 #pragma once
 
 #include "decode_mfma.hpp"
@@ -59,6 +67,28 @@ struct PrefillMfmaCfg {
   static constexpr int NP = NT / RP;                  // pieces per thread and step, of K and of V
   static constexpr int PARTB = 4 * (CT * SB + 1) * 64 * 16;  // bytes of one part's state
 };
+
+template <int BITS, int GS, int D, int CT>
+struct PrefillMfmaCfg<KvAffine<BITS, GS>, D, CT> {
+  static constexpr int NT = D > 128 ? 32 : 64, KS = D / 32, SB = D / 16, COLS = 64 * CT, G = D / GS;
+  static constexpr int KSTR = D + 8;                    // halves per K row
+  static constexpr int VSTR = NT + 8;                   // halves per V dim: 16 dims' reads on distinct banks
+  static constexpr int RBK = D * BITS / 8;              // bytes of a key's codes
+  static constexpr int PR = RBK / 16;                   // 16-byte pieces of them
+  static constexpr int NPK = NT * PR;                   // K pieces of a step
+  static constexpr int NP = (NPK + 255) / 256;
+  static constexpr int UT = 64 / BITS, U = NT / UT;     // V units: 8 bytes, UT tokens of one dim
+  static constexpr int NPV = D * U / 256;               // V units per thread
+  static constexpr int NPS = 4 * G * NT / 8;            // 16-byte scale pieces of a step
+  static constexpr int PARTB = 4 * (CT * SB + 1) * 64 * 16;
+  static_assert(NPS <= 64 && D * U % 256 == 0, "one scale piece per lane, whole V units per thread");
+};
+
+// Where key k of a step sits in the K rows and scale arrays over affine pages: position
+// 16 t + 4 q + e of its 32-key block for k = 8 q + 4 t + e.
+__device__ __forceinline__ constexpr int affine_pos(int k) {
+  return (k & ~31) | ((k & 4) << 2) | ((k & 24) >> 1) | (k & 3);
+}
 
 // 16-byte piece of the cache -> LDS row position, as 16-bit operand values.
 template <class C>
@@ -98,16 +128,24 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   const int col = lane & 15, jj = lane >> 4;
 
   // LDS, carved from the shared arena
+  constexpr bool AFF = C::kAffine;
+  constexpr int G = [] {
+    if constexpr (C::kAffine) return P::G;
+    return 1;
+  }();
   constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oKe = lds_next(oWred, 16);
-  constexpr int oVe = lds_next(oKe, 2 * NT * P::KSTR), oKsf = lds_next(oVe, 2 * NT * P::VSTR);
-  constexpr int oVsf = lds_next(oKsf, 4 * NT), oEnd = lds_next(oVsf, 4 * NT);
+  constexpr int oVe = lds_next(oKe, 2 * NT * P::KSTR), oKsf = lds_next(oVe, 2 * (AFF ? D : NT) * P::VSTR);
+  constexpr int oVsf = lds_next(oKsf, 4 * G * NT), oVbf = lds_next(oVsf, 4 * G * NT);
+  constexpr int oKbe = lds_next(oVbf, AFF ? 4 * G * NT : 0), oEnd = lds_next(oKbe, AFF ? 16 * NT : 0);
   static_assert(oEnd <= kArenaBytes, "LDS arena too small");
   int(&tcum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oTcum);
   int(&wred)[4] = lds_at<int[4]>(oWred);
   uint16_t* ke = &lds_at<uint16_t>(oKe);  // [key][KSTR]
-  uint16_t* ve = &lds_at<uint16_t>(oVe);  // [key][VSTR]
-  float* ksf = &lds_at<float>(oKsf);      // FP8: key / value scale of each key
-  float* vsf = &lds_at<float>(oVsf);
+  uint16_t* ve = &lds_at<uint16_t>(oVe);  // [key][VSTR]; affine: [dim][VSTR]
+  float* ksf = &lds_at<float>(oKsf);      // key scale of each key; affine: [group][NT], * 2^kCodeExp
+  float* vsf = &lds_at<float>(oVsf);      // value scales / 2^vexp
+  float* vbf = &lds_at<float>(oVbf);      // affine: value biases
+  h16* kbe = &lds_at<h16>(oKbe);          // affine: bias operand rows, key bias of group g at 2 g, 2 g + 1
 
   // ---- work item: tiles per sequence, scanned by the workgroup; the last tile (most keys) first
   {
@@ -188,25 +226,50 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
 
   // ---- query operands (zeros for absent columns)
   Op qB[CT][P::KS];
+  Op qbias[CT];  // affine, lane group 0: the query's sum over each group as fp16 hi + lo at 2 g, 2 g + 1
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const bool ok = ctok[ct] >= 0;
     const QT* qp = reinterpret_cast<const QT*>(a.q) +
                    ((size_t)(q0 + (ok ? ctok[ct] : 0)) * a.Hq + (size_t)kvh * HG + (ok ? chead[ct] : 0)) * D + 8 * jj;
+    float gsum[G] = {};
 #pragma unroll
     for (int w = 0; w < P::KS; ++w) {
       const u32x4 x = *reinterpret_cast<const u32x4*>(qp + 32 * w);
-      qB[ct][w] = __builtin_bit_cast(Op, ok ? x : u32x4{0u, 0u, 0u, 0u});
+      const Op v = __builtin_bit_cast(Op, ok ? x : u32x4{0u, 0u, 0u, 0u});
+      if constexpr (AFF) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          qB[ct][w][i] = v[slot_perm<C::kBits>(i)];  // the unpacked codes' order
+          gsum[32 * w / C::kGS] += (float)v[i];
+        }
+      } else {
+        qB[ct][w] = v;
+      }
+    }
+    if constexpr (AFF) {
+      qbias[ct] = Op{};
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float x = rows4_sum(gsum[g]);
+        const h16 hi = (h16)x;
+        if (jj == 0) {
+          qbias[ct][2 * g] = hi;
+          qbias[ct][2 * g + 1] = (h16)(x - (float)hi);
+        }
+      }
     }
   }
 
   // ---- pages: lane l holds the page id of key l of a step (positions past the tile's last key repeat it)
-  const char* kbase = reinterpret_cast<const char*>(a.kc) + (size_t)kvh * (D * P::EB);
-  const char* vbase = reinterpret_cast<const char*>(a.vc) + (size_t)kvh * (D * P::EB);
-  const size_t rowb = (size_t)a.Hkv * D * P::EB;
+  const size_t rowb = (size_t)a.Hkv * D * sizeof(typename C::ET);  // token-major
+  const char* kbase = reinterpret_cast<const char*>(a.kc) + (AFF ? 0 : (size_t)kvh * (D * sizeof(typename C::ET)));
+  const char* vbase = reinterpret_cast<const char*>(a.vc) + (AFF ? 0 : (size_t)kvh * (D * sizeof(typename C::ET)));
   const int32_t* bt = a.block_tables + (size_t)s * a.max_blocks;
   auto page_id = [&](const int st) { return bt[page_of(min(st * NT + (lane & (NT - 1)), k_hi), A.inv_bs)]; };
   u32x4 rk[P::NP], rv[P::NP];  // the next step's pieces
+  u32x2 ru[AFF ? 8 : 1];       // affine: its V units
+  u32x4 rs;                    // affine: scale piece `lane` (every wave loads them: the largest scale is a wave's business)
   uint64_t okn = 0;            // keys of that step on a valid page
   float psk = 0.f, psv = 0.f;  // FP8: page scales of key `lane` of that step
   auto load_step = [&](const int st, const int blk) {
@@ -214,16 +277,47 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     const bool ok = (unsigned)blk < (unsigned)a.nb;
     okn = __ballot(ok);
     const int b = ok ? blk : 0;
-    const int row = b * a.bs + (pos - page_of(pos, A.inv_bs) * a.bs);
-    if constexpr (C::kFp8) {
-      psk = a.kps[b];
-      psv = a.vps[b];
-    }
+    const int off = pos - page_of(pos, A.inv_bs) * a.bs;
+    if constexpr (AFF) {
+      constexpr int B = C::kBits;
+      const int row = (b * a.Hkv + kvh) * a.bs + off;
+      {
+        const int pc = min(lane, P::NPS - 1), seg = pc / (NT / 8), arr = seg / G, g = seg % G;
+        const int r8 = __shfl(row, 8 * (pc % (NT / 8)), 64), o8 = __shfl(off, 8 * (pc % (NT / 8)), 64);
+        const h16 *b_ks = a.ks, *b_kb = a.kb, *b_vs = a.vs, *b_vb = a.vb;
+        asm("" : "+s"(b_ks), "+s"(b_kb), "+s"(b_vs), "+s"(b_vb));  // picked from registers, not by a vector load
+        const h16* base = arr == 0 ? b_ks : arr == 1 ? b_kb : arr == 2 ? b_vs : b_vb;
+        typedef const __attribute__((address_space(1))) u32x4* gu32x4;
+        // (past the tile's last key the group's first token may repeat it: aligned down, inside the page)
+        rs = *(gu32x4)(base + (size_t)G * (r8 - o8) + (size_t)g * a.bs + (o8 & ~7));
+      }
 #pragma unroll
-    for (int n = 0; n < P::NP; ++n) {
-      const size_t off = (size_t)__shfl(row, tid / P::PR + n * P::RP, 64) * rowb + 16 * (tid % P::PR);
-      rk[n] = *reinterpret_cast<const u32x4*>(kbase + off);
-      rv[n] = *reinterpret_cast<const u32x4*>(vbase + off);
+      for (int n = 0; n < P::NP; ++n) {
+        const int e = tid + 256 * n;  // (fewer than 256 pieces: the others repeat them)
+        const int r = __shfl(row, (e / P::PR) & (NT - 1), 64);
+        rk[n] = *reinterpret_cast<const u32x4*>(kbase + (size_t)r * P::RBK + 16 * (e % P::PR));
+      }
+      const int T = min(a.bs, 256 / B);  // tokens of a value tile (a power of two)
+#pragma unroll
+      for (int n = 0; n < P::NPV; ++n) {
+        const int e = tid + 256 * n, u = e % P::U, dim = e / P::U;
+        const int r = __shfl(row, u * P::UT, 64);
+        const int o = (r & (T - 1)) & ~(P::UT - 1);
+        ru[n] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint32_t*>(vbase) +
+                                                (size_t)(r & ~(T - 1)) * (D * B / 32) + (dim * T + o) * B / 32);
+      }
+    } else {
+      const int row = b * a.bs + off;
+      if constexpr (C::kFp8) {
+        psk = a.kps[b];
+        psv = a.vps[b];
+      }
+#pragma unroll
+      for (int n = 0; n < P::NP; ++n) {
+        const size_t o = (size_t)__shfl(row, tid / P::PR + n * P::RP, 64) * rowb + 16 * (tid % P::PR);
+        rk[n] = *reinterpret_cast<const u32x4*>(kbase + o);
+        rv[n] = *reinterpret_cast<const u32x4*>(vbase + o);
+      }
     }
   };
 
@@ -237,7 +331,11 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     for (int b = 0; b < P::SB; ++b) acc[ct][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const float sl2 = a.scale_log2;
-  int vexp = 0;  // FP8: acc holds the sum / 2^vexp
+  int vexp = 0;          // FP8, affine: acc holds the sum / 2^vexp
+  float pb[CT][G] = {};  // affine: sum p * v_bias
+  if constexpr (AFF) {   // the bias operand's unused halves stay zero
+    for (int i = tid; i < NT; i += 256) *reinterpret_cast<u32x4*>(kbe + 8 * i) = u32x4{0u, 0u, 0u, 0u};
+  }
 
   int blk1 = 0;
   if (step_lo <= step_hi) {
@@ -246,13 +344,84 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   }
   for (int st = step_lo; st <= step_hi; ++st) {
     __syncthreads();  // the previous step's tiles are no longer read
+    if constexpr (AFF) {
+      constexpr int B = C::kBits;
 #pragma unroll
-    for (int n = 0; n < P::NP; ++n) {
-      const int r = tid / P::PR + n * P::RP, c = (tid % P::PR) * (16 / P::EB);
-      put_piece<C>(ke + r * P::KSTR + c, rk[n]);
-      put_piece<C>(ve + r * P::VSTR + c, rv[n]);
+      for (int n = 0; n < P::NP; ++n) {
+        const int e = tid + 256 * n;
+        uint16_t* kr = ke + affine_pos((e / P::PR) & (NT - 1)) * P::KSTR + (e % P::PR) * (128 / B);
+        if (e < P::NPK) {
+          if constexpr (B == 4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<h16x8*>(kr + 8 * i) = unpack4_high(rk[n][i]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) *reinterpret_cast<h16x8*>(kr + 8 * i) = unpack8(rk[n][2 * i], rk[n][2 * i + 1]);
+          }
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < P::NPV; ++n) {
+        const int e = tid + 256 * n;
+        uint16_t* vr = ve + (e / P::U) * P::VSTR + (e % P::U) * P::UT;
+        if constexpr (B == 4) {
+          *reinterpret_cast<h16x8*>(vr) = unpack4_high(ru[n][0]);
+          *reinterpret_cast<h16x8*>(vr + 8) = unpack4_high(ru[n][1]);
+        } else {
+          *reinterpret_cast<h16x8*>(vr) = unpack8(ru[n][0], ru[n][1]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int n = 0; n < P::NP; ++n) {
+        const int r = tid / P::PR + n * P::RP, c = (tid % P::PR) * (16 / P::EB);
+        put_piece<C>(ke + r * P::KSTR + c, rk[n]);
+        put_piece<C>(ve + r * P::VSTR + c, rv[n]);
+      }
     }
     const uint64_t okm = okn;
+    if constexpr (AFF) {
+      // scales of keys past the tile's last one or on an invalid page (which may hold anything) as zeros
+      const int pc = min(lane, P::NPS - 1), t8 = 8 * (pc % (NT / 8)), seg = pc / (NT / 8), arr = seg / G, g = seg % G;
+      const int live = k_hi + 1 - st * NT - t8;
+      u32x4 x = rs;
+      if (live < 8 || !((okm >> t8) & 1)) {
+        const int n = (okm >> t8) & 1 ? live : 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] &= (2 * e < n ? 0x0000FFFFu : 0u) | (2 * e + 1 < n ? 0xFFFF0000u : 0u);
+      }
+      int vm = 0;  // largest |v_scale|, as fp16 bits
+      if (arr == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vm = max(vm, (int)max(x[e] & 0x7FFFu, (x[e] >> 16) & 0x7FFFu));
+      }
+      // the accumulator's exponent follows the value scales' (exact powers of two; 6 binades of slack)
+      const int ex = ((int)wave_max((float)vm) >> 10) - 15;
+      if (ex > vexp || ex < vexp - 6) {
+        const float f = __uint_as_float((uint32_t)(127 + vexp - ex) << 23);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int b = 0; b < P::SB; ++b) acc[ct][b] *= f;
+        vexp = ex;
+      }
+      if (wv == 0 && lane < P::NPS) {
+        const float down = __uint_as_float((uint32_t)(127 - vexp) << 23);
+        const float f = arr == 0 ? (float)(1 << C::kCodeExp) : arr == 2 ? down : 1.f;
+        const h16x8 hv = __builtin_bit_cast(h16x8, x);
+        if (arr == 1) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            *reinterpret_cast<h16x2*>(kbe + 8 * affine_pos(t8 + e) + 2 * g) = h16x2{hv[e], hv[e]};
+        } else {
+          float* dst = (arr == 0 ? ksf : arr == 2 ? vsf : vbf) + g * NT;
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            *reinterpret_cast<f32x4*>(dst + affine_pos(t8 + 4 * q)) =
+                f32x4{(float)hv[4 * q] * f, (float)hv[4 * q + 1] * f, (float)hv[4 * q + 2] * f, (float)hv[4 * q + 3] * f};
+        }
+      }
+    }
     float down = 1.f;
     if constexpr (C::kFp8) {
       // value scales enter with the probabilities, brought near 1 by a power of two that the
@@ -287,21 +456,41 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const uint16_t* kr = ke + (32 * h + 16 * t + col) * P::KSTR + 8 * jj;
-        f32x4 c[CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) c[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < P::KS; ++w) {
-          const Op K = *reinterpret_cast<const Op*>(kr + 32 * w);
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct) c[ct] = mfma_op(K, qB[ct][w], c[ct]);
-        }
-        f32x4 ks4 = {1.f, 1.f, 1.f, 1.f};
-        if constexpr (C::kFp8) ks4 = *reinterpret_cast<const f32x4*>(ksf + 32 * h + 16 * t + 4 * jj);
+        f32x4 c[CT][G];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) sc[ct][4 * t + r] = C::kFp8 ? c[ct][r] * ks4[r] : c[ct][r];
+          for (int g = 0; g < G; ++g) c[ct][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < P::KS; ++w) {
+          const Op K = *reinterpret_cast<const Op*>(kr + 32 * w);
+          const int g = w * G / P::KS;
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) c[ct][g] = mfma_op(K, qB[ct][w], c[ct][g]);
+        }
+        if constexpr (AFF) {
+          // (the bias operand is zero outside lane group 0)
+          const Op KB = *reinterpret_cast<const Op*>(kbe + 8 * (32 * h + 16 * t + col));
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            f32x4 v = mfma_op(KB, qbias[ct], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+              const f32x4 ks4 = *reinterpret_cast<const f32x4*>(ksf + g * NT + 32 * h + 16 * t + 4 * jj);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[r] = fmaf(c[ct][g][r], ks4[r], v[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[ct][4 * t + r] = v[r];
+          }
+        } else {
+          f32x4 ks4 = {1.f, 1.f, 1.f, 1.f};
+          if constexpr (C::kFp8) ks4 = *reinterpret_cast<const f32x4*>(ksf + 32 * h + 16 * t + 4 * jj);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[ct][4 * t + r] = C::kFp8 ? c[ct][0][r] * ks4[r] : c[ct][0][r];
+        }
       }
 
       // ---- mask where a key of the half is not visible to every column
@@ -315,7 +504,7 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const int k = 16 * (e >> 2) + 4 * jj + (e & 3);
+            const int k = AFF ? 8 * jj + e : 16 * (e >> 2) + 4 * jj + (e & 3);
             if (kp + k < start[ct] || kp + k > limit[ct] || !((okh >> k) & 1u)) sc[ct][e] = -INFINITY;
           }
       }
@@ -339,6 +528,10 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
           l_part[ct] *= al;
 #pragma unroll
           for (int b = 0; b < P::SB; ++b) acc[ct][b] *= al;
+          if constexpr (AFF) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) pb[ct][g] *= al;
+          }
           if (up) m_run[ct] = m_new[ct];
         }
       }
@@ -361,21 +554,57 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
             for (int r = 0; r < 4; ++r) sc[ct][4 * t + r] *= vs4[r];
           }
         }
-        split_p(sc[ct], pB[ct]);
+        if constexpr (!AFF) split_p(sc[ct], pB[ct]);
       }
 
       // ---- O^T += V^T P^T
 #pragma unroll
-      for (int b = 0; b < P::SB; ++b) {
-        const u32x2 v0 = read_tr(ve, P::VSTR, 32 * h, 16 * b, col, jj);
-        const u32x2 v1 = read_tr(ve, P::VSTR, 32 * h + 16, 16 * b, col, jj);
-        const Op V = __builtin_bit_cast(Op, u32x4{v0[0], v0[1], v1[0], v1[1]});
+      for (int g = 0; g < G; ++g) {
+        if constexpr (AFF) {  // this group's operand: p * v_scale; the bias term in fp32
+          f32x4 vs4[2], vb4[2];
 #pragma unroll
-        for (int k = 0; k < C::kParts; ++k)
+          for (int t = 0; t < 2; ++t) {
+            vs4[t] = *reinterpret_cast<const f32x4*>(vsf + g * NT + 32 * h + 16 * t + 4 * jj);
+            vb4[t] = *reinterpret_cast<const f32x4*>(vbf + g * NT + 32 * h + 16 * t + 4 * jj);
+          }
 #pragma unroll
-          for (int ct = 0; ct < CT; ++ct) acc[ct][b] = mfma_op(V, pB[ct][k], acc[ct][b]);
+          for (int ct = 0; ct < CT; ++ct) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              x[e] = sc[ct][e] * vs4[e >> 2][e & 3];
+              pb[ct][g] = fmaf(sc[ct][e], vb4[e >> 2][e & 3], pb[ct][g]);
+            }
+            split_p(x, pB[ct]);
+          }
+        }
+#pragma unroll
+        for (int b = g * P::SB / G; b < (g + 1) * P::SB / G; ++b) {
+          Op V;
+          if constexpr (AFF) {
+            V = *reinterpret_cast<const Op*>(ve + (16 * b + col) * P::VSTR + 32 * h + 8 * jj);
+          } else {
+            const u32x2 v0 = read_tr(ve, P::VSTR, 32 * h, 16 * b, col, jj);
+            const u32x2 v1 = read_tr(ve, P::VSTR, 32 * h + 16, 16 * b, col, jj);
+            V = __builtin_bit_cast(Op, u32x4{v0[0], v0[1], v1[0], v1[1]});
+          }
+#pragma unroll
+          for (int k = 0; k < C::kParts; ++k)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) acc[ct][b] = mfma_op(V, pB[ct][k], acc[ct][b]);
+        }
       }
     }
+  }
+  if constexpr (AFF) {  // codes entered as code * 2^-kCodeExp; the bias term joins its group's dims
+    const float f = __uint_as_float((uint32_t)(127 + vexp + C::kCodeExp) << 23);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int b = 0; b < P::SB; ++b) {
+        const float bias = rows4_sum(pb[ct][b * G / P::SB]);
+        acc[ct][b] = acc[ct][b] * f + bias;
+      }
   }
   if constexpr (C::kFp8) {  // the codes entered as value * 2^-8
     const float f = __uint_as_float((uint32_t)(127 + vexp + 8) << 23);

@@ -206,7 +206,7 @@ def paged_attention(
         nb, hkv, bs = int(key_cache.shape[0]), int(key_cache.shape[1]), int(key_cache.shape[2])
         need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
         if need and not single_token_decode:  # room for the prefill key split
-            need += int(lib.emx_paged_prefill_workspace_bytes(total, S, hq, hkv, d))
+            need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
         if need and workspace is None:
             workspace = _workspace(dev, stream, need)
         ws_ptr = workspace.data_ptr() if workspace is not None else None

@@ -187,6 +187,29 @@ def test_ragged(cuda, kind, d, page, hq, hkv):
         check(b, run(b, cuda, window, decode=False), expected(b, window))
 
 
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("d,page,hq,hkv,gs", [(64, 16, 8, 2, 64), (64, 128, 4, 4, 64), (128, 16, 6, 2, 64),
+                                              (128, 32, 40, 2, 128), (128, 192, 7, 1, 64), (256, 64, 4, 4, 64),
+                                              (256, 16, 16, 1, 128), (256, 128, 9, 3, 64)])
+def test_ragged_affine(cuda, kind, d, page, hq, hkv, gs):
+    print(f"[affine ragged {kind} d{d} page{page} {hq}/{hkv} g{gs}]", flush=True)
+    b = batch(kind, [q for q, _ in RAGGED], [k for _, k in RAGGED], hq, hkv, d, page, seed=d + page + hq, gs=gs,
+              invalid=[(3, 1), (3, 2), (8, 0), (10, 3)] if page < 64 else [])
+    for window in (0, 50):
+        check(b, run(b, cuda, window, decode=False), expected(b, window))
+
+
+def test_ragged_affine_stale_scales(cuda):
+    """Scales past a sequence's last key may hold anything."""
+    print("[affine ragged stale scales]", flush=True)
+    b = batch("q4", [40, 1], [60, 35], 6, 2, 64, 32, seed=6)
+    exp = expected(b)
+    for s_, p in ((0, 61), (1, 36)):
+        for n in ("k_scales", "k_biases", "v_scales", "v_biases"):
+            b["scales"][n][int(b["tables"][s_, p // 32]), :, :, p % 32] = float("nan")
+    check(b, run(b, cuda, decode=False), exp)
+
+
 def test_ragged_without_workspace(cuda):
     """The C entry point with no workspace: single-token rows go as query tiles, no tile is cut."""
     from easymlx_amd import _native
