@@ -158,10 +158,11 @@ void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_
   p.max_items = part ? (int)items : 0;
   p.ws_cnt = ws_part_cnt;
   p.ws_part = part;
-  // Decode workgroups by the decode rows' share of the step (at most S of the T rows):
-  // bytes per key of a decode row against matrix work per key of a query row.
-  const double bytes = c.kind == KvKind::affine ? c.bits / 16.0 : c.kind == KvKind::fp8 ? 0.5 : 1.0;
-  const double share = 100.0 * bytes * c.S / std::max(1, c.T - c.S) * c.Hkv / c.Hq;
+  // Decode workgroups by the decode rows' share of the step (at most S of the T rows), so that
+  // their streams end with the matrix work.  512-token chunks beside 28 rows: 16 bits 176 / 121 /
+  // 120 / 125 / 128 us at a factor of 10 / 30 / 40 / 70 / 100, FP8 190 / 160 / 139 / 137 at
+  // 12 / 20 / 35 / 50, 8-bit pages (20 rows beside two chunks) 74 / 41 / 38 at 5 / 20 / 35.
+  const double share = 45.0 * c.S / std::max(1, c.T - c.S) * c.Hkv / c.Hq;
   const int ndec = ws_cnt ? std::clamp((int)(1024.0 * share), 64, kDecodeMfmaWGs) & ~7 : 0;
   hipLaunchKernelGGL(mixed_fn(c), dim3((unsigned)(items * c.Hkv * p.nparts + ndec)), dim3(256), 0, st, p, d, ndec);
 }

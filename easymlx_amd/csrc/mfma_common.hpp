@@ -89,7 +89,9 @@ __device__ __forceinline__ void split_p(const float (&x)[8], h16x8 (&p)[2]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const h16x2 h = __builtin_convertvector(f32x2v{x[2 * i], x[2 * i + 1]}, h16x2);
-    const h16x2 l = __builtin_convertvector(f32x2v{x[2 * i] - (float)h[0], x[2 * i + 1] - (float)h[1]}, h16x2);
+    // (as fused multiply-adds: one mixed-precision instruction each)
+    const h16x2 l = __builtin_convertvector(
+        f32x2v{__builtin_fmaf((float)h[0], -1.f, x[2 * i]), __builtin_fmaf((float)h[1], -1.f, x[2 * i + 1])}, h16x2);
     hi[i] = __builtin_bit_cast(uint32_t, h);
     lo[i] = __builtin_bit_cast(uint32_t, l);
   }
