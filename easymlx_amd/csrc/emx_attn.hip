@@ -391,6 +391,25 @@ int launch_generic_only(const emx::GenericArgs& ga, const KV& kv, hipStream_t st
   return check_launch("paged_generic");
 }
 
+// Turns rows [rows, heads, D] of queries or keys (rope_rows, or rope_rows_vec where the rows go
+// in 16-byte pieces: the same bits).
+int launch_rope_rows(emx::h16* x, const emx::h16* src, int rows, int heads, int D, const emx::RopeArgs& r,
+                     hipStream_t st) {
+  if (emx::turn_rows_vec_ok(D, r.rot, r.traditional) && r.rot / 2 <= emx::kRopeVecTab && aligned16(x) &&
+      aligned16(src)) {
+    // tokens per workgroup: two 16-byte pairs of pieces per thread, an angle table that fits
+    const int per = heads * ((r.traditional ? r.rot / 8 : r.rot / 16) + (D - r.rot) / 8);
+    const int tt = std::clamp((512 + per - 1) / per, 1, emx::kRopeVecTab / (r.rot / 2));
+    hipLaunchKernelGGL(emx::rope_rows_vec, dim3((unsigned)((rows + tt - 1) / tt)), dim3(256), 0, st, x, src, rows,
+                       heads, D, r, tt);
+    return check_launch("rope_rows_vec");
+  }
+  const long n = (long)rows * heads * (D / 2);
+  hipLaunchKernelGGL(emx::rope_rows, dim3((unsigned)std::min<long>((n + 255) / 256, 4096)), dim3(256), 0, st, x, src,
+                     rows, heads, D, r);
+  return check_launch("rope_rows");
+}
+
 // What `ga` holds, over the given cache, as a call of the MFMA kernels.
 emx::MfmaCall mfma_call(emx::KvKind kind, const emx::GenericArgs& ga, const void* k, const void* v) {
   emx::MfmaCall c{};
@@ -611,13 +630,8 @@ static int affine_write_impl(const void* keys, const void* values, const int32_t
   else
     hipLaunchKernelGGL(emx::affine_cache_write<8>, grid, dim3(256), 0, st, a);
   if (int rc = check_launch("affine_cache_write")) return rc;
-  if (rope.inv_freq != nullptr && queries != nullptr) {  // larger writes: the queries in their own launch
-    const long n = (long)num_tokens * num_q_heads * (head_dim / 2);
-    const unsigned qgrid = (unsigned)std::min<long>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(emx::rope_rows, dim3(qgrid), dim3(256), 0, st, a.q, a.q_in, num_tokens, num_q_heads, head_dim,
-                       rope);
-    return check_launch("rope_rows");
-  }
+  if (rope.inv_freq != nullptr && queries != nullptr)  // larger writes: the queries in their own launch
+    return launch_rope_rows(a.q, a.q_in, num_tokens, num_q_heads, head_dim, rope, st);
   return EMX_OK;
 }
 
@@ -1029,12 +1043,9 @@ int emx_rope_rows(void* x, int rows, int heads, int head_dim, const int32_t* pos
   if (rows == 0) return EMX_OK;
   if (!x || !rope_ok(positions, inv_freq, rot_dims, head_dim))
     return fail(EMX_ERR_INVALID, "rope: x, positions and inv_freq needed, rot_dims even and in (0, head_dim]");
-  const long n = (long)rows * heads * (rot_dims / 2);
-  const unsigned grid = (unsigned)std::min<long>((n + 255) / 256, 4096);
-  hipLaunchKernelGGL(emx::rope_rows, dim3(grid), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                     reinterpret_cast<emx::h16*>(x), reinterpret_cast<const emx::h16*>(x), rows, heads, head_dim,
-                     emx::RopeArgs{inv_freq, positions, rot_dims, traditional ? 1 : 0});
-  return check_launch("rope_rows");
+  return launch_rope_rows(reinterpret_cast<emx::h16*>(x), reinterpret_cast<const emx::h16*>(x), rows, heads, head_dim,
+                          emx::RopeArgs{inv_freq, positions, rot_dims, traditional ? 1 : 0},
+                          reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t emx_paged_prefill_workspace_bytes(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads,
@@ -1410,12 +1421,8 @@ static int fp8_write_impl(const void* keys, const void* values, int dtype, const
       break;
   }
   if (int rc = check_launch("fp8_cache_write")) return rc;
-  if (turn_q) {  // larger writes: the queries in their own launch
-    const long nq = (long)num_tokens * num_q_heads * (head_dim / 2);
-    hipLaunchKernelGGL(emx::rope_rows, dim3((unsigned)std::min<long>((nq + 255) / 256, 4096)), dim3(256), 0, st,
-                       a.q, a.q_in, num_tokens, num_q_heads, head_dim, rope);
-    return check_launch("rope_rows");
-  }
+  if (turn_q)  // larger writes: the queries in their own launch
+    return launch_rope_rows(a.q, a.q_in, num_tokens, num_q_heads, head_dim, rope, st);
   return EMX_OK;
 }
 

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from easymlx_amd import affine_quantize as gpu_quantize
+from easymlx_amd.caching import affine_pool
 from easymlx_amd.workloads import decode_workload
 from oracle.affine import affine_quantize
 from tests.helpers import gpu_cache, gpu_pages_to_logical, oracle_logical_pages
@@ -123,3 +124,27 @@ def test_cache_write_appends_and_unaligned_chunks(cuda, bits, chunks):
         for i in range(3):
             np.testing.assert_array_equal(after[name][i][~written], before[name][i][~written],
                                           err_msg=f"{name} array {i}: unwritten slots changed")
+
+
+@pytest.mark.parametrize("starts", [(0, 0), (5, 3), (13, 7), (127, 64)], ids=str)
+@pytest.mark.parametrize("page", [16, 128])
+def test_write_chunks_at_any_offset(cuda, starts, page):
+    """Chunks that start inside a value word, and words that straddle two workgroups, bit-exact."""
+    print(f"[write chunks {starts} page {page}]", flush=True)
+    wl = decode_workload(seed=17, num_seqs=2, num_q_heads=4, num_kv_heads=2, block_size=page, ctx_range=(400, 400),
+                         bits=4)
+    view = affine_pool(num_blocks=wl.num_blocks, num_kv_heads=2, head_dim=128, block_size=page, bits=4, group_size=64,
+                       block_tables=torch.from_numpy(wl.block_tables).to(cuda),
+                       kv_lens=torch.from_numpy(wl.kv_lens).to(cuda))
+    idx = np.concatenate([np.arange(400 * i + s, 400 * i + s + 201) for i, s in enumerate(starts)])  # 402 tokens
+    k, v = torch.from_numpy(wl.k[idx]).to(cuda), torch.from_numpy(wl.v[idx]).to(cuda)
+    slot = wl.slot[idx].astype(np.int32)
+    view.write_slots(k, v, torch.from_numpy(slot).to(cuda))
+    torch.cuda.synchronize()
+    got = gpu_pages_to_logical(view)
+    b, o = slot // page, slot % page
+    for name, x in (("k", wl.k[idx]), ("v", wl.v[idx])):
+        for full, part in zip(got[name], affine_quantize(x, 64, 4)):
+            exp = np.zeros_like(full)
+            exp[b, o] = part
+            np.testing.assert_array_equal(full, exp)

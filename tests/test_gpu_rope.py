@@ -227,3 +227,20 @@ def test_fp8_concatenate_fused_vs_callable(cuda):
             outs.append(o.float().cpu().numpy())
         torch.cuda.synchronize()
         assert_attention_close(outs[0], outs[1].astype(np.float64), f"fp8 fused vs callable {qlens}")
+
+
+@pytest.mark.parametrize("rows,heads,d,dims,traditional", [(1, 1, 64, 64, False), (3, 5, 128, 64, False),
+                                                           (17, 32, 128, 128, True), (33, 3, 256, 256, False),
+                                                           (5, 1, 32, 16, False), (9, 2, 256, 8, True)])
+def test_rope_rows_pieces_same_bits(cuda, rows, heads, d, dims, traditional):
+    """16-byte pieces with a table of angles against the pair-at-a-time kernel (a view 8 bytes off takes it)."""
+    print(f"[rope rows pieces {rows}x{heads}x{d} rot {dims} traditional={traditional}]", flush=True)
+    rng = np.random.default_rng(rows)
+    rope = RotaryEmbedding(dims, base=500000.0, traditional=traditional)
+    x = torch.from_numpy(rng.standard_normal((rows, heads, d)).astype(np.float16)).to(cuda)
+    pos = torch.from_numpy(rng.integers(0, 100000, rows).astype(np.int32)).to(cuda)
+    off = torch.empty(x.numel() + 4, dtype=torch.float16, device=cuda)[4:].view_as(x).copy_(x)
+    assert x.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 8
+    _rope_rows(x, pos, rope)
+    _rope_rows(off, pos, rope)
+    assert torch.equal(x, off)
