@@ -95,6 +95,7 @@ def _is_single_token_decode(query_start_loc: torch.Tensor, total_tokens: int) ->
 
 _ws_lock = threading.Lock()
 _ws_cache: dict[tuple[int, int], torch.Tensor] = {}
+_ws_outgrown: list[torch.Tensor] = []
 
 
 def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
@@ -102,7 +103,9 @@ def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor |
 
     Launches on one stream are serialised, so one buffer per (device, stream)
     is race-free.  It is zero-filled when allocated: the library keeps its
-    arrival counters zero between calls.
+    arrival counters zero between calls.  A buffer grows at least twofold and the
+    one it replaces stays allocated, for the replays of a graph that was captured
+    with it: together at most the size of the last.
     """
     if nbytes == 0:
         return None
@@ -111,10 +114,32 @@ def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor |
         ws = _ws_cache.get(key)
         if ws is None or ws.numel() < nbytes:
             if ws is not None:
-                torch.cuda.current_stream(device).synchronize()  # the old buffer may still be in use
+                _ws_outgrown.append(ws)
+                nbytes = max(nbytes, 2 * ws.numel())
             ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
             _ws_cache[key] = ws
         return ws
+
+
+def _call_workspace(lib, device: torch.device, stream: int, total: int, S: int, hq: int, hkv: int, d: int,
+                    max_blocks: int, bs: int, decode: bool, dense: bool = False) -> torch.Tensor | None:
+    """The stream's workspace for one call; for a ragged call with the room in which long tiles are cut into parts.
+
+    A captured ragged call does not grow the stream's buffer for that room, and over unquantized caches it takes no
+    buffer at all: every row then runs as an uncut query tile, with nothing shared between a replay and the stream's
+    own work.
+    """
+    need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
+    if need == 0 or decode:
+        return _workspace(device, stream, need)
+    full = need + int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
+    if torch.cuda.is_current_stream_capturing():
+        if dense:
+            return None
+        held = _ws_cache.get((device.index if device.index is not None else torch.cuda.current_device(), stream))
+        if held is not None and held.numel() < full:
+            full = need
+    return _workspace(device, stream, full)
 
 
 def _i32(t, device) -> torch.Tensor:
@@ -204,11 +229,8 @@ def paged_attention(
         if queries.dtype != torch.float16:
             raise NotImplementedError("affine paged attention takes fp16 queries")
         nb, hkv, bs = int(key_cache.shape[0]), int(key_cache.shape[1]), int(key_cache.shape[2])
-        need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
-        if need and not single_token_decode:  # room for the prefill key split
-            need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
-        if need and workspace is None:
-            workspace = _workspace(dev, stream, need)
+        if workspace is None:
+            workspace = _call_workspace(lib, dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode)
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
         tensors = [key_cache, value_cache, k_scales, k_biases, v_scales, v_biases]
@@ -240,11 +262,8 @@ def paged_attention(
         v_scale = v_scale.to(device=dev, dtype=torch.float32).contiguous()
         if k_scale.numel() != nb or v_scale.numel() != nb:
             raise ValueError("k_scale/v_scale must hold one scale per block: [num_blocks]")
-        need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
-        if need and not single_token_decode:  # room for the prefill key split
-            need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
-        if need and workspace is None:
-            workspace = _workspace(dev, stream, need)
+        if workspace is None:
+            workspace = _call_workspace(lib, dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode)
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
         _native.check(
@@ -264,13 +283,9 @@ def paged_attention(
     key_cache = key_cache.contiguous()
     value_cache = value_cache.contiguous()
     nb, bs, hkv = int(key_cache.shape[0]), int(key_cache.shape[1]), int(key_cache.shape[2])
-    need = 0
-    if single_token_decode or queries.dtype != torch.float32:
-        need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
-        if need and not single_token_decode:  # room for the prefill key split
-            need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
-    if need and workspace is None:
-        workspace = _workspace(dev, stream, need)
+    if workspace is None and (single_token_decode or queries.dtype != torch.float32):
+        workspace = _call_workspace(lib, dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode,
+                                    dense=True)
     ws_ptr = workspace.data_ptr() if workspace is not None else None
     ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
     _native.check(

@@ -228,6 +228,31 @@ def test_ragged_without_workspace(cuda):
     check(b, out.double().cpu().numpy(), expected(b))
 
 
+def test_ragged_captured(cuda):
+    """A ragged call over unquantized pages in a graph, after a smaller call on the stream: each replay as eager."""
+    print("[token-major ragged, captured]", flush=True)
+    small = batch("f16", [1, 1], [20, 30], 4, 2, 128, 16, seed=2)
+    b = batch("f16", [q for q, _ in RAGGED], [k for _, k in RAGGED], 4, 2, 128, 16, seed=5)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+    q, k, v = b["q"].to(cuda), b["cache"][0].to(cuda), b["cache"][1].to(cuda)
+    args, out = [t(b[n]) for n in ("tables", "kvl", "qsl")], torch.empty_like(q)
+    exp = expected(b)
+    side = torch.cuda.Stream(cuda)
+    with torch.cuda.stream(side):
+        run(small, cuda)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        paged_attention(q, k, v, *args, single_token_decode=False, out=out)
+    for _ in range(3):
+        out.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        check(b, out.double().cpu().numpy(), exp)
+        with torch.cuda.stream(side):  # eager work on the stream of the capture
+            check(b, run(b, cuda, decode=False), exp)
+
+
 def test_ragged_infinities(cuda):
     """A value a row does not see (a later token of the prompt, a stale one) leaves it as it is."""
     print("[token-major ragged infinities]", flush=True)
