@@ -92,6 +92,18 @@ long prefill_max_items(int num_tokens, int num_seqs, int tokb) {
   return (long)(num_tokens + tokb - 1) / tokb + std::min(num_seqs, num_tokens / 2);
 }
 
+// Tiles over all kv heads up to which the prefill kernel cuts them into parts.  More keep
+// the 256 compute units full uncut, without partials to store and merge.  4-bit pages of 128,
+// cut / uncut us: 264 tiles (a 1000-token prompt) 36 / 49, 776 (four 512-token chunks after
+// 2048 tokens beside 28 rows) 88 / 106, 888 (six such chunks beside 8) 158 / 134, 1056 (four
+// 2048-token prompts) 289 / 235, 1288 (eight chunks beside 28) 236 / 209, 2056 (an 8192-token
+// prompt) 822 / 767; at eight 8-bit chunks 238 / 221.
+constexpr long kPrefillCutTiles = 832;
+bool prefill_cuts(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads) {
+  return prefill_max_items(num_tokens, num_seqs, 128 / (num_q_heads / num_kv_heads)) * num_kv_heads <=
+         kPrefillCutTiles;
+}
+
 // Wires the key split of the prefill kernel when the workspace holds the
 // partial states after the decode region (`need` bytes).
 void prefill_split(emx::PrefillArgs& p, int num_tokens, int num_q_heads, int num_kv_heads, void* workspace,
@@ -101,7 +113,9 @@ void prefill_split(emx::PrefillArgs& p, int num_tokens, int num_q_heads, int num
   p.ws_cnt = nullptr;
   p.ws_part = nullptr;
   const size_t extra = emx_paged_prefill_workspace_bytes(num_tokens, p.S, num_q_heads, num_kv_heads, 128);
-  if (extra == 0 || workspace == nullptr || workspace_bytes < need + extra) return;
+  if (extra == 0 || workspace == nullptr || workspace_bytes < need + extra ||
+      !prefill_cuts(num_tokens, p.S, num_q_heads, num_kv_heads))
+    return;
   const size_t base = (need + 255) & ~(size_t)255;
   p.nparts = emx::kPrefillParts;
   p.max_items = (int)prefill_max_items(num_tokens, p.S, 128 / (num_q_heads / num_kv_heads));
@@ -1066,8 +1080,10 @@ size_t emx_paged_ragged_workspace_bytes(int num_tokens, int num_seqs, int num_q_
     return 0;
   const size_t part = emx::mixed_mfma_part_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim,
                                                  emx::kPrefillCounters);
+  const size_t affine =
+      emx_paged_prefill_workspace_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim);
   return std::max(part ? 256 + part : 0,
-                  emx_paged_prefill_workspace_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim));
+                  affine && prefill_cuts(num_tokens, num_seqs, num_q_heads, num_kv_heads) ? affine : 0);
 }
 
 size_t emx_paged_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads, int head_dim,

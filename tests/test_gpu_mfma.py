@@ -228,6 +228,24 @@ def test_ragged_without_workspace(cuda):
     check(b, out.double().cpu().numpy(), expected(b))
 
 
+@pytest.mark.parametrize("kind,page,seqs,qlen,ctx,hq,hkv", [
+    ("f16", 16, 1, 1290, 1290, 64, 1), ("bf16", 16, 2, 645, 1300, 64, 1),  # about 645 tiles: in two parts
+    ("f16", 16, 3, 560, 700, 64, 1),                                      # about 840: uncut
+    ("q4", 128, 4, 190, 800, 128, 8), ("q4", 128, 4, 215, 800, 128, 8)])  # the affine kernel: cut, uncut
+def test_ragged_many_tiles(cuda, kind, page, seqs, qlen, ctx, hq, hkv):
+    """Tile counts on both sides of the lines at which fewer parts are cut, tiles longer than a part."""
+    print(f"[ragged {seqs}x{qlen}/{ctx} {kind} {hq}/{hkv}]", flush=True)
+    d = 128 if kind == "q4" else 64
+    b = batch(kind, [qlen] * seqs + [1], [ctx] * seqs + [77], hq, hkv, d, page, seed=qlen)
+    got, exp = run(b, cuda, decode=False), expected(b)
+    if kind != "q4":
+        check(b, got, exp)
+        return
+    # prefill_affine rounds values and probabilities to fp16: 2^-11 of the largest value each, beside the output's
+    bound = 2.0 ** -11 * np.abs(exp) + 2 * 2.0 ** -11 * np.abs(b["exact"][1]).max()
+    assert (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
+
+
 def test_ragged_captured(cuda):
     """A ragged call over unquantized pages in a graph, after a smaller call on the stream: each replay as eager."""
     print("[token-major ragged, captured]", flush=True)
