@@ -148,7 +148,18 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   h16* kbe = &lds_at<h16>(oKbe);          // affine: bias operand rows, key bias of group g at 2 g, 2 g + 1
 
   // ---- work item: tiles per sequence, scanned by the workgroup; the last tile (most keys) first
-  {
+  const int kvh = bid % a.Hkv;
+  const int item = bid / a.Hkv / A.nparts;
+  int part = (bid / a.Hkv) % A.nparts;
+  // workgroups go round the chip in turn, so that with two parts the uncut tiles, which use one
+  // of the two, would take every other place (half the chip idle: 512-token prompts 48.5 against
+  // 37.2 us at three parts): the part that works changes place every other tile
+  if (A.nparts == 2) part ^= (item >> 1) & 1;
+  TileItem ti;
+  if (a.S <= 64) {
+    ti = tile_item64(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, item);
+    if (ti.tile < 0) return;
+  } else {
     const int ch = (a.S + 255) / 256, s0 = tid * ch;
     int tsum = 0;
     for (int i = 0; i < ch; ++i) {
@@ -178,28 +189,22 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
       run += n;
     }
     if (tid == 255) tcum[a.S] = base + x;
+    __syncthreads();
+    if (item >= tcum[a.S]) return;
+    int s = 0;
+    for (int c = 0; c < a.S; c += 64) {
+      const int si = c + lane;
+      s += __builtin_popcountll(__ballot(si < a.S && tcum[si + 1] <= item));
+    }
+    s = __builtin_amdgcn_readfirstlane(s);
+    ti.tile = __builtin_amdgcn_readfirstlane(tcum[s + 1] - 1 - item);
+    ti.s = s;
+    ti.q0 = __builtin_amdgcn_readfirstlane(a.qsl[s]);
+    ti.qlen = __builtin_amdgcn_readfirstlane(a.qsl[s + 1]) - ti.q0;
+    ti.kv_len = __builtin_amdgcn_readfirstlane(a.kv_lens[s]);
   }
-  __syncthreads();
-  const int ntiles = tcum[a.S];
-  const int kvh = bid % a.Hkv;
-  const int item = bid / a.Hkv / A.nparts;
-  int part = (bid / a.Hkv) % A.nparts;
-  // workgroups go round the chip in turn, so that with two parts the uncut tiles, which use one
-  // of the two, would take every other place (half the chip idle: 512-token prompts 48.5 against
-  // 37.2 us at three parts): the part that works changes place every other tile
-  if (A.nparts == 2) part ^= (item >> 1) & 1;
-  if (item >= ntiles) return;
-  int s = 0;
-  for (int c = 0; c < a.S; c += 64) {
-    const int si = c + lane;
-    s += __builtin_popcountll(__ballot(si < a.S && tcum[si + 1] <= item));
-  }
-  s = __builtin_amdgcn_readfirstlane(s);
-  const int nt_s = tcum[s + 1] - tcum[s];
-  const int tile = __builtin_amdgcn_readfirstlane(nt_s - 1 - (item - tcum[s]));
-  const int q0 = __builtin_amdgcn_readfirstlane(a.qsl[s]);
-  const int qlen = __builtin_amdgcn_readfirstlane(a.qsl[s + 1]) - q0;
-  const int kv_len = __builtin_amdgcn_readfirstlane(min(max(a.kv_lens[s], 0), a.max_blocks * a.bs));
+  const int s = ti.s, tile = ti.tile, q0 = ti.q0, qlen = ti.qlen;
+  const int kv_len = min(max(ti.kv_len, 0), a.max_blocks * a.bs);
   const int past = kv_len - qlen;  // query i sees keys [.., past + i]
   const int tok_lo = tile * A.tokb;
   const int HG = a.Hq / a.Hkv;

@@ -86,6 +86,11 @@ def check(b, got, exp):
     assert (err <= bound).all(), f"{int((err > bound).sum())} of {err.size}, worst {(err / bound).max():.2f} of the bound"
 
 
+def affine_bound(b, exp):
+    """prefill_affine rounds values and probabilities to fp16: 2^-11 of the largest value each, beside the output's."""
+    return 2.0 ** -11 * np.abs(exp) + 2 * 2.0 ** -11 * np.abs(b["exact"][1]).max()
+
+
 # item (128), wave (32) and quad (4) edges, and contexts cut between workgroups
 CONTEXTS = [1, 3, 31, 32, 33, 127, 128, 129, 0, 300, 1000, 5]
 
@@ -241,9 +246,24 @@ def test_ragged_many_tiles(cuda, kind, page, seqs, qlen, ctx, hq, hkv):
     if kind != "q4":
         check(b, got, exp)
         return
-    # prefill_affine rounds values and probabilities to fp16: 2^-11 of the largest value each, beside the output's
-    bound = 2.0 ** -11 * np.abs(exp) + 2 * 2.0 ** -11 * np.abs(b["exact"][1]).max()
-    assert (np.abs(got - exp) <= bound).all(), (np.abs(got - exp) / bound).max()
+    assert (np.abs(got - exp) <= affine_bound(b, exp)).all()
+
+
+@pytest.mark.parametrize("kind,page,hq", [("f16", 16, 6), ("q4", 128, 8)])  # prefill_mfma, prefill_affine
+@pytest.mark.parametrize("seqs", [15, 16, 17, 33, 63, 64, 65, 130])
+def test_ragged_sequence_counts(cuda, kind, page, hq, seqs):
+    """Tiles found by a wave's scan (rows of 16 lanes, up to 64 sequences) and by the workgroup's."""
+    print(f"[ragged {seqs} sequences {kind}]", flush=True)
+    rng = np.random.default_rng(seqs)
+    qlens = [int(x) for x in rng.choice([0, 1, 2, 31, 64, 65], size=seqs)]
+    qlens[-1] = 40  # the last lane holds a tile
+    b = batch(kind, qlens, [n + int(x) for n, x in zip(qlens, rng.integers(0, 60, size=seqs))], hq, 2, 128, page,
+              seed=seqs)
+    got, exp = run(b, cuda, decode=False), expected(b)
+    if kind == "f16":
+        check(b, got, exp)
+    else:
+        assert (np.abs(got - exp) <= affine_bound(b, exp)).all()
 
 
 def test_ragged_captured(cuda):
