@@ -32,8 +32,8 @@
 // Bound by the matrix and vector units together (the probability parts double the PV
 // products of fp16, triple those of bf16).  It took over from paged_generic, one wave per
 // (token, kv head) on the VALU: four 512-token chunks beside 28 decode rows, bf16, D 128,
-// pages of 16: 20.8 ms -> 128 us; a 1531-token prompt, fp16, D 256, window 700: 9.6 ms ->
-// 53 us; three 203-token chunks beside 9 rows, 4-bit pages of 16: 5.47 ms -> 55 us.  Over 4-bit
+// pages of 16: 20.8 ms -> 110 us; a 1531-token prompt, fp16, D 256, window 700: 9.6 ms ->
+// 51 us; three 203-token chunks beside 9 rows, 4-bit pages of 16: 5.47 ms -> 52 us.  Over 4-bit
 // pages of 128 tokens prefill_affine (value codes dequantized to fp16 once per workgroup)
 // remains the faster kernel where it applies.
 #pragma once

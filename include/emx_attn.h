@@ -330,10 +330,11 @@ size_t emx_paged_prefill_workspace_bytes(int num_tokens, int num_seqs, int num_q
                                          int head_dim);
 
 /*
- * The same for ragged calls of emx_paged_attention_dense (fp16 / bf16) and
- * emx_paged_attention_fp8 over every shape their MFMA kernels take (head_dim
- * 64, 128 or 256, pages of a multiple of 8 tokens, any GQA ratio up to 128, 64
- * at head_dim 256): at least emx_paged_prefill_workspace_bytes(...).
+ * The same for ragged calls of emx_paged_attention_dense (fp16 / bf16),
+ * emx_paged_attention_fp8 and emx_paged_attention_affine over every shape their
+ * MFMA kernels take (head_dim 64, 128 or 256, pages of a multiple of 8 tokens,
+ * any GQA ratio up to 128, 64 at head_dim 256).  0 where a launch has enough
+ * tiles to fill the GPU uncut.
  */
 size_t emx_paged_ragged_workspace_bytes(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads,
                                         int head_dim);
@@ -342,8 +343,10 @@ size_t emx_paged_ragged_workspace_bytes(int num_tokens, int num_seqs, int num_q_
  * Paged attention over affine pages; queries/out fp16 [num_tokens, Hq, head_dim].
  * block_tables int32 [num_seqs, max_blocks_per_seq]; kv_lens int32 [num_seqs];
  * query_start_loc int32 [num_seqs+1].  single_token_decode != 0 means token i
- * belongs to sequence i (num_tokens == num_seqs) and selects the split-K MFMA
- * decode kernel when head_dim == 128 and page_size % 128 == 0.
+ * belongs to sequence i (num_tokens == num_seqs) and selects the split-K
+ * decode kernels (head_dim 128 with page_size % 128 == 0 needs the workspace;
+ * head_dim 64, 128 or 256 over other pages of a multiple of 8 tokens uses the
+ * matrix units with one).
  * Replaces: paged_attention(...) lib/python/easymlx/operations/kernels/unified_attention.py:1377-1512
  *   (kernels :290-609 and FP8 in-kernel dequant :776-1268), with
  *   k_scale/v_scale generalised to per-(token, group) scales and biases.
@@ -444,8 +447,10 @@ int emx_fp8_cache_write_rope(const void* keys, const void* values, int dtype, co
  * K = dec(code) * k_scale[page].  queries/out in dtype (EMX_DTYPE_*).
  * With fp16 queries, head_dim 128 and page_size % 32 == 0, decode rows run on
  * the split-K decode kernel, which needs the workspace sized by
- * emx_paged_workspace_bytes (same rules as emx_paged_attention_affine);
- * other calls ignore it.
+ * emx_paged_workspace_bytes (same rules as emx_paged_attention_affine).  Other
+ * fp16 calls with head_dim 64, 128 or 256 and pages of a multiple of 8 tokens
+ * run on the matrix units: single-token decode when the workspace holds those
+ * bytes, ragged calls with or without it.
  * Replaces: paged_attention(..., k_scale=, v_scale=)
  *   lib/python/easymlx/operations/kernels/unified_attention.py:1377-1512 with the
  *   FP8 kernels :776-1268 (decoder :1275-1285).
