@@ -97,7 +97,8 @@ long prefill_max_items(int num_tokens, int num_seqs, int tokb) {
 // cut / uncut us: 264 tiles (a 1000-token prompt) 36 / 49, 776 (four 512-token chunks after
 // 2048 tokens beside 28 rows) 88 / 106, 888 (six such chunks beside 8) 158 / 134, 1056 (four
 // 2048-token prompts) 289 / 235, 1288 (eight chunks beside 28) 236 / 209, 2056 (an 8192-token
-// prompt) 822 / 767; at eight 8-bit chunks 238 / 221.
+// prompt) 822 / 767; at eight 8-bit chunks 238 / 221.  FP8 pages of 128: 297 / 253 (four
+// 2048-token prompts), 564 / 579 (eight chunks after 8192 tokens, the one size found slower uncut).
 constexpr long kPrefillCutTiles = 832;
 bool prefill_cuts(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads) {
   return prefill_max_items(num_tokens, num_seqs, 128 / (num_q_heads / num_kv_heads)) * num_kv_heads <=
