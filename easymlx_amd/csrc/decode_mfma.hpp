@@ -44,6 +44,7 @@ struct DecodeMfmaArgs {
   DecodeArgs d;      // kc / vc: the caches; nt: DecodeMfmaCfg::NT; ws_cnt, ws_o [slot][hc][D], ws_ml [slot][hc][2]
   int hc, nhc;       // query heads per unit (<= 16) and units per kv head
   uint32_t inv_bs;   // ceil(2^32 / bs)
+  int T;             // query rows
 };
 
 // Items longer than this many on average are cut freely; below, a unit that would be cut
@@ -144,11 +145,11 @@ __device__ __forceinline__ bool write4(const f32x4 O, const float L, QT* out) {
 }
 
 // Per-sequence tables in LDS: cum[s] = items (of NT tokens, per unit) of the decoded
-// sequences before s, kvl[s] = clamped kv_len (-1: not a single-token row), qrw[s] = query row.
+// sequences before s, kvl[s] = clamped kv_len (-1: not a single-token row of the call's T), qrw[s] = query row.
 // (seq_table of decode_affine.hpp with a constant item size: its two divisions by a run-time
 // one and the serial 64-bit range arithmetic were a third of a short call.)
 template <int NT>
-__device__ __forceinline__ void decode_mfma_table(const DecodeArgs& a, int* cum, int* kvl, int* qrw, int* wsum) {
+__device__ __forceinline__ void decode_mfma_table(const DecodeArgs& a, const int T, int* cum, int* kvl, int* qrw, int* wsum) {
   const int ch = (a.S + 255) / 256, s0 = threadIdx.x * ch;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   int tsum = 0;
@@ -157,7 +158,7 @@ __device__ __forceinline__ void decode_mfma_table(const DecodeArgs& a, int* cum,
     if (s >= a.S) break;
     const int kl = max(min(a.kv_lens[s], a.max_blocks * a.bs), 0);
     const int q0 = a.qsl ? a.qsl[s] : s, q1 = a.qsl ? a.qsl[s + 1] : s + 1;
-    const bool dec = q1 - q0 == 1;
+    const bool dec = q1 - q0 == 1 && (unsigned)q0 < (unsigned)T;
     const int st = a.window > 0 ? max(0, kl - a.window) : 0;
     const int n = dec && kl > 0 ? (kl - 1) / NT - st / NT + 1 : 0;
     kvl[s] = dec ? kl : -1;
@@ -213,7 +214,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   float* xml = &lds_at<float>(oXml);    // [wave][head][2]
   int& flag = lds_at<int>(oFlag);
   h16* stage = &lds_at<h16>(oStage) + wv * P::STAGE;  // affine: this wave's [array][group][token] scales
-  decode_mfma_table<NT>(a, cum, kvl, qrw, reinterpret_cast<int*>(xml));
+  decode_mfma_table<NT>(a, A.T, cum, kvl, qrw, reinterpret_cast<int*>(xml));
   const int S = a.S, HG = a.Hq / a.Hkv, Hu = a.Hkv * A.nhc;
   {  // decoded sequences without a live token produce zeros (the reference's l == 0 case)
     const int per_seq = a.Hq * D / 8;

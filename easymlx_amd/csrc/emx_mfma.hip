@@ -90,6 +90,7 @@ static DecodeMfmaArgs decode_args(const MfmaCall& c, int* ws_cnt, float* partial
   A.hc = head_chunk(c.Hq, c.Hkv);
   A.nhc = head_chunks(c.Hq, c.Hkv);
   A.inv_bs = (uint32_t)(((1ULL << 32) + c.bs - 1) / c.bs);
+  A.T = c.T;
   a.ws_cnt = ws_cnt;
   a.ws_o = partials;
   a.ws_ml = partials + (kDecodeMfmaWGs + (size_t)c.S * c.Hkv * A.nhc) * A.hc * c.D;
@@ -163,6 +164,8 @@ void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_
   p.min_q = ws_cnt ? 2 : 1;
   p.tokb = 64 * ct_of(c.D) / (c.Hq / c.Hkv);
   const long items = tile_items(c.T, c.S, p.tokb, p.min_q);
+  p.T = c.T;
+  p.items = (int)items;
   p.nparts = part ? tile_parts(items * c.Hkv) : 1;
   p.max_items = part ? (int)items : 0;
   p.ws_cnt = ws_part_cnt;

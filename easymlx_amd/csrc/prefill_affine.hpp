@@ -102,20 +102,21 @@ __device__ __forceinline__ int prefill_tiles(const PrefillArgs& a, const int s, 
 __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >> 2) + 4 * (k >> 4) + (k & 3); }
 
 // The query tile `item` of a launch over at most 64 sequences: its sequence, the tile within it
-// (the last, with most keys, first) and the sequence's lengths; tile < 0: no such item.  Every
+// (the last, with most keys, first), the sequence's lengths and the launch's tiles; tile < 0: no such item.  Every
 // wave finds it alone, a sequence to a lane: one trip to memory and a scan in registers, where the
 // workgroup's scan through LDS (any number of sequences) has two trips and two barriers before
 // the first query is read.  4-bit pages of 128, four 512-token chunks beside 28 rows 87.1 -> 85.0
 // us, without a prefix 48.4 -> 45.7; sixteen 256-token chunks 57.7 -> 55.7; prefill_mfma, two
-// 700-token chunks at head_dim 64 26.7 -> 24.0.
+// 700-token chunks at head_dim 64 26.7 -> 24.0.  `rows`: query rows of the call; tiles past the
+// last one are not counted.
 struct TileItem {
-  int tile, s, q0, qlen, kv_len;
+  int tile, s, q0, qlen, kv_len, total;
 };
 __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
-                                                int item) {
+                                                int item, int rows = INT32_MAX) {
   const int lane = threadIdx.x & 63, si = min(lane, S - 1);
   const int q0 = qsl[si], ql = qsl[si + 1] - q0, kv = kv_lens[si];
-  const int n = lane < S && ql >= min_q ? (ql + tokb - 1) / tokb : 0;
+  const int n = lane < S && ql >= min_q ? (max(min(ql, rows - max(q0, 0)), 0) + tokb - 1) / tokb : 0;
   int x = n;  // inclusive scan: rows of 16 lanes, then the totals of the rows below
   x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
   x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
@@ -124,9 +125,10 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
   x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
   x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
   const int s = __builtin_popcountll(__ballot(x <= item));
-  if (s > 63) return {-1, 0, 0, 0, 0};
+  const int total = __builtin_amdgcn_readlane(x, 63);
+  if (s > 63) return {-1, 0, 0, 0, 0, total};
   return {__builtin_amdgcn_readlane(x, s) - 1 - item, s, __builtin_amdgcn_readlane(q0, s),
-          __builtin_amdgcn_readlane(ql, s), __builtin_amdgcn_readlane(kv, s)};
+          __builtin_amdgcn_readlane(ql, s), __builtin_amdgcn_readlane(kv, s), total};
 }
 
 // FP8: the same kernel over an FP8 cache, on the 64-key step geometry of BITS 4

@@ -48,6 +48,8 @@ struct PrefillMfmaArgs {
   uint32_t inv_bs;  // ceil(2^32 / bs)
   int min_q;        // sequences with fewer query tokens are not taken
   int tokb;         // query tokens per tile: columns / HG
+  int T;            // query rows
+  int items;        // tiles per kv head the grid has room for
   int nparts, max_items;
   int* ws_cnt;      // [max_items * Hkv * 4], zero before and after every launch
   float* ws_part;   // [max_items * Hkv][nparts][part bytes]
@@ -115,6 +117,21 @@ __device__ __forceinline__ u32x2 read_tr(const uint16_t* v, const int stride, co
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p));
 }
 
+// Query rows that no sequence holds (before query_start_loc[0], a padded call's rows past the
+// last entry) are zeros, as the reference's (unified_attention.py:341-344).  Written by the grid's
+// workgroups past the last tile, `idx` of `n` (there are some whenever there are such rows: tile_items
+// rounds the call's rows up to tiles, and counts one tile more for every sequence that can have tiles).
+template <class QT>
+__device__ void zero_other_rows(const DecodeArgs& a, const int T, const int D, const int idx, const int n) {
+  const int lo = min(max(a.qsl[0], 0), T), hi = min(max(a.qsl[a.S], lo), T);
+  const int per_row = a.Hq * D / 8;
+  const size_t total = (size_t)(lo + T - hi) * per_row;
+  for (size_t i = (size_t)idx * 256 + threadIdx.x; i < total; i += (size_t)n * 256) {
+    const size_t r = i / per_row;
+    reinterpret_cast<u32x4*>(a.out)[(r < lo ? r : r - lo + hi) * per_row + i % per_row] = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
 template <class C, int D, int CT>
 __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, const int bid) {
   using P = PrefillMfmaCfg<C, D, CT>;
@@ -157,16 +174,15 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   if (A.nparts == 2) part ^= (item >> 1) & 1;
   TileItem ti;
   if (a.S <= 64) {
-    ti = tile_item64(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, item);
-    if (ti.tile < 0) return;
+    ti = tile_item64(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, item, A.T);
   } else {
     const int ch = (a.S + 255) / 256, s0 = tid * ch;
     int tsum = 0;
     for (int i = 0; i < ch; ++i) {
       const int si = s0 + i;
       if (si >= a.S) break;
-      const int ql = a.qsl[si + 1] - a.qsl[si];
-      const int n = ql >= A.min_q ? (ql + A.tokb - 1) / A.tokb : 0;
+      const int q0 = a.qsl[si], ql = a.qsl[si + 1] - q0;
+      const int n = ql >= A.min_q ? (max(min(ql, A.T - q0), 0) + A.tokb - 1) / A.tokb : 0;
       tcum[si] = n;  // the count for now
       tsum += n;
     }
@@ -190,18 +206,26 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     }
     if (tid == 255) tcum[a.S] = base + x;
     __syncthreads();
-    if (item >= tcum[a.S]) return;
-    int s = 0;
-    for (int c = 0; c < a.S; c += 64) {
-      const int si = c + lane;
-      s += __builtin_popcountll(__ballot(si < a.S && tcum[si + 1] <= item));
+    ti.total = __builtin_amdgcn_readfirstlane(tcum[a.S]);
+    ti.tile = -1;
+    if (item < ti.total) {
+      int s = 0;
+      for (int c = 0; c < a.S; c += 64) {
+        const int si = c + lane;
+        s += __builtin_popcountll(__ballot(si < a.S && tcum[si + 1] <= item));
+      }
+      s = __builtin_amdgcn_readfirstlane(s);
+      ti.tile = __builtin_amdgcn_readfirstlane(tcum[s + 1] - 1 - item);
+      ti.s = s;
+      ti.q0 = __builtin_amdgcn_readfirstlane(a.qsl[s]);
+      ti.qlen = __builtin_amdgcn_readfirstlane(a.qsl[s + 1]) - ti.q0;
+      ti.kv_len = __builtin_amdgcn_readfirstlane(a.kv_lens[s]);
     }
-    s = __builtin_amdgcn_readfirstlane(s);
-    ti.tile = __builtin_amdgcn_readfirstlane(tcum[s + 1] - 1 - item);
-    ti.s = s;
-    ti.q0 = __builtin_amdgcn_readfirstlane(a.qsl[s]);
-    ti.qlen = __builtin_amdgcn_readfirstlane(a.qsl[s + 1]) - ti.q0;
-    ti.kv_len = __builtin_amdgcn_readfirstlane(a.kv_lens[s]);
+  }
+  if (ti.tile < 0) {
+    const int per = a.Hkv * A.nparts;
+    zero_other_rows<QT>(a, A.T, D, bid - ti.total * per, (A.items - ti.total) * per);
+    return;
   }
   const int s = ti.s, tile = ti.tile, q0 = ti.q0, qlen = ti.qlen;
   const int kv_len = min(max(ti.kv_len, 0), a.max_blocks * a.bs);
@@ -219,10 +243,10 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     chead[ct] = c - t * HG;
     limit[ct] = min(past + ctok[ct], kv_len - 1);
     start[ct] = a.window > 0 ? max(0, past + ctok[ct] - a.window + 1) : 0;
-    if (t >= A.tokb || ctok[ct] >= qlen) ctok[ct] = -1;  // no such column
+    if (t >= A.tokb || ctok[ct] >= qlen || (unsigned)(q0 + ctok[ct]) >= (unsigned)A.T) ctok[ct] = -1;  // no such column
     if (ctok[ct] < 0) limit[ct] = -1;
   }
-  const int t_last = min(tok_lo + A.tokb, qlen) - 1;
+  const int t_last = min(tok_lo + A.tokb, min(qlen, A.T - q0)) - 1;
   const int k_hi = min(past + t_last, kv_len - 1);
   const int k_lo = a.window > 0 ? max(0, past + tok_lo - a.window + 1) : 0;
   const int steps_all = k_hi >= 0 ? max(k_hi / NT - k_lo / NT + 1, 0) : 0;
@@ -240,7 +264,7 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   for (int ct = 0; ct < CT; ++ct) {
     const bool ok = ctok[ct] >= 0;
     const QT* qp = reinterpret_cast<const QT*>(a.q) +
-                   ((size_t)(q0 + (ok ? ctok[ct] : 0)) * a.Hq + (size_t)kvh * HG + (ok ? chead[ct] : 0)) * D + 8 * jj;
+                   ((size_t)(ok ? q0 + ctok[ct] : 0) * a.Hq + (size_t)kvh * HG + (ok ? chead[ct] : 0)) * D + 8 * jj;
     float gsum[G] = {};
 #pragma unroll
     for (int w = 0; w < P::KS; ++w) {
@@ -674,7 +698,7 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     l += __shfl_xor(l, 32, 64);
     const bool ok = ctok[ct] >= 0;
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    const size_t orow = ((size_t)(q0 + (ok ? ctok[ct] : 0)) * a.Hq + (size_t)kvh * HG + (ok ? chead[ct] : 0)) * D;
+    const size_t orow = ((size_t)(ok ? q0 + ctok[ct] : 0) * a.Hq + (size_t)kvh * HG + (ok ? chead[ct] : 0)) * D;
     QT* op = reinterpret_cast<QT*>(a.out) + orow;
     bool bad = not_finite(l);
 #pragma unroll

@@ -60,7 +60,7 @@ def batch(kind, qlens, kvl, hq, hkv, d, page, seed, invalid=(), gs=64):
                 qsl=np.concatenate([[0], np.cumsum(qlens)]).astype(np.int32))
 
 
-def run(b, dev, window=0, decode=True):
+def run(b, dev, window=0, decode=True, out=None):
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
     sc = b["scales"]
     if isinstance(sc, dict):
@@ -68,7 +68,7 @@ def run(b, dev, window=0, decode=True):
     else:
         kw = dict(k_scale=t(sc[0]), v_scale=t(sc[1])) if sc is not None else {}
     out = paged_attention(b["q"].to(dev), b["cache"][0].to(dev), b["cache"][1].to(dev), t(b["tables"]), t(b["kvl"]),
-                          t(b["qsl"]), sliding_window=window or None, single_token_decode=decode, **kw)
+                          t(b["qsl"]), sliding_window=window or None, single_token_decode=decode, out=out, **kw)
     torch.cuda.synchronize()
     return out.double().cpu().numpy()
 
@@ -212,6 +212,33 @@ def test_ragged_affine_stale_scales(cuda):
     for s_, p in ((0, 61), (1, 36)):
         for n in ("k_scales", "k_biases", "v_scales", "v_biases"):
             b["scales"][n][int(b["tables"][s_, p // 32]), :, :, p % 32] = float("nan")
+    check(b, run(b, cuda, decode=False), exp)
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16", "fp8", "q4"])
+@pytest.mark.parametrize("pad", [(0, 1), (3, 0), (5, 300)], ids=str)
+@pytest.mark.parametrize("seqs", [len(RAGGED), 70])
+def test_ragged_rows_of_no_sequence(cuda, kind, pad, seqs):
+    """Rows before query_start_loc[0] and past its last entry (a padded call) are zeros, the others as without."""
+    print(f"[ragged padded {kind} {pad} {seqs} sequences]", flush=True)
+    lens = (RAGGED * 7)[:seqs] if seqs > 64 else RAGGED
+    qlens = [min(q, 9) for q, _ in lens] if seqs > 64 else [q for q, _ in lens]
+    b = batch(kind, qlens, [min(k, 90) if seqs > 64 else k for _, k in lens], 6, 2, 128, 16, seed=21)
+    b["q"] = torch.cat([torch.ones_like(b["q"][:1]).expand(pad[0], -1, -1), b["q"],
+                        torch.ones_like(b["q"][:1]).expand(pad[1], -1, -1)])
+    b["qsl"] = b["qsl"] + np.int32(pad[0])
+    out = torch.full_like(b["q"], 7.0).to(cuda)
+    check(b, run(b, cuda, decode=False, out=out), expected(b))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "q8"])
+@pytest.mark.parametrize("keep", [1, 34, 100, 199])  # the 34th row is a single-token sequence's, cut inside a chunk
+def test_ragged_query_start_loc_past_the_rows(cuda, kind, keep):
+    """query_start_loc may run past the rows given: those given are as in the whole call, nothing else is touched."""
+    print(f"[ragged {keep} rows of {sum(q for q, _ in RAGGED)} {kind}]", flush=True)
+    b = batch(kind, [q for q, _ in RAGGED], [k for _, k in RAGGED], 6, 2, 128, 16, seed=22)
+    exp = expected(b)[:keep]
+    b["q"] = b["q"][:keep]
     check(b, run(b, cuda, decode=False), exp)
 
 
