@@ -59,6 +59,8 @@ SIGNATURES: dict[str, tuple] = {
     "emx_paged_workspace_bytes": (_SZ, [_I, _I, _I, _I, _I, _I]),
     "emx_paged_prefill_workspace_bytes": (_SZ, [_I, _I, _I, _I, _I]),
     "emx_paged_ragged_workspace_bytes": (_SZ, [_I, _I, _I, _I, _I]),
+    "emx_paged_workspace_zeroed_bytes": (_SZ, []),
+    "emx_stream_capture_id": (_SZ, [_P]),
     "emx_paged_attention_affine": (
         _I,
         [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _I, _P, _P, _F, _I, _I, _P, _SZ, _P, _P],

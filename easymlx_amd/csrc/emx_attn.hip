@@ -1109,6 +1109,19 @@ size_t emx_paged_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads
   return std::max(fast, part ? kPartialsInt * sizeof(int) + part : 0);
 }
 
+size_t emx_paged_workspace_zeroed_bytes(void) { return kPartialsInt * sizeof(int); }
+
+size_t emx_stream_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (!stream) return 0;  // the null stream cannot be captured
+  if (hipStreamGetCaptureInfo(reinterpret_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? id : 0;
+}
+
 int emx_paged_attention_affine(const void* queries, int num_tokens, int num_q_heads, int head_dim,
                                const uint32_t* k_codes, const void* k_scales, const void* k_biases,
                                const uint32_t* v_codes, const void* v_scales, const void* v_biases, int num_blocks,

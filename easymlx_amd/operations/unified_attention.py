@@ -96,9 +96,10 @@ def _is_single_token_decode(query_start_loc: torch.Tensor, total_tokens: int) ->
 _ws_lock = threading.Lock()
 _ws_cache: dict[tuple[int, int], torch.Tensor] = {}
 _ws_outgrown: list[torch.Tensor] = []
+_ws_captured: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}  # (capture, its buffer), the last per stream
 
 
-def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
+def _workspace(device: torch.device, stream: int, nbytes: int, own: bool = False) -> torch.Tensor | None:
     """Split-K workspace shared by the launches of one stream (grow-only).
 
     Launches on one stream are serialised, so one buffer per (device, stream)
@@ -106,18 +107,34 @@ def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor |
     arrival counters zero between calls.  A buffer grows at least twofold and the
     one it replaces stays allocated, for the replays of a graph that was captured
     with it: together at most the size of the last.
+
+    A call under graph capture takes the stream's buffer only if it is large
+    enough (and not ``own``).  Else the calls of the capture share one from the
+    graph's own memory: its counters are cleared by a recorded fill, which has not
+    run before the first replay, so eager calls and other captures never see it.
     """
     if nbytes == 0:
         return None
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
+    own = own and torch.cuda.is_current_stream_capturing()
     with _ws_lock:
         ws = _ws_cache.get(key)
-        if ws is None or ws.numel() < nbytes:
-            if ws is not None:
-                _ws_outgrown.append(ws)
-                nbytes = max(nbytes, 2 * ws.numel())
-            ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
-            _ws_cache[key] = ws
+        if ws is not None and ws.numel() >= nbytes and not own:
+            return ws
+        lib = _native.load()
+        capture = int(lib.emx_stream_capture_id(stream))
+        if capture:
+            held, ws = _ws_captured.get(key, (0, None))
+            if held != capture or ws.numel() < nbytes:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+                ws[:int(lib.emx_paged_workspace_zeroed_bytes())].zero_()
+                _ws_captured[key] = (capture, ws)
+            return ws
+        if ws is not None:
+            _ws_outgrown.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        _ws_cache[key] = ws
         return ws
 
 
@@ -125,21 +142,14 @@ def _call_workspace(lib, device: torch.device, stream: int, total: int, S: int, 
                     max_blocks: int, bs: int, decode: bool, dense: bool = False) -> torch.Tensor | None:
     """The stream's workspace for one call; for a ragged call with the room in which long tiles are cut into parts.
 
-    A captured ragged call does not grow the stream's buffer for that room, and over unquantized caches it takes no
-    buffer at all: every row then runs as an uncut query tile, with nothing shared between a replay and the stream's
-    own work.
+    A captured ragged call over unquantized caches takes a buffer of its capture: nothing is shared between a replay
+    and the stream's own work.
     """
     need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
     if need == 0 or decode:
         return _workspace(device, stream, need)
-    full = need + int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
-    if torch.cuda.is_current_stream_capturing():
-        if dense:
-            return None
-        held = _ws_cache.get((device.index if device.index is not None else torch.cuda.current_device(), stream))
-        if held is not None and held.numel() < full:
-            full = need
-    return _workspace(device, stream, full)
+    need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
+    return _workspace(device, stream, need, own=dense)
 
 
 def _i32(t, device) -> torch.Tensor:

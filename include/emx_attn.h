@@ -317,6 +317,22 @@ size_t emx_paged_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads
                                  int max_blocks_per_seq, int page_size);
 
 /*
+ * The part of a workspace, from its start, that has to be zero before its first
+ * use (arrival counters and the plan cache; the same for every call).  What
+ * follows may hold anything.
+ * No direct reference counterpart (emx_paged_workspace_bytes).
+ */
+size_t emx_paged_workspace_zeroed_bytes(void);
+
+/*
+ * The id of the graph capture that `stream` is part of, 0 if it is not capturing:
+ * a workspace made under capture is cleared by the replays only, so it is kept
+ * apart from the stream's own.
+ * No direct reference counterpart.
+ */
+size_t emx_stream_capture_id(void* stream);
+
+/*
  * Extra workspace bytes, after emx_paged_workspace_bytes(...), with which the
  * prefill kernel of emx_paged_attention_affine / emx_paged_attention_fp8 cuts
  * tiles of many keys into up to three parts (one workgroup each) and merges

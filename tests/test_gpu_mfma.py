@@ -318,6 +318,54 @@ def test_ragged_captured(cuda):
             check(b, run(b, cuda, decode=False), exp)
 
 
+@pytest.mark.parametrize("kind,page,decode", [("f16", 16, True), ("q4", 128, True), ("q4", 16, False),
+                                              ("q4", 128, False), ("fp8", 16, False), ("bf16", 16, False)])
+def test_captured_past_the_streams_buffer(cuda, kind, page, decode):
+    """Two captures that need more than the stream's buffer: eager work before any replay, the second replayed first."""
+    print(f"[captured past the buffer {kind} p{page} {'decode' if decode else 'ragged'}]", flush=True)
+    small = batch(kind, [1], [20], 4, 2, 128, page, seed=2)
+    lens = [(1, k) for k in [700, 3, 129, 0, 2000] * 8] if decode else RAGGED
+    b = batch(kind, [q for q, _ in lens], [k for _, k in lens], 4, 2, 128, page, seed=5)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+    q, k, v = b["q"].to(cuda), b["cache"][0].to(cuda), b["cache"][1].to(cuda)
+    sc = b["scales"]
+    if isinstance(sc, dict):
+        kw = {n: x.to(cuda) if isinstance(x, torch.Tensor) else x for n, x in sc.items()}
+    else:
+        kw = dict(k_scale=t(sc[0]), v_scale=t(sc[1])) if sc is not None else {}
+    args, outs = [t(b[n]) for n in ("tables", "kvl", "qsl")], [torch.empty_like(q) for _ in range(2)]
+    exp = expected(b)
+
+    def right(out):
+        got = out.double().cpu().numpy() if isinstance(out, torch.Tensor) else out
+        if kind == "q4" and page == 128:
+            assert (np.abs(got - exp) <= affine_bound(b, exp)).all()
+        else:
+            check(b, got, exp)
+
+    side = torch.cuda.Stream(cuda)
+    with torch.cuda.stream(side):
+        run(small, cuda)
+    torch.cuda.synchronize()
+    graphs = []
+    for out in outs:
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=side):
+            for _ in range(2):  # two layers share the capture's buffer
+                paged_attention(q, k, v, *args, single_token_decode=decode, out=out, **kw)
+    with torch.cuda.stream(side):
+        run(small, cuda, decode=decode)
+        right(run(b, cuda, decode=decode))
+    for _ in range(3):
+        for g, out in zip(graphs[::-1], outs[::-1]):
+            out.fill_(7.0)
+            g.replay()
+            torch.cuda.synchronize()
+            right(out)
+        with torch.cuda.stream(side):
+            right(run(b, cuda, decode=decode))
+
+
 def test_ragged_infinities(cuda):
     """A value a row does not see (a later token of the prompt, a stale one) leaves it as it is."""
     print("[token-major ragged infinities]", flush=True)

@@ -279,6 +279,47 @@ def test_abi_rope_and_prefill_split_arguments(lib):
     assert lib.emx_paged_prefill_workspace_bytes(10 ** 7, 32, 32, 8, 128) == 0  # counters would not fit
 
 
+def test_workspace_of_a_capture_stays_apart(monkeypatch):
+    """A buffer made under graph capture is cleared by replays only: eager calls and other captures never get it."""
+    from easymlx_amd.operations import unified_attention as ua
+
+    class Lib:
+        capture = 0
+
+        def emx_stream_capture_id(self, stream):
+            return self.capture
+
+        def emx_paged_workspace_zeroed_bytes(self):
+            return 64
+
+    lib = Lib()
+    monkeypatch.setattr(ua._native, "load", lambda: lib)
+    monkeypatch.setattr(ua.torch.cuda, "is_current_stream_capturing", lambda: lib.capture != 0)
+    for name in ("_ws_cache", "_ws_captured"):
+        monkeypatch.setattr(ua, name, {}, raising=False)
+    monkeypatch.setattr(ua, "_ws_outgrown", [])
+    dev = torch.device("cpu", 0)
+    get = lambda n, **kw: ua._workspace(dev, 1234, n, **kw)  # noqa: E731
+    lib.capture = 7  # nothing held yet
+    first = get(100)
+    assert first[:64].eq(0).all() and get(80) is first
+    lib.capture = 0
+    eager = get(100)
+    assert eager is not first and eager.eq(0).all()
+    lib.capture = 8
+    assert get(90) is eager  # large enough: captured with the stream's buffer, which eager work keeps cleared
+    grown = get(1000)
+    assert grown is not eager and grown is not first and get(1000) is grown
+    assert get(90, own=True) is grown
+    lib.capture = 9  # another capture, replayed first: not the buffer that capture 8 clears
+    other = get(1000)
+    assert other is not grown
+    lib.capture = 0
+    assert get(100) is eager
+    bigger = get(1000)
+    assert bigger is not grown and bigger is not other and bigger.eq(0).all() and get(100) is bigger
+
+
 def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True,
                        timeout=60)
