@@ -157,6 +157,32 @@ def test_decode_short_contexts_whole_units(cuda):
         check(b, run(b, cuda), expected(b))
 
 
+def test_decode_units_just_past_the_workgroups(cuda):
+    """520 and 528 equal long units over 512 workgroups are cut: as whole units a workgroup would hold two of them,
+    twice an equal share, and the call take nearly twice the time of 512 units (1.5 times at most is asked for)."""
+    print("[decode 65 and 66 long rows]", flush=True)
+    one = batch("f16", [1] * 66, [4096] + [1] * 65, 16, 8, 64, 16, seed=14)
+    one["tables"][:] = one["tables"][0]  # every sequence reads the same pages
+    one["kvl"][:] = 4096
+    exp, took = expected(one), {}
+    for seqs in (64, 65, 66):
+        b = dict(one, q=one["q"][:seqs], tables=one["tables"][:seqs], kvl=one["kvl"][:seqs], qsl=one["qsl"][:seqs + 1])
+        check(b, run(b, cuda), exp[:seqs])
+        q, k, v = b["q"].to(cuda), b["cache"][0].to(cuda), b["cache"][1].to(cuda)
+        args = [torch.from_numpy(b[n]).to(cuda) for n in ("tables", "kvl", "qsl")]
+        best = float("inf")
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            for _ in range(20):
+                paged_attention(q, k, v, *args, single_token_decode=True)
+            t1.record()
+            torch.cuda.synchronize()
+            best = min(best, t0.elapsed_time(t1))
+        took[seqs] = best
+    assert took[65] < 1.5 * took[64] and took[66] < 1.5 * took[64], took
+
+
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_decode_infinities(cuda, kind):
     """An infinity or NaN outside the visible keys leaves a row as it is; a visible infinity stays one."""
