@@ -92,34 +92,34 @@ long prefill_max_items(int num_tokens, int num_seqs, int tokb) {
   return (long)(num_tokens + tokb - 1) / tokb + std::min(num_seqs, num_tokens / 2);
 }
 
-// Tiles over all kv heads up to which the prefill kernel cuts them into parts.  More keep
-// the 256 compute units full uncut, without partials to store and merge.  4-bit pages of 128,
-// cut / uncut us: 264 tiles (a 1000-token prompt) 36 / 49, 776 (four 512-token chunks after
-// 2048 tokens beside 28 rows) 88 / 106, 888 (six such chunks beside 8) 158 / 134, 1056 (four
-// 2048-token prompts) 289 / 235, 1288 (eight chunks beside 28) 236 / 209, 2056 (an 8192-token
-// prompt) 822 / 767; at eight 8-bit chunks 238 / 221.  FP8 pages of 128: 297 / 253 (four
-// 2048-token prompts), 564 / 579 (eight chunks after 8192 tokens, the one size found slower uncut).
-constexpr long kPrefillCutTiles = 832;
-bool prefill_cuts(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads) {
-  return prefill_max_items(num_tokens, num_seqs, 128 / (num_q_heads / num_kv_heads)) * num_kv_heads <=
-         kPrefillCutTiles;
+// Fewest: all tokens are in tiles but one of a sequence at most.
+long prefill_min_items(int num_tokens, int num_seqs, int tokb) {
+  return (std::max(num_tokens - num_seqs, 0) + tokb - 1) / tokb;
+}
+
+// Workspace bytes the parts of a launch's tiles take (the kernel counts the tiles, anything
+// between the two bounds); 0 where the shape cannot split or has too many tiles to be cut.
+size_t prefill_part_bytes(int num_tokens, int num_seqs, int num_q_heads, int num_kv_heads, int head_dim) {
+  if (emx_paged_prefill_workspace_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim) == 0) return 0;
+  const int tokb = 128 / (num_q_heads / num_kv_heads);
+  if (emx::PrefillRule::most_parts(prefill_min_items(num_tokens, num_seqs, tokb) * num_kv_heads, INFINITY) == 1) return 0;
+  const long most = prefill_max_items(num_tokens, num_seqs, tokb) * num_kv_heads;
+  return 256 + (size_t)std::min<long>(most * emx::kPrefillParts, emx::kPrefillCutSlots) * emx::kPrefillPartBytes;
 }
 
 // Wires the key split of the prefill kernel when the workspace holds the
 // partial states after the decode region (`need` bytes).
 void prefill_split(emx::PrefillArgs& p, int num_tokens, int num_q_heads, int num_kv_heads, void* workspace,
                    size_t workspace_bytes, size_t need) {
+  const int tokb = 128 / (num_q_heads / num_kv_heads);
   p.nparts = 1;
-  p.max_items = 0;
+  p.items = (num_tokens + tokb - 1) / tokb + p.S;  // a sequence has at most its tokens / tokb + 1
   p.ws_cnt = nullptr;
   p.ws_part = nullptr;
-  const size_t extra = emx_paged_prefill_workspace_bytes(num_tokens, p.S, num_q_heads, num_kv_heads, 128);
-  if (extra == 0 || workspace == nullptr || workspace_bytes < need + extra ||
-      !prefill_cuts(num_tokens, p.S, num_q_heads, num_kv_heads))
-    return;
+  const size_t extra = prefill_part_bytes(num_tokens, p.S, num_q_heads, num_kv_heads, 128);
+  if (extra == 0 || workspace == nullptr || workspace_bytes < need + extra) return;
   const size_t base = (need + 255) & ~(size_t)255;
-  p.nparts = emx::kPrefillParts;
-  p.max_items = (int)prefill_max_items(num_tokens, p.S, 128 / (num_q_heads / num_kv_heads));
+  p.nparts = emx::PrefillRule::most_parts(prefill_min_items(num_tokens, p.S, tokb) * num_kv_heads, INFINITY);
   p.ws_cnt = reinterpret_cast<int*>(workspace) + kPrefillCounterOff;
   p.ws_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + base);
 }
@@ -464,7 +464,7 @@ bool run_mfma(const emx::MfmaCall& c, void* ws, size_t ws_bytes, hipStream_t st,
     return true;
   }
   if (!emx::mixed_mfma_ok(c)) return false;
-  const size_t part = emx::mixed_mfma_part_bytes(c.T, c.S, c.Hq, c.Hkv, c.D, emx::kPrefillCounters);
+  const size_t part = emx::mixed_mfma_part_bytes(c.T, c.S, c.Hq, c.Hkv, c.D);
   const size_t base = (need + 255) & ~(size_t)255;
   const bool cut = have && part > 0 && ws_bytes >= base + part;
   emx::launch_mixed_mfma(c, have ? wi : nullptr, partials, wi + (cut ? kPrefillCounterOff : 0),
@@ -1079,12 +1079,9 @@ size_t emx_paged_ragged_workspace_bytes(int num_tokens, int num_seqs, int num_q_
                                         int head_dim) {
   if (num_tokens <= 0 || num_seqs <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0)
     return 0;
-  const size_t part = emx::mixed_mfma_part_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                                                 emx::kPrefillCounters);
-  const size_t affine =
-      emx_paged_prefill_workspace_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim);
+  const size_t part = emx::mixed_mfma_part_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim);
   return std::max(part ? 256 + part : 0,
-                  affine && prefill_cuts(num_tokens, num_seqs, num_q_heads, num_kv_heads) ? affine : 0);
+                  prefill_part_bytes(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim));
 }
 
 size_t emx_paged_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads, int head_dim,
@@ -1189,9 +1186,7 @@ int emx_paged_attention_affine(const void* queries, int num_tokens, int num_q_he
       PrefillFn pf = bits == 4 ? pick_prefill_gs<4>(group_size, hg) : pick_prefill_gs<8>(group_size, hg);
       if (!pf)
         return fail(EMX_ERR_UNSUPPORTED, "no prefill kernel for bits=%d group_size=%d gqa=%d", bits, group_size, hg);
-      // tiles of 128/hg query tokens: at most num_tokens/tile + num_seqs of them per kv head
-      const int tokb = 128 / hg;
-      pgrid = (long)((num_tokens + tokb - 1) / tokb + num_seqs) * num_kv_heads * p.nparts;
+      pgrid = (long)p.items * num_kv_heads * p.nparts;
       // prefill and decode rows go out as one launch (below) when a unified kernel
       // pairs this prefill with the decode kernel picked for the rows
       const bool q4u = bits == 4 && (page_size & (page_size - 1)) == 0 && pick_decode_q4(group_size, hg, page_size);
@@ -1639,10 +1634,7 @@ int emx_paged_attention_fp8(const void* queries, int num_tokens, int num_q_heads
     prefill_split(p, num_tokens, num_q_heads, num_kv_heads, workspace, workspace_bytes, need);
     return p;
   };
-  auto prefill_grid = [&](const emx::PrefillArgs& p) {
-    const int tokb = 128 / hg;
-    return (long)((num_tokens + tokb - 1) / tokb + num_seqs) * num_kv_heads * p.nparts;
-  };
+  auto prefill_grid = [&](const emx::PrefillArgs& p) { return (long)p.items * num_kv_heads * p.nparts; };
   auto launch_prefill = [&](int min_q) {
     const emx::PrefillArgs p = prefill_args(min_q);
     hipLaunchKernelGGL(pf, dim3((unsigned)prefill_grid(p)), dim3(256), 0, st, p);

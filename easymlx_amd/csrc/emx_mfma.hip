@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "decode_mfma.hpp"
 #include "mfma_launch.hpp"
@@ -108,14 +109,8 @@ namespace {
 constexpr int ct_of(int D) { return D > 128 ? 1 : 2; }
 // Most query tiles per kv head: a sequence of q >= min_q query tokens has at most q / tokb + 1.
 long tile_items(int T, int S, int tokb, int min_q) { return (long)(T + tokb - 1) / tokb + std::min(S, T / min_q); }
-// Most parts a tile is cut into, by the launch's tiles over all kv heads (256 compute units
-// hold two workgroups each): few tiles are cut to fill the chip, many keep it full uncut and
-// are spared the partials.  3 / 2 / 1 parts, us: 264 tiles (a 1000-token prompt, bf16) 41 / 42 /
-// 59, 512 (2000 tokens) 91 / 92 / 112, 760 (3000 tokens) 172 / 165 / 169, 776 (four 512-token
-// chunks beside 28 rows) 122 / 115 / 119, 888 (3500 tokens, fp16) 197 / 189 / 177, 1024
-// (4 x 2048) 299 / - / 244, 4096 (16384 tokens) 3390 / - / 3195.  At 544 and 1088 tiles of 8700
-// keys the cut is worth 1% and 5% (298 / 288 / 329, 556 / 555 / 583).
-constexpr int tile_parts(long units) { return units <= 640 ? 3 : units <= 832 ? 2 : 1; }
+// Fewest: all but one token of a sequence at most are in tiles.
+long tile_items_least(int T, int S, int tokb) { return (std::max(T - S, 0) + tokb - 1) / tokb; }
 
 typedef void (*MixedFn)(PrefillMfmaArgs, DecodeMfmaArgs, int);
 
@@ -146,13 +141,16 @@ bool mixed_mfma_ok(const MfmaCall& c) {
   return mfma_ok(c) && c.qsl && c.Hq / c.Hkv <= 64 * ct_of(c.D) && (long long)c.nb * c.bs * (c.kind == KvKind::affine ? c.Hkv : 1) < (1LL << 31);
 }
 
-size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_counters) {
+size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D) {
   const int hg = Hq / Hkv;
   if (!head_ok(D) || hg > 64 * ct_of(D)) return 0;
-  const long units = tile_items(T, S, 64 * ct_of(D) / hg, 2) * Hkv;
-  const int parts = tile_parts(units);
-  if (parts == 1 || units * 4 > max_counters) return 0;
-  return (size_t)units * parts * (4 * (ct_of(D) * (D / 16) + 1) * 1024);
+  const int tokb = 64 * ct_of(D) / hg;
+  const long least = tile_items_least(T, S, tokb) * Hkv, most = tile_items(T, S, tokb, 2) * Hkv;
+  const int parts = MfmaRule::most_parts(least, INFINITY);
+  if (parts == 1) return 0;
+  // (tile, part) pairs: the kernel counts the tiles, anything between the two bounds
+  const long slots = std::min<long>(most * parts, 2 * kPrefillCutTiles);
+  return (size_t)slots * (4 * (ct_of(D) * (D / 16) + 1) * 1024);
 }
 
 void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
@@ -166,8 +164,7 @@ void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_
   const long items = tile_items(c.T, c.S, p.tokb, p.min_q);
   p.T = c.T;
   p.items = (int)items;
-  p.nparts = part ? tile_parts(items * c.Hkv) : 1;
-  p.max_items = part ? (int)items : 0;
+  p.nparts = part ? MfmaRule::most_parts(tile_items_least(c.T, c.S, p.tokb) * c.Hkv, INFINITY) : 1;
   p.ws_cnt = ws_part_cnt;
   p.ws_part = part;
   // Decode workgroups by the decode rows' share of the step (at most S of the T rows), so that

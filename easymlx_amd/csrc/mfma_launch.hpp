@@ -43,7 +43,7 @@ void launch_decode_mfma(const MfmaCall& c, int* ws_cnt, float* partials, hipStre
 // ws_cnt null (no workspace): every row as a query tile, nothing cut.  part null: tiles
 // are not cut; else mixed_mfma_part_bytes bytes (ws_part_cnt: their counters).
 bool mixed_mfma_ok(const MfmaCall& c);
-size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D, int max_counters);
+size_t mixed_mfma_part_bytes(int T, int S, int Hq, int Hkv, int D);
 void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_part_cnt, float* part,
                        hipStream_t st);
 

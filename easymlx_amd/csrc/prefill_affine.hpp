@@ -58,9 +58,9 @@ struct PrefillArgs {
   // workgroup each); every wave stores its part's state and the last of a
   // wave's parts merges them.  nparts = 1: no split (ws_* unused).
   int nparts;
-  int max_items;                // tiles the workspace holds per kv head
-  int* ws_cnt;                  // [max_items * Hkv * 4] arrival counters: zero before and after every launch
-  float* ws_part;               // [max_items * Hkv][kPrefillParts][kPrefillPartFloats]
+  int items;                    // tiles per kv head the grid has room for
+  int* ws_cnt;                  // [tiles * 4] arrival counters: zero before and after every launch
+  float* ws_part;               // [tiles][parts][kPrefillPartBytes]
 };
 
 constexpr int kPrefillParts = 3;          // most parts a tile is split into
@@ -68,7 +68,33 @@ constexpr float kLazyMax = 8.f;           // growth of a column's maximum (log2 
 constexpr int kPrefillSplitKeys = 512;    // keys per part the split aims at (c3: 768 -> 121.5, 512 -> 111.7, 384 -> 117.6 us)
 constexpr int kPrefillPartVec = 17;       // f32x4 per lane of a stored state: acc[2][8], (m0, m1, l0, l1)
 constexpr int kPrefillPartBytes = 4 * kPrefillPartVec * 64 * 16;  // one part of one workgroup
-constexpr int kPrefillCounters = 65536;   // arrival counters (max_items * Hkv * 4 must fit)
+constexpr int kPrefillCounters = 65536;   // arrival counters, four a cut tile
+// Most parts of a tile in a launch of `tiles` over all kv heads with contexts of `keys` on
+// average (by tile, at most the window).  The kernel counts both from query_start_loc:
+// single-token rows are no tiles, and the host cannot tell them.  Few tiles are cut to fill the
+// chip; more keep the 256 compute units full uncut, without partials to store and merge, unless
+// contexts are long, where the cut evens out their ends.  Pages of 128 tokens, 3 / 2 / 1 parts, us:
+// 4-bit, 128 tiles (a 512-token chunk beside 96 rows) 72 / 74 / 92, 512 (four beside 96) 86 / 91 /
+// 97, 256 (a 1000-token prompt) 33 / 33 / 48, 640 (five chunks after 3000 tokens) 98 / 109 / 107;
+// 656 (2 x 1300) 96 / 95 / 94, 1024 (4 x 1000) 91 / 98 / 88, (eight chunks after up to 8192) 670 /
+// 647 / 709, 1280 (ten after up to 6000) 481 / 471 / 513; FP8 507 / 499 / 526 and 489 / 527 / 537,
+// 8-bit 642 / 655 / 733 and 444 / 446 / 486; 1504 (4 x 1500) 181 / 186 / 156, 2048 (4 x 2048
+// after up to 4096) 559 / 546 / 500.
+constexpr int kPrefillFewTiles = 640, kPrefillCutTiles = 1280;
+constexpr float kPrefillLongKeys = 2560.f;
+struct PrefillRule {
+  static __host__ __device__ constexpr int most_parts(long tiles, float keys) {
+    return tiles <= kPrefillFewTiles ? kPrefillParts : tiles <= kPrefillCutTiles && keys >= kPrefillLongKeys ? 2 : 1;
+  }
+};
+// Most (tile, part) pairs of a launch.
+constexpr int kPrefillCutSlots =
+    kPrefillParts * kPrefillFewTiles > 2 * kPrefillCutTiles ? kPrefillParts * kPrefillFewTiles : 2 * kPrefillCutTiles;
+static_assert(kPrefillCutTiles * 4 <= kPrefillCounters, "a counter per wave and cut tile");
+// Parts of a tile of `keys` keys.
+__device__ __forceinline__ int prefill_parts(int keys, int most) {
+  return max(1, min(most, (keys + kPrefillSplitKeys - 1) / kPrefillSplitKeys));
+}
 
 template <int BITS, int GS, int HG>
 struct PrefillCfg {
@@ -90,19 +116,14 @@ struct PrefillCfg {
   static_assert(W * NT == 1024, "a step's K codes are 4 KiB: one 16-byte piece per thread");
 };
 
-// Number of query-token tiles of sequence s (0 for decode rows and empty rows).
-__device__ __forceinline__ int prefill_tiles(const PrefillArgs& a, const int s, const int tokb) {
-  const int ql = a.qsl[s + 1] - a.qsl[s];
-  return ql >= a.min_q ? (ql + tokb - 1) / tokb : 0;
-}
-
 // Position, inside its 32-key block, at which the dequantized value of key k
 // (0..31 within the block) is stored: the PV B operand of lane (col, kg) holds
 // keys kg*4 + {0..3} and 16 + kg*4 + {0..3} of the block, in that order.
 __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >> 2) + 4 * (k >> 4) + (k & 3); }
 
-// The query tile `item` of a launch over at most 64 sequences: its sequence, the tile within it
-// (the last, with most keys, first), the sequence's lengths and the launch's tiles; tile < 0: no such item.  Every
+// The query tile and part of workgroup `bid` of a launch over at most 64 sequences (kv head fastest, then
+// the part of as many as the rule allows, then the tile): its sequence, the tile within it (the last, with
+// most keys, first), the sequence's lengths and the launch's tiles; tile < 0: no such tile.  Every
 // wave finds it alone, a sequence to a lane: one trip to memory and a scan in registers, where the
 // workgroup's scan through LDS (any number of sequences) has two trips and two barriers before
 // the first query is read.  4-bit pages of 128, four 512-token chunks beside 28 rows 87.1 -> 85.0
@@ -110,10 +131,13 @@ __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >
 // 700-token chunks at head_dim 64 26.7 -> 24.0.  `rows`: query rows of the call; tiles past the
 // last one are not counted.
 struct TileItem {
-  int tile, s, q0, qlen, kv_len, total;
+  int tile, s, q0, qlen, kv_len;
+  int item, part, most;  // most: parts a tile of this launch may have
+  int total;
 };
+template <class Rule>
 __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
-                                                int item, int rows = INT32_MAX) {
+                                                int window, int bid, int Hkv, int grid_parts, int rows = INT32_MAX) {
   const int lane = threadIdx.x & 63, si = min(lane, S - 1);
   const int q0 = qsl[si], ql = qsl[si + 1] - q0, kv = kv_lens[si];
   const int n = lane < S && ql >= min_q ? (max(min(ql, rows - max(q0, 0)), 0) + tokb - 1) / tokb : 0;
@@ -124,11 +148,92 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
   x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
   x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
   x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
-  const int s = __builtin_popcountll(__ballot(x <= item));
-  const int total = __builtin_amdgcn_readlane(x, 63);
-  if (s > 63) return {-1, 0, 0, 0, 0, total};
-  return {__builtin_amdgcn_readlane(x, s) - 1 - item, s, __builtin_amdgcn_readlane(q0, s),
-          __builtin_amdgcn_readlane(ql, s), __builtin_amdgcn_readlane(kv, s), total};
+  TileItem r;
+  r.total = __builtin_amdgcn_readlane(x, 63);
+  r.most = 1;
+  if (grid_parts > 1) {
+    const int tiles = r.total * Hkv;
+    float keys = 0.f;
+    if (tiles > kPrefillFewTiles && tiles <= kPrefillCutTiles)  // (the sum is worth 0.5 us)
+      keys = wave_sum((float)n * (float)(window > 0 ? min(kv, window) : kv)) / (float)r.total;
+    r.most = __builtin_amdgcn_readfirstlane(min(grid_parts, Rule::most_parts(tiles, keys)));
+  }
+  r.item = bid / Hkv / r.most;
+  r.part = bid / Hkv - r.item * r.most;
+  const int s = __builtin_popcountll(__ballot(x <= r.item));
+  r.tile = -1;
+  if (s > 63) return r;
+  r.tile = __builtin_amdgcn_readlane(x, s) - 1 - r.item;
+  r.s = s;
+  r.q0 = __builtin_amdgcn_readlane(q0, s);
+  r.qlen = __builtin_amdgcn_readlane(ql, s);
+  r.kv_len = __builtin_amdgcn_readlane(kv, s);
+  return r;
+}
+
+// The same for any number of sequences, scanned by the workgroup: tcum [S + 1] and wred [8] in LDS.
+template <class Rule>
+__device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
+                                                  int window, int bid, int Hkv, int grid_parts, int* tcum, int* wred,
+                                                  int rows = INT32_MAX) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int ch = (S + 255) / 256, s0 = tid * ch;
+  int tsum = 0;
+  float ksum = 0.f;
+  for (int i = 0; i < ch; ++i) {
+    const int si = s0 + i;
+    if (si >= S) break;
+    const int q0 = qsl[si], ql = qsl[si + 1] - q0;
+    const int n = ql >= min_q ? (max(min(ql, rows - max(q0, 0)), 0) + tokb - 1) / tokb : 0;
+    if (n > 0) ksum += (float)n * (float)(window > 0 ? min(kv_lens[si], window) : kv_lens[si]);
+    tcum[si] = n;  // the count for now
+    tsum += n;
+  }
+  int x = tsum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  ksum = wave_sum(ksum);
+  if (lane == 63) {
+    wred[wv] = x;
+    wred[4 + wv] = __float_as_int(ksum);
+  }
+  __syncthreads();
+  int base = 0;
+  for (int w = 0; w < wv; ++w) base += wred[w];
+  ksum = __int_as_float(wred[4]) + __int_as_float(wred[5]) + __int_as_float(wred[6]) + __int_as_float(wred[7]);
+  int run = base + x - tsum;
+  for (int i = 0; i < ch; ++i) {
+    const int si = s0 + i;
+    if (si >= S) break;
+    const int n = tcum[si];
+    tcum[si] = run;
+    run += n;
+  }
+  if (tid == 255) tcum[S] = base + x;
+  __syncthreads();
+  TileItem r;
+  r.total = __builtin_amdgcn_readfirstlane(tcum[S]);
+  r.most = __builtin_amdgcn_readfirstlane(
+      min(grid_parts, Rule::most_parts(r.total * Hkv, ksum / (float)r.total)));
+  r.item = bid / Hkv / r.most;
+  r.part = bid / Hkv - r.item * r.most;
+  r.tile = -1;
+  if (r.item >= r.total) return r;
+  int s = 0;
+  for (int c = 0; c < S; c += 64) {
+    const int si = c + lane;
+    s += __builtin_popcountll(__ballot(si < S && tcum[si + 1] <= r.item));
+  }
+  s = __builtin_amdgcn_readfirstlane(s);
+  r.tile = __builtin_amdgcn_readfirstlane(tcum[s + 1] - 1 - r.item);
+  r.s = s;
+  r.q0 = __builtin_amdgcn_readfirstlane(qsl[s]);
+  r.qlen = __builtin_amdgcn_readfirstlane(qsl[s + 1]) - r.q0;
+  r.kv_len = __builtin_amdgcn_readfirstlane(kv_lens[s]);
+  return r;
 }
 
 // FP8: the same kernel over an FP8 cache, on the 64-key step geometry of BITS 4
@@ -155,60 +260,19 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int bid
   // ---- per-sequence tile counts, scanned by the whole workgroup (one pass of
   // global loads in parallel, not a serial walk by one thread)
   // LDS, carved from the shared arena
-  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oRawv = lds_next(oWred, 16);
+  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oRawv = lds_next(oWred, 32);
   constexpr int oRaws = lds_next(oRawv, RAWV), oKe = lds_next(oRaws, 2 * 4 * G * NT);
   constexpr int oVe = lds_next(oKe, 2 * NT * P::KSTR), oKsf = lds_next(oVe, 2 * D * P::VSTR);
   constexpr int oKbe = lds_next(oKsf, 4 * G * NT), oEnd = lds_next(oKbe, 16 * NT);
   static_assert(oEnd <= kArenaBytes, "LDS arena too small");
   int(&tcum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oTcum);
-  int(&wred)[4] = lds_at<int[4]>(oWred);
+  int(&wred)[8] = lds_at<int[8]>(oWred);
   const int kvh = bid % a.Hkv;
-  const int part = (bid / a.Hkv) % a.nparts;
-  const int item = bid / a.Hkv / a.nparts;
-  TileItem ti;
-  if (a.S <= 64) {
-    ti = tile_item64(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, item);
-    if (ti.tile < 0) return;
-  } else {
-    const int ch = (a.S + 255) / 256, s0 = tid * ch;
-    int tsum = 0;
-    for (int i = 0; i < ch; ++i) {
-      const int si = s0 + i;
-      if (si >= a.S) break;
-      const int nt = prefill_tiles(a, si, P::TOKB);
-      tcum[si] = nt;  // the count for now
-      tsum += nt;
-    }
-    int x = tsum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wred[tid >> 6] = x;
-    __syncthreads();
-    int base = 0;
-    for (int w = 0; w < (tid >> 6); ++w) base += wred[w];
-    int run = base + x - tsum;
-    for (int i = 0; i < ch; ++i) {
-      const int si = s0 + i;
-      if (si >= a.S) break;
-      const int n = tcum[si];
-      tcum[si] = run;
-      run += n;
-    }
-    if (tid == 255) tcum[a.S] = base + x;
-    __syncthreads();
-    if (item >= tcum[a.S]) return;
-    int s = 0;
-    while (tcum[s + 1] <= item) ++s;
-    s = __builtin_amdgcn_readfirstlane(s);
-    ti.tile = __builtin_amdgcn_readfirstlane(tcum[s + 1] - 1 - item);  // last tile first
-    ti.s = s;
-    ti.q0 = a.qsl[s];
-    ti.qlen = a.qsl[s + 1] - ti.q0;
-    ti.kv_len = a.kv_lens[s];
-  }
+  const TileItem ti =
+      a.S <= 64 ? tile_item64<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.nparts)
+                : tile_item_any<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.nparts,
+                                             tcum, wred);
+  if (ti.tile < 0) return;
   const int s = ti.s, tile = ti.tile, q0 = ti.q0, qlen = ti.qlen;
   const int kv_len = min(max(ti.kv_len, 0), a.max_blocks * a.bs);
   const int past = kv_len - qlen;  // query i sees keys [.., past + i]
@@ -232,10 +296,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int bid
   const int k_hi = min(past + t_last, kv_len - 1);
   const int k_lo = a.window > 0 ? max(0, past + t_first - a.window + 1) : 0;
   const int steps_all = k_hi >= 0 ? max(k_hi / NT - k_lo / NT + 1, 0) : 0;
-  // parts of this tile: the steps split evenly, at most nparts, about kPrefillSplitKeys keys each
-  const int nparts = a.nparts > 1 && item < a.max_items
-                         ? max(1, min(a.nparts, (steps_all * NT + kPrefillSplitKeys - 1) / kPrefillSplitKeys))
-                         : 1;
+  // parts of this tile: the steps split evenly
+  const int item = ti.item, part = ti.part, nparts = prefill_parts(steps_all * NT, ti.most);
   if (part >= nparts) return;
   const int step_lo = k_lo / NT + part * steps_all / nparts;
   const int step_hi = k_lo / NT + (part + 1) * steps_all / nparts - 1;
@@ -592,8 +654,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int bid
   if (nparts > 1) {
     const int u = item * a.Hkv + kvh;
     const __amdgpu_buffer_rsrc_t rp =
-        uniform_rsrc(reinterpret_cast<uint8_t*>(a.ws_part) + (size_t)u * kPrefillParts * kPrefillPartBytes,
-                     kPrefillParts * kPrefillPartBytes);
+        uniform_rsrc(reinterpret_cast<uint8_t*>(a.ws_part) + (size_t)u * ti.most * kPrefillPartBytes,
+                     ti.most * kPrefillPartBytes);
     auto vo = [&](int k) { return ((wv * kPrefillPartVec + k) * 64 + lane) * 16; };
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct)

@@ -43,6 +43,23 @@
 
 namespace emx {
 
+// As PrefillRule (prefill_affine.hpp): a third part only where all of three fit the 512 places of
+// the chip.  3 / 2 / 1 parts, bf16 pages of 16, us: 16 tiles (a 64-token chunk after 9000) 110 / 156 /
+// 292, 88 (330 tokens) 162 / 220 / 422, 256 (a 1000-token prompt) 38 / 39 / 57, 352 (2 x 700 beside
+// 60 rows) 137 / 133 / 154, 512 (four 512-token chunks) 132 / 119 / 126, (beside 64 rows) 166 / 168 /
+// 187, 656 (2 x 1300) 126 / 126 / 114, 752 (a 3000-token prompt) 167 / 163 / 168, 1024 (4 x 1000)
+// 116 / 111 / 111, (eight chunks after up to 8192) 647 / 643 / 796, 1504 217 / 214 / 192, 2048
+// 331 / 320 / 281; 4-bit pages of 16: 512 beside 28 rows 171 / 151 / 157, 1280 779 / 827 / 929.
+constexpr int kTiles3 = 170;
+static_assert(3 * kTiles3 <= 2 * kPrefillCutTiles, "the workspace holds either");
+struct MfmaRule {
+  static __host__ __device__ constexpr int most_parts(long tiles, float keys) {
+    return tiles <= kTiles3 ? 3
+           : tiles <= kPrefillFewTiles || (tiles <= kPrefillCutTiles && keys >= kPrefillLongKeys) ? 2
+                                                                                                   : 1;
+  }
+};
+
 struct PrefillMfmaArgs {
   DecodeArgs d;     // kc / vc: the caches; nt, ws_* unused
   uint32_t inv_bs;  // ceil(2^32 / bs)
@@ -50,9 +67,9 @@ struct PrefillMfmaArgs {
   int tokb;         // query tokens per tile: columns / HG
   int T;            // query rows
   int items;        // tiles per kv head the grid has room for
-  int nparts, max_items;
-  int* ws_cnt;      // [max_items * Hkv * 4], zero before and after every launch
-  float* ws_part;   // [max_items * Hkv][nparts][part bytes]
+  int nparts;       // most parts of a tile the grid has room for (1: no workspace for them)
+  int* ws_cnt;      // [tiles * Hkv * 4], zero before and after every launch
+  float* ws_part;   // [tiles * Hkv][parts][part bytes]
 };
 
 template <class C, int D, int CT>
@@ -150,13 +167,13 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     if constexpr (C::kAffine) return P::G;
     return 1;
   }();
-  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oKe = lds_next(oWred, 16);
+  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oKe = lds_next(oWred, 32);
   constexpr int oVe = lds_next(oKe, 2 * NT * P::KSTR), oKsf = lds_next(oVe, 2 * (AFF ? D : NT) * P::VSTR);
   constexpr int oVsf = lds_next(oKsf, 4 * G * NT), oVbf = lds_next(oVsf, 4 * G * NT);
   constexpr int oKbe = lds_next(oVbf, AFF ? 4 * G * NT : 0), oEnd = lds_next(oKbe, AFF ? 16 * NT : 0);
   static_assert(oEnd <= kArenaBytes, "LDS arena too small");
   int(&tcum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oTcum);
-  int(&wred)[4] = lds_at<int[4]>(oWred);
+  int(&wred)[8] = lds_at<int[8]>(oWred);
   uint16_t* ke = &lds_at<uint16_t>(oKe);  // [key][KSTR]
   uint16_t* ve = &lds_at<uint16_t>(oVe);  // [key][VSTR]; affine: [dim][VSTR]
   float* ksf = &lds_at<float>(oKsf);      // key scale of each key; affine: [group][NT], * 2^kCodeExp
@@ -164,69 +181,21 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   float* vbf = &lds_at<float>(oVbf);      // affine: value biases
   h16* kbe = &lds_at<h16>(oKbe);          // affine: bias operand rows, key bias of group g at 2 g, 2 g + 1
 
-  // ---- work item: tiles per sequence, scanned by the workgroup; the last tile (most keys) first
+  // ---- work item
   const int kvh = bid % a.Hkv;
-  const int item = bid / a.Hkv / A.nparts;
-  int part = (bid / a.Hkv) % A.nparts;
-  // workgroups go round the chip in turn, so that with two parts the uncut tiles, which use one
-  // of the two, would take every other place (half the chip idle: 512-token prompts 48.5 against
-  // 37.2 us at three parts): the part that works changes place every other tile
-  if (A.nparts == 2) part ^= (item >> 1) & 1;
-  TileItem ti;
-  if (a.S <= 64) {
-    ti = tile_item64(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, item, A.T);
-  } else {
-    const int ch = (a.S + 255) / 256, s0 = tid * ch;
-    int tsum = 0;
-    for (int i = 0; i < ch; ++i) {
-      const int si = s0 + i;
-      if (si >= a.S) break;
-      const int q0 = a.qsl[si], ql = a.qsl[si + 1] - q0;
-      const int n = ql >= A.min_q ? (max(min(ql, A.T - q0), 0) + A.tokb - 1) / A.tokb : 0;
-      tcum[si] = n;  // the count for now
-      tsum += n;
-    }
-    int x = tsum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wred[tid >> 6] = x;
-    __syncthreads();
-    int base = 0;
-    for (int w = 0; w < (tid >> 6); ++w) base += wred[w];
-    int run = base + x - tsum;
-    for (int i = 0; i < ch; ++i) {
-      const int si = s0 + i;
-      if (si >= a.S) break;
-      const int n = tcum[si];
-      tcum[si] = run;
-      run += n;
-    }
-    if (tid == 255) tcum[a.S] = base + x;
-    __syncthreads();
-    ti.total = __builtin_amdgcn_readfirstlane(tcum[a.S]);
-    ti.tile = -1;
-    if (item < ti.total) {
-      int s = 0;
-      for (int c = 0; c < a.S; c += 64) {
-        const int si = c + lane;
-        s += __builtin_popcountll(__ballot(si < a.S && tcum[si + 1] <= item));
-      }
-      s = __builtin_amdgcn_readfirstlane(s);
-      ti.tile = __builtin_amdgcn_readfirstlane(tcum[s + 1] - 1 - item);
-      ti.s = s;
-      ti.q0 = __builtin_amdgcn_readfirstlane(a.qsl[s]);
-      ti.qlen = __builtin_amdgcn_readfirstlane(a.qsl[s + 1]) - ti.q0;
-      ti.kv_len = __builtin_amdgcn_readfirstlane(a.kv_lens[s]);
-    }
-  }
+  TileItem ti = a.S <= 64 ? tile_item64<MfmaRule>(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, a.window, bid, a.Hkv,
+                                                  A.nparts, A.T)
+                          : tile_item_any<MfmaRule>(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, a.window, bid, a.Hkv,
+                                                    A.nparts, tcum, wred, A.T);
   if (ti.tile < 0) {
-    const int per = a.Hkv * A.nparts;
-    zero_other_rows<QT>(a, A.T, D, bid - ti.total * per, (A.items - ti.total) * per);
+    const int first = ti.total * a.Hkv * ti.most;
+    zero_other_rows<QT>(a, A.T, D, bid - first, A.items * a.Hkv * A.nparts - first);
     return;
   }
+  // workgroups go round the chip in turn, so that with two parts the uncut tiles, which use one
+  // of the two, would take every other place (half the chip idle: 512-token prompts 48.5 against
+  // 37.2 us): the part that works changes place every other tile
+  if (ti.most == 2) ti.part ^= (ti.item >> 1) & 1;
   const int s = ti.s, tile = ti.tile, q0 = ti.q0, qlen = ti.qlen;
   const int kv_len = min(max(ti.kv_len, 0), a.max_blocks * a.bs);
   const int past = kv_len - qlen;  // query i sees keys [.., past + i]
@@ -250,9 +219,7 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   const int k_hi = min(past + t_last, kv_len - 1);
   const int k_lo = a.window > 0 ? max(0, past + tok_lo - a.window + 1) : 0;
   const int steps_all = k_hi >= 0 ? max(k_hi / NT - k_lo / NT + 1, 0) : 0;
-  const int nparts = A.nparts > 1 && item < A.max_items
-                         ? max(1, min(A.nparts, (steps_all * NT + kPrefillSplitKeys - 1) / kPrefillSplitKeys))
-                         : 1;
+  const int item = ti.item, part = ti.part, nparts = prefill_parts(steps_all * NT, ti.most);
   if (part >= nparts) return;
   const int step_lo = k_lo / NT + part * steps_all / nparts;
   const int step_hi = k_lo / NT + (part + 1) * steps_all / nparts - 1;
@@ -651,8 +618,7 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
   if (nparts > 1) {
     const int u = item * a.Hkv + kvh;
     const __amdgpu_buffer_rsrc_t rp =
-        uniform_rsrc(reinterpret_cast<uint8_t*>(A.ws_part) + (size_t)u * A.nparts * P::PARTB,
-                     A.nparts * P::PARTB);
+        uniform_rsrc(reinterpret_cast<uint8_t*>(A.ws_part) + (size_t)u * ti.most * P::PARTB, ti.most * P::PARTB);
     constexpr int NV = CT * P::SB;
     auto vo = [&](int k) { return ((wv * (NV + 1) + k) * 64 + lane) * 16; };
 #pragma unroll

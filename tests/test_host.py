@@ -279,6 +279,35 @@ def test_abi_rope_and_prefill_split_arguments(lib):
     assert lib.emx_paged_prefill_workspace_bytes(10 ** 7, 32, 32, 8, 128) == 0  # counters would not fit
 
 
+def test_ragged_workspace_bytes(lib):
+    """Room for the parts of a ragged call's tiles: 0 where nothing can be cut, whatever rows stand beside the chunks."""
+    size = lib.emx_paged_ragged_workspace_bytes
+    for bad in ((0, 1, 32, 8, 128), (10, 0, 32, 8, 128), (10, 1, 32, 0, 128), (10, 1, 0, 8, 128), (10, 1, 30, 8, 128),
+                (10, 1, 32, 8, 96), (500, 1, 129, 1, 128), (500, 1, 65, 1, 256)):
+        assert size(*bad) == 0, bad
+    assert size(500, 1, 128, 1, 64) > 0 and size(500, 1, 64, 1, 256) > 0
+    assert size(8192, 1, 32, 8, 128) == 0  # 2048 tiles fill the GPU uncut
+    for d in (64, 128):  # four 512-token chunks are 512 tiles beside any number of single-token rows
+        for rows in (0, 28, 35, 96, 400):
+            assert size(4 * 512 + rows, 4 + rows, 32, 8, d) > 0, rows
+    # what the kernels index (tiles over all kv heads x their most parts x a part's state) fits, for any split of the
+    # rows into sequences; 64 ct query columns a tile, 4 (ct d / 16 + 1) KiB a part
+    rng = np.random.default_rng(3)
+    for _ in range(3000):
+        d, hkv = int(rng.choice([64, 128, 256])), int(rng.choice([1, 2, 3, 8, 16]))
+        ct = 1 if d == 256 else 2
+        hq = hkv * int(rng.integers(1, 64 * ct + 1))
+        qlens = rng.integers(0, rng.choice([2, 3, 40, 900]), size=int(rng.integers(1, 60)))
+        total = int(qlens.sum())
+        if total == 0:
+            continue
+        tokb = 64 * ct // (hq // hkv)
+        units = hkv * sum(-(-int(q) // tokb) for q in qlens if q >= 2)
+        parts = 3 if units <= 170 else 2 if units <= 1280 else 1
+        if parts > 1:
+            assert size(total, len(qlens), hq, hkv, d) >= units * parts * 4 * (ct * d // 16 + 1) * 1024, (qlens, hq, hkv, d)
+
+
 def test_workspace_of_a_capture_stays_apart(monkeypatch):
     """A buffer made under graph capture is cleared by replays only: eager calls and other captures never get it."""
     from easymlx_amd.operations import unified_attention as ua
