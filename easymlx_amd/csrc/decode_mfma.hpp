@@ -295,9 +295,13 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
 
   auto start_of = [&](int kl) { return a.window > 0 ? max(0, kl - a.window) : 0; };
   // An item: item j of the n of unit y of sequence s; this wave's tokens start at tb.
+  // (No bool: the compiler kept the bytes that pad it as arrays in LDS, whose index needs the workgroup's
+  // size from the dispatch packet in host memory, 7 us and more before the first product with all compute
+  // units at it: 25 contexts of 8 to 17 tokens, bf16, D 64, 19.1 -> 7.4 us; batch 32 over FP8 pages of 16
+  // 46 -> 34.)
   struct Item {
     int s, y, j, n, kl, st, tb;
-    bool has;  // inside the range
+    int has;  // inside the range
   };
   auto tb_of = [&](int st, int jx) { return (st / NT + jx) * NT + P::NTW * wv; };
   Item it0;

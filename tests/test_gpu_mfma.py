@@ -183,6 +183,33 @@ def test_decode_units_just_past_the_workgroups(cuda):
     assert took[65] < 1.5 * took[64] and took[66] < 1.5 * took[64], took
 
 
+def test_decode_short_contexts_side_by_side(cuda):
+    """200 workgroups with one short item each take about what 8 take: they share no slow memory (2.2 times as long
+    where each read the dispatch packet, in host memory; 1.5 times at most is asked for)."""
+    print("[decode 25 short rows]", flush=True)
+    took = {}
+    for seqs in (1, 25):
+        b = batch("bf16", [1] * seqs, [12] * seqs, 32, 8, 64, 16, seed=15)
+        check(b, run(b, cuda), expected(b))
+        q, k, v = b["q"].to(cuda), b["cache"][0].to(cuda), b["cache"][1].to(cuda)
+        args, out = [torch.from_numpy(b[n]).to(cuda) for n in ("tables", "kvl", "qsl")], torch.empty_like(q)
+        side, g = torch.cuda.Stream(cuda), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            for _ in range(40):  # (in a graph: the host takes longer than these kernels)
+                paged_attention(q, k, v, *args, single_token_decode=True, out=out)
+        took[seqs] = float("inf")
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            g.replay()
+            t1.record()
+            torch.cuda.synchronize()
+            took[seqs] = min(took[seqs], t0.elapsed_time(t1))
+        check(b, out.double().cpu().numpy(), expected(b))
+    assert took[25] < 1.5 * took[1], took
+
+
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_decode_infinities(cuda, kind):
     """An infinity or NaN outside the visible keys leaves a row as it is; a visible infinity stays one."""
