@@ -797,6 +797,8 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
           if (whole) {
             bad |= write4(O, L, out + (size_t)h * D + dim);
           } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) bad |= not_finite(O[k]);
             store_f32x4(O, ro, (h * D + dim) * 4, me * A.hc * D * 4);
             if (rd == 0 && c == 0)
               __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{M, L}), rm, h * 8, me * A.hc * 8,
@@ -804,7 +806,30 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
           }
         }
       }
-      bool done = whole;
+      // ---- rows that are not finite over this workgroup's keys: again in fp32 (attend_row)
+      if (__syncthreads_or(bad)) {
+        __builtin_amdgcn_s_waitcnt(0);  // every wave's stores above come first
+        __syncthreads();
+        const int b0 = start_k / NT - unit_first;  // item g of the unit: tokens from (b0 + g) NT
+        // (a piece's sums are of p = 2^(x - m + kPBias), as the others')
+        const int k0 = max(start_k, (b0 + seg0) * NT), k1 = min(kv_len, (b0 + g + 1) * NT);
+        for (int h = wv; h < nh; h += 4) {
+          float mr, lr, x[D / 64];
+          const QT* qp = reinterpret_cast<const QT*>(a.q) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0 + h) * D;
+          attend_row<C, D>(a, s, kvh, qp, k0, k1, mr, lr, x, lane);
+#pragma unroll
+          for (int i = 0; i < D / 64; ++i) {
+            if (whole)
+              from_f32(lr > 0.f ? x[i] / lr : 0.f, out + (size_t)h * D + lane + 64 * i);
+            else
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[i] * kPScale), ro, (h * D + lane + 64 * i) * 4,
+                                                    me * A.hc * D * 4, kCoherent);
+          }
+          if (!whole && lane == 0)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{mr, lr * kPScale}), rm, h * 8, me * A.hc * 8,
+                                                  kCoherent);
+        }
+      }
       if (!whole) {
         __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete before the workgroup is counted
         __syncthreads();
@@ -814,8 +839,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
           flag = old == np - 1;
         }
         __syncthreads();
-        done = flag != 0;
-        if (done) {
+        if (flag != 0) {
           // the workgroup counted last merges the pieces (page_attention.py:2006-2059):
           // NE float4 elements; with fewer than 256, groups of threads share the pieces
           const int NE = nh * (D / 4);
@@ -843,7 +867,11 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
                 }
 #pragma unroll
                 for (int k = 0; k < NB; ++k) {
-                  if (p0 + k * ng >= np || ml[k].x == -INFINITY) continue;
+                  if (p0 + k * ng >= np) continue;
+                  if (ml[k].x == -INFINITY) {  // no live key, or scores of NaN only
+                    L += ml[k].y;
+                    continue;
+                  }
                   const float Mn = fmaxf(M, ml[k].x);
                   const float fo = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
                   const float fp = __builtin_amdgcn_exp2f(ml[k].x - Mn);
@@ -865,7 +893,10 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
               if (act && grp == 0) {
                 for (int q = 1; q < ng; ++q) {
                   const float* x = xo + (q * NE + e) * 6;
-                  if (x[0] == -INFINITY) continue;
+                  if (x[0] == -INFINITY) {
+                    L += x[1];
+                    continue;
+                  }
                   const float Mn = fmaxf(M, x[0]);
                   const float fo = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
                   const float fp = __builtin_amdgcn_exp2f(x[0] - Mn);
@@ -876,20 +907,8 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
                 }
               }
             }
-            if (act && grp == 0) {
-              bad |= write4(O, L, out + 4 * e);
-            }
+            if (act && grp == 0) write4(O, L, out + 4 * e);
           }
-        }
-      }
-      // ---- a row that is not finite: again in fp32, key by key (attend_row)
-      if (__syncthreads_or(done && bad)) {
-        for (int h = wv; h < nh; h += 4) {
-          float lr, x[D / 64];
-          const QT* qp = reinterpret_cast<const QT*>(a.q) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0 + h) * D;
-          attend_row<C, D>(a, s, kvh, qp, start_k, kv_len, lr, x, lane);
-#pragma unroll
-          for (int i = 0; i < D / 64; ++i) from_f32(lr > 0.f ? x[i] / lr : 0.f, out + (size_t)h * D + lane + 64 * i);
         }
       }
       clear();

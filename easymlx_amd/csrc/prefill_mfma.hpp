@@ -679,7 +679,7 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
       }
       if (ok) *reinterpret_cast<Four*>(op + 16 * b + 4 * jj) = v;
     }
-    // columns that are not finite: again in fp32, key by key (attend_row)
+    // columns that are not finite: again in fp32 (attend_row)
     uint64_t todo = __ballot(bad && ok);
     todo = (todo | (todo >> 16) | (todo >> 32) | (todo >> 48)) & 0xFFFFu;
     while (todo) {
@@ -688,8 +688,8 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
       const int t = __builtin_amdgcn_readlane(ctok[ct], c), hh = __builtin_amdgcn_readlane(chead[ct], c);
       const int k0 = __builtin_amdgcn_readlane(start[ct], c), k1 = __builtin_amdgcn_readlane(limit[ct], c) + 1;
       const size_t ro = ((size_t)(q0 + t) * a.Hq + (size_t)kvh * HG + hh) * D;
-      float lr, x[D / 64];
-      attend_row<C, D>(a, s, kvh, reinterpret_cast<const QT*>(a.q) + ro, k0, k1, lr, x, lane);
+      float mr, lr, x[D / 64];
+      attend_row<C, D>(a, s, kvh, reinterpret_cast<const QT*>(a.q) + ro, k0, k1, mr, lr, x, lane);
       const float li = lr > 0.f ? 1.f / lr : 0.f;
 #pragma unroll
       for (int i = 0; i < D / 64; ++i) from_f32(x[i] * li, reinterpret_cast<QT*>(a.out) + ro + lane + 64 * i);

@@ -228,6 +228,54 @@ def test_decode_infinities(cuda, kind):
     check(b, got, exp)
 
 
+@pytest.mark.parametrize("kind,d,page", [("f16", 64, 16), ("bf16", 128, 8), ("f16", 256, 32), ("q4", 64, 16),
+                                          ("q8", 256, 64)])
+def test_decode_infinities_in_cut_rows(cuda, kind, d, page):
+    """Rows cut over many workgroups: an infinity stays one wherever it lies, a page of NaN keys gives zeros (the sum
+    of the probabilities is no number), the other rows and dims stay as they are; in about the time of finite rows."""
+    print(f"[decode infinities, cut rows {kind} d{d}]", flush=True)
+    kvl = [3000, 3000, 3000, 70]
+    b = batch(kind, [1] * 4, kvl, 4, 2, d, page, seed=18)
+    exp = expected(b)
+
+    def timed():
+        got, best = run(b, cuda), float("inf")
+        t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)  # noqa: E731
+        sc = b["scales"] or {}
+        kw = {n: x.to(cuda) if isinstance(x, torch.Tensor) else x for n, x in sc.items()}
+        args = [b["q"].to(cuda), b["cache"][0].to(cuda), b["cache"][1].to(cuda), t(b["tables"]), t(b["kvl"]), t(b["qsl"])]
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            for _ in range(10):
+                paged_attention(*args, single_token_decode=True, **kw)
+            t1.record()
+            torch.cuda.synchronize()
+            best = min(best, t0.elapsed_time(t1) * 100)
+        return got, best
+
+    finite, us = timed()
+    check(b, finite, exp)
+    at = lambda s, p: (int(b["tables"][s, p // page]), p % page)  # noqa: E731
+    dims = slice(9, 10)
+    if kind in ("q4", "q8"):
+        dims = slice(0, 64)
+        blk, off = at(0, 1500)
+        b["scales"]["v_biases"][blk, 1, 0, off] = float("inf")
+        blk, off = at(1, 0)
+        b["scales"]["v_biases"][blk, 1, 0, off] = float("inf")
+        b["scales"]["k_biases"][at(2, 1000)[0], 0, 0, :] = float("nan")
+    else:
+        b["cache"][1][at(0, 1500)][1, 9] = float("inf")
+        b["cache"][1][at(1, 0)][1, 9] = float("inf")
+        b["cache"][0][at(2, 1000)[0], :, 0, 3] = float("nan")
+    got, us2 = timed()
+    assert np.isposinf(got[:2, 2:, dims]).all() and (got[2, :2] == 0).all()
+    got[:2, 2:, dims], got[2, :2] = exp[:2, 2:, dims], exp[2, :2]
+    check(b, got, exp)
+    assert us2 < 8 * us + 50, (us, us2)
+
+
 # chunks around the tile and step edges, over cached prefixes, beside single-token and empty rows
 RAGGED = [(33, 40), (1, 129), (2, 2), (130, 700), (1, 1), (0, 5), (65, 65), (7, 3), (1, 600), (5, 0), (64, 1300)]
 
