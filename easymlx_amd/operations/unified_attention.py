@@ -17,6 +17,7 @@ silently, ``unified_attention.py:1499-1512``).
 
 from __future__ import annotations
 
+import functools
 import math
 import threading
 import typing as tp
@@ -138,18 +139,27 @@ def _workspace(device: torch.device, stream: int, nbytes: int, own: bool = False
         return ws
 
 
-def _call_workspace(lib, device: torch.device, stream: int, total: int, S: int, hq: int, hkv: int, d: int,
+@functools.lru_cache(maxsize=1024)
+def _workspace_bytes(S: int, hq: int, hkv: int, d: int, max_blocks: int, bs: int) -> int:
+    return int(_native.load().emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
+
+
+@functools.lru_cache(maxsize=1024)
+def _ragged_bytes(total: int, S: int, hq: int, hkv: int, d: int) -> int:
+    return int(_native.load().emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
+
+
+def _call_workspace(device: torch.device, stream: int, total: int, S: int, hq: int, hkv: int, d: int,
                     max_blocks: int, bs: int, decode: bool, dense: bool = False) -> torch.Tensor | None:
     """The stream's workspace for one call; for a ragged call with the room in which long tiles are cut into parts.
 
     A captured ragged call over unquantized caches takes a buffer of its capture: nothing is shared between a replay
     and the stream's own work.
     """
-    need = int(lib.emx_paged_workspace_bytes(S, hq, hkv, d, max_blocks, bs))
+    need = _workspace_bytes(S, hq, hkv, d, max_blocks, bs)
     if need == 0 or decode:
         return _workspace(device, stream, need)
-    need += int(lib.emx_paged_ragged_workspace_bytes(total, S, hq, hkv, d))
-    return _workspace(device, stream, need, own=dense)
+    return _workspace(device, stream, need + _ragged_bytes(total, S, hq, hkv, d), own=dense)
 
 
 def _i32(t, device) -> torch.Tensor:
@@ -240,7 +250,7 @@ def paged_attention(
             raise NotImplementedError("affine paged attention takes fp16 queries")
         nb, hkv, bs = int(key_cache.shape[0]), int(key_cache.shape[1]), int(key_cache.shape[2])
         if workspace is None:
-            workspace = _call_workspace(lib, dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode)
+            workspace = _call_workspace(dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode)
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
         tensors = [key_cache, value_cache, k_scales, k_biases, v_scales, v_biases]
@@ -273,7 +283,7 @@ def paged_attention(
         if k_scale.numel() != nb or v_scale.numel() != nb:
             raise ValueError("k_scale/v_scale must hold one scale per block: [num_blocks]")
         if workspace is None:
-            workspace = _call_workspace(lib, dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode)
+            workspace = _call_workspace(dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode)
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
         _native.check(
@@ -294,7 +304,7 @@ def paged_attention(
     value_cache = value_cache.contiguous()
     nb, bs, hkv = int(key_cache.shape[0]), int(key_cache.shape[1]), int(key_cache.shape[2])
     if workspace is None and (single_token_decode or queries.dtype != torch.float32):
-        workspace = _call_workspace(lib, dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode,
+        workspace = _call_workspace(dev, stream, total, S, hq, hkv, d, max_blocks, bs, single_token_decode,
                                     dense=True)
     ws_ptr = workspace.data_ptr() if workspace is not None else None
     ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
