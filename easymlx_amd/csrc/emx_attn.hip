@@ -407,10 +407,15 @@ int launch_generic_only(const emx::GenericArgs& ga, const KV& kv, hipStream_t st
 }
 
 // Turns rows [rows, heads, D] of queries or keys (rope_rows, or rope_rows_vec where the rows go
-// in 16-byte pieces: the same bits).
+// in 16-byte pieces and there are enough of them: the same bits).
+// The table and its barrier stand before the first store: fewer values than this are turned sooner
+// pair by pair, us by values, rope_rows / rope_rows_vec: 0.04M (9 tokens of 32 heads, D 128) 2.2 / 3.5,
+// 0.5M 2.7 / 3.6, 1.05M 3.5 / 3.8, 1.43M 4.2 / 3.9 (D 64) and 4.2 / 4.2 (8 heads, D 256), 2.1M
+// 5.3 / 4.3, 8.4M 15.3 / 6.8.
+constexpr long kRopeVecValues = 5L << 18;
 int launch_rope_rows(emx::h16* x, const emx::h16* src, int rows, int heads, int D, const emx::RopeArgs& r,
                      hipStream_t st) {
-  if (emx::turn_rows_vec_ok(D, r.rot, r.traditional) && r.rot / 2 <= emx::kRopeVecTab && aligned16(x) &&
+  if ((long)rows * heads * D >= kRopeVecValues && emx::turn_rows_vec_ok(D, r.rot, r.traditional) && r.rot / 2 <= emx::kRopeVecTab && aligned16(x) &&
       aligned16(src)) {
     // tokens per workgroup: two 16-byte pairs of pieces per thread, an angle table that fits
     const int per = heads * ((r.traditional ? r.rot / 8 : r.rot / 16) + (D - r.rot) / 8);

@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void rope_rows(h16* x, const h16* src, int row
 // takes `tt` tokens from b * tt, tabulates their (sin, cos) of every pair once for
 // all heads (rope_rows evaluates them per head and pair, which bounds it) and turns
 // the rows from the table (TurnRowsVec: the same bits).  2048 tokens of 32 heads, D
-// 128 (33.6 MB): 15.2 -> 7.6 us.  Needs turn_rows_vec_ok, 16-byte
+// 128 (33.6 MB): 15.3 -> 6.8 us.  Needs turn_rows_vec_ok, 16-byte
 // aligned rows and tt * rot / 2 <= kRopeVecTab.
 constexpr int kRopeVecTab = 1024;
 __global__ __launch_bounds__(256) void rope_rows_vec(h16* x, const h16* src, int rows, int heads, int D, RopeArgs r,
