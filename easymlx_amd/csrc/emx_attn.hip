@@ -112,14 +112,14 @@ size_t prefill_part_bytes(int num_tokens, int num_seqs, int num_q_heads, int num
 void prefill_split(emx::PrefillArgs& p, int num_tokens, int num_q_heads, int num_kv_heads, void* workspace,
                    size_t workspace_bytes, size_t need) {
   const int tokb = 128 / (num_q_heads / num_kv_heads);
-  p.nparts = 1;
+  p.places = 1;
   p.items = (num_tokens + tokb - 1) / tokb + p.S;  // a sequence has at most its tokens / tokb + 1
   p.ws_cnt = nullptr;
   p.ws_part = nullptr;
   const size_t extra = prefill_part_bytes(num_tokens, p.S, num_q_heads, num_kv_heads, 128);
   if (extra == 0 || workspace == nullptr || workspace_bytes < need + extra) return;
   const size_t base = (need + 255) & ~(size_t)255;
-  p.nparts = emx::PrefillRule::most_parts(prefill_min_items(num_tokens, p.S, tokb) * num_kv_heads, INFINITY);
+  p.places = emx::prefill_places(prefill_min_items(num_tokens, p.S, tokb) * num_kv_heads);
   p.ws_cnt = reinterpret_cast<int*>(workspace) + kPrefillCounterOff;
   p.ws_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + base);
 }
@@ -1191,7 +1191,7 @@ int emx_paged_attention_affine(const void* queries, int num_tokens, int num_q_he
       PrefillFn pf = bits == 4 ? pick_prefill_gs<4>(group_size, hg) : pick_prefill_gs<8>(group_size, hg);
       if (!pf)
         return fail(EMX_ERR_UNSUPPORTED, "no prefill kernel for bits=%d group_size=%d gqa=%d", bits, group_size, hg);
-      pgrid = (long)p.items * num_kv_heads * p.nparts;
+      pgrid = (long)p.items * num_kv_heads * p.places;
       // prefill and decode rows go out as one launch (below) when a unified kernel
       // pairs this prefill with the decode kernel picked for the rows
       const bool q4u = bits == 4 && (page_size & (page_size - 1)) == 0 && pick_decode_q4(group_size, hg, page_size);
@@ -1639,7 +1639,7 @@ int emx_paged_attention_fp8(const void* queries, int num_tokens, int num_q_heads
     prefill_split(p, num_tokens, num_q_heads, num_kv_heads, workspace, workspace_bytes, need);
     return p;
   };
-  auto prefill_grid = [&](const emx::PrefillArgs& p) { return (long)p.items * num_kv_heads * p.nparts; };
+  auto prefill_grid = [&](const emx::PrefillArgs& p) { return (long)p.items * num_kv_heads * p.places; };
   auto launch_prefill = [&](int min_q) {
     const emx::PrefillArgs p = prefill_args(min_q);
     hipLaunchKernelGGL(pf, dim3((unsigned)prefill_grid(p)), dim3(256), 0, st, p);

@@ -164,7 +164,7 @@ void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_
   const long items = tile_items(c.T, c.S, p.tokb, p.min_q);
   p.T = c.T;
   p.items = (int)items;
-  p.nparts = part ? MfmaRule::most_parts(tile_items_least(c.T, c.S, p.tokb) * c.Hkv, INFINITY) : 1;
+  p.places = part ? prefill_places(tile_items_least(c.T, c.S, p.tokb) * c.Hkv) : 1;
   p.ws_cnt = ws_part_cnt;
   p.ws_part = part;
   // Decode workgroups by the decode rows' share of the step (at most S of the T rows), so that
@@ -173,7 +173,7 @@ void launch_mixed_mfma(const MfmaCall& c, int* ws_cnt, float* partials, int* ws_
   // 12 / 20 / 35 / 50, 8-bit pages (20 rows beside two chunks) 74 / 41 / 38 at 5 / 20 / 35.
   const double share = 45.0 * c.S / std::max(1, c.T - c.S) * c.Hkv / c.Hq;
   const int ndec = ws_cnt ? std::clamp((int)(1024.0 * share), 64, kDecodeMfmaWGs) & ~7 : 0;
-  hipLaunchKernelGGL(mixed_fn(c), dim3((unsigned)(items * c.Hkv * p.nparts + ndec)), dim3(256), 0, st, p, d, ndec);
+  hipLaunchKernelGGL(mixed_fn(c), dim3((unsigned)(items * c.Hkv * p.places + ndec)), dim3(256), 0, st, p, d, ndec);
 }
 
 }  // namespace emx

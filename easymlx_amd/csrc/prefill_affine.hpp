@@ -54,10 +54,11 @@ struct PrefillArgs {
   const uint8_t* v8;
   const float* kps;             // [nb]
   const float* vps;             // [nb]
-  // Key split: a tile with many key steps is cut into up to nparts parts (one
+  // Key split: a tile with many key steps is cut into parts (PrefillRule; one
   // workgroup each); every wave stores its part's state and the last of a
-  // wave's parts merges them.  nparts = 1: no split (ws_* unused).
-  int nparts;
+  // wave's parts merges them.  places: workgroups the grid has for a tile
+  // (prefill_places; 1: no split, ws_* unused).
+  int places;
   int items;                    // tiles per kv head the grid has room for
   int* ws_cnt;                  // [tiles * 4] arrival counters: zero before and after every launch
   float* ws_part;               // [tiles][parts][kPrefillPartBytes]
@@ -87,6 +88,8 @@ struct PrefillRule {
     return tiles <= kPrefillFewTiles ? kPrefillParts : tiles <= kPrefillCutTiles && keys >= kPrefillLongKeys ? 2 : 1;
   }
 };
+// Workgroups a grid has for a tile, in a launch of `tiles` at least that may cut them.
+__host__ inline int prefill_places(long tiles) { return tiles <= kPrefillFewTiles ? kPrefillParts : 2; }
 // Most (tile, part) pairs of a launch.
 constexpr int kPrefillCutSlots =
     kPrefillParts * kPrefillFewTiles > 2 * kPrefillCutTiles ? kPrefillParts * kPrefillFewTiles : 2 * kPrefillCutTiles;
@@ -122,8 +125,11 @@ struct PrefillCfg {
 __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >> 2) + 4 * (k >> 4) + (k & 3); }
 
 // The query tile and part of workgroup `bid` of a launch over at most 64 sequences (kv head fastest, then
-// the part of as many as the rule allows, then the tile): its sequence, the tile within it (the last, with
-// most keys, first), the sequence's lengths and the launch's tiles; tile < 0: no such tile.  Every
+// the part, then the tile): its sequence, the tile within it (the last, with most keys, first), the
+// sequence's lengths and the launch's tiles; tile < 0: no such tile.  A launch of few tiles that cuts has
+// three places for a tile also where the rule allows two parts: workgroups go round the chip in turn, and
+// tiles that use one place of two would leave every other compute unit idle (bf16, GQA 7, four 514-token
+// prompts 44 us against 62, four 230-token ones 23 against 25).  Every
 // wave finds it alone, a sequence to a lane: one trip to memory and a scan in registers, where the
 // workgroup's scan through LDS (any number of sequences) has two trips and two barriers before
 // the first query is read.  4-bit pages of 128, four 512-token chunks beside 28 rows 87.1 -> 85.0
@@ -132,12 +138,12 @@ __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >
 // last one are not counted.
 struct TileItem {
   int tile, s, q0, qlen, kv_len;
-  int item, part, most;  // most: parts a tile of this launch may have
+  int item, part, most, places;  // most: parts a tile of this launch may have
   int total;
 };
 template <class Rule>
 __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
-                                                int window, int bid, int Hkv, int grid_parts, int rows = INT32_MAX) {
+                                                int window, int bid, int Hkv, int grid_places, int rows = INT32_MAX) {
   const int lane = threadIdx.x & 63, si = min(lane, S - 1);
   const int q0 = qsl[si], ql = qsl[si + 1] - q0, kv = kv_lens[si];
   const int n = lane < S && ql >= min_q ? (max(min(ql, rows - max(q0, 0)), 0) + tokb - 1) / tokb : 0;
@@ -151,15 +157,16 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
   TileItem r;
   r.total = __builtin_amdgcn_readlane(x, 63);
   r.most = 1;
-  if (grid_parts > 1) {
+  if (grid_places > 1) {
     const int tiles = r.total * Hkv;
     float keys = 0.f;
     if (tiles > kPrefillFewTiles && tiles <= kPrefillCutTiles)  // (the sum is worth 0.5 us)
       keys = wave_sum((float)n * (float)(window > 0 ? min(kv, window) : kv)) / (float)r.total;
-    r.most = __builtin_amdgcn_readfirstlane(min(grid_parts, Rule::most_parts(tiles, keys)));
+    r.most = __builtin_amdgcn_readfirstlane(Rule::most_parts(tiles, keys));
   }
-  r.item = bid / Hkv / r.most;
-  r.part = bid / Hkv - r.item * r.most;
+  r.places = r.most > 1 ? grid_places : 1;
+  r.item = bid / Hkv / r.places;
+  r.part = bid / Hkv - r.item * r.places;
   const int s = __builtin_popcountll(__ballot(x <= r.item));
   r.tile = -1;
   if (s > 63) return r;
@@ -174,7 +181,7 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
 // The same for any number of sequences, scanned by the workgroup: tcum [S + 1] and wred [8] in LDS.
 template <class Rule>
 __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
-                                                  int window, int bid, int Hkv, int grid_parts, int* tcum, int* wred,
+                                                  int window, int bid, int Hkv, int grid_places, int* tcum, int* wred,
                                                   int rows = INT32_MAX) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int ch = (S + 255) / 256, s0 = tid * ch;
@@ -216,10 +223,10 @@ __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int3
   __syncthreads();
   TileItem r;
   r.total = __builtin_amdgcn_readfirstlane(tcum[S]);
-  r.most = __builtin_amdgcn_readfirstlane(
-      min(grid_parts, Rule::most_parts(r.total * Hkv, ksum / (float)r.total)));
-  r.item = bid / Hkv / r.most;
-  r.part = bid / Hkv - r.item * r.most;
+  r.most = grid_places > 1 ? __builtin_amdgcn_readfirstlane(Rule::most_parts(r.total * Hkv, ksum / (float)r.total)) : 1;
+  r.places = r.most > 1 ? grid_places : 1;
+  r.item = bid / Hkv / r.places;
+  r.part = bid / Hkv - r.item * r.places;
   r.tile = -1;
   if (r.item >= r.total) return r;
   int s = 0;
@@ -269,8 +276,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int bid
   int(&wred)[8] = lds_at<int[8]>(oWred);
   const int kvh = bid % a.Hkv;
   const TileItem ti =
-      a.S <= 64 ? tile_item64<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.nparts)
-                : tile_item_any<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.nparts,
+      a.S <= 64 ? tile_item64<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.places)
+                : tile_item_any<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.places,
                                              tcum, wred);
   if (ti.tile < 0) return;
   const int s = ti.s, tile = ti.tile, q0 = ti.q0, qlen = ti.qlen;

@@ -67,7 +67,7 @@ struct PrefillMfmaArgs {
   int tokb;         // query tokens per tile: columns / HG
   int T;            // query rows
   int items;        // tiles per kv head the grid has room for
-  int nparts;       // most parts of a tile the grid has room for (1: no workspace for them)
+  int places;       // workgroups the grid has for a tile (prefill_places), 1: no workspace for parts
   int* ws_cnt;      // [tiles * Hkv * 4], zero before and after every launch
   float* ws_part;   // [tiles * Hkv][parts][part bytes]
 };
@@ -183,19 +183,15 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
 
   // ---- work item
   const int kvh = bid % a.Hkv;
-  TileItem ti = a.S <= 64 ? tile_item64<MfmaRule>(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, a.window, bid, a.Hkv,
-                                                  A.nparts, A.T)
+  const TileItem ti = a.S <= 64 ? tile_item64<MfmaRule>(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, a.window, bid, a.Hkv,
+                                                  A.places, A.T)
                           : tile_item_any<MfmaRule>(a.qsl, a.kv_lens, a.S, A.min_q, A.tokb, a.window, bid, a.Hkv,
-                                                    A.nparts, tcum, wred, A.T);
+                                                    A.places, tcum, wred, A.T);
   if (ti.tile < 0) {
-    const int first = ti.total * a.Hkv * ti.most;
-    zero_other_rows<QT>(a, A.T, D, bid - first, A.items * a.Hkv * A.nparts - first);
+    const int first = ti.total * a.Hkv * ti.places;
+    zero_other_rows<QT>(a, A.T, D, bid - first, A.items * a.Hkv * A.places - first);
     return;
   }
-  // workgroups go round the chip in turn, so that with two parts the uncut tiles, which use one
-  // of the two, would take every other place (half the chip idle: 512-token prompts 48.5 against
-  // 37.2 us): the part that works changes place every other tile
-  if (ti.most == 2) ti.part ^= (ti.item >> 1) & 1;
   const int s = ti.s, tile = ti.tile, q0 = ti.q0, qlen = ti.qlen;
   const int kv_len = min(max(ti.kv_len, 0), a.max_blocks * a.bs);
   const int past = kv_len - qlen;  // query i sees keys [.., past + i]
