@@ -84,6 +84,7 @@ constexpr int kPrefillCounters = 65536;   // arrival counters, four a cut tile
 constexpr int kPrefillFewTiles = 640, kPrefillCutTiles = 1280;
 constexpr float kPrefillLongKeys = 2560.f;
 struct PrefillRule {
+  static constexpr int kFew = kPrefillFewTiles;  // up to as many, contexts make no difference
   static __host__ __device__ constexpr int most_parts(long tiles, float keys) {
     return tiles <= kPrefillFewTiles ? kPrefillParts : tiles <= kPrefillCutTiles && keys >= kPrefillLongKeys ? 2 : 1;
   }
@@ -126,20 +127,32 @@ __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >
 
 // The query tile and part of workgroup `bid` of a launch over at most 64 sequences (kv head fastest, then
 // the part, then the tile): its sequence, the tile within it (the last, with most keys, first), the
-// sequence's lengths and the launch's tiles; tile < 0: no such tile.  A launch of few tiles that cuts has
-// three places for a tile also where the rule allows two parts: workgroups go round the chip in turn, and
-// tiles that use one place of two would leave every other compute unit idle (bf16, GQA 7, four 514-token
-// prompts 44 us against 62, four 230-token ones 23 against 25).  Every
+// sequence's lengths and the launch's tiles; tile < 0: no such tile (set_places has the places).  Every
 // wave finds it alone, a sequence to a lane: one trip to memory and a scan in registers, where the
 // workgroup's scan through LDS (any number of sequences) has two trips and two barriers before
 // the first query is read.  4-bit pages of 128, four 512-token chunks beside 28 rows 87.1 -> 85.0
 // us, without a prefix 48.4 -> 45.7; sixteen 256-token chunks 57.7 -> 55.7; prefill_mfma, two
 // 700-token chunks at head_dim 64 26.7 -> 24.0.  `rows`: query rows of the call; tiles past the
 // last one are not counted.
+// Places: where most tiles are cut, as many as their parts; else three also for two parts.  Workgroups go
+// round the chip in turn, and tiles that use one place of two leave every other compute unit idle, although
+// the part that works changes place every other tile (bf16, GQA 7, four 514-token prompts 62 us, at three
+// places 44; four 230-token ones 25 / 23; 4-bit pages of 16, five 512-token chunks after up to 3000 tokens
+// 250 / 290).
 struct TileItem {
   int tile, s, q0, qlen, kv_len;
   int item, part, most, places;  // most: parts a tile of this launch may have
   int total;
+
+  template <class Rule>
+  __device__ __forceinline__ void set_places(int tiles, float keys, int bid, int Hkv, int grid_places) {
+    most = grid_places > 1 ? __builtin_amdgcn_readfirstlane(Rule::most_parts(tiles, keys)) : 1;
+    const bool mostly_cut = __builtin_amdgcn_readfirstlane(keys >= 2.f * kPrefillSplitKeys);
+    places = most == 1 ? 1 : most == 2 && mostly_cut ? 2 : grid_places;
+    item = bid / Hkv / places;
+    part = bid / Hkv - item * places;
+    if (places == 2) part ^= (item >> 1) & 1;
+  }
 };
 template <class Rule>
 __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
@@ -156,17 +169,13 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
   x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
   TileItem r;
   r.total = __builtin_amdgcn_readlane(x, 63);
-  r.most = 1;
-  if (grid_places > 1) {
-    const int tiles = r.total * Hkv;
-    float keys = 0.f;
-    if (tiles > kPrefillFewTiles && tiles <= kPrefillCutTiles)  // (the sum is worth 0.5 us)
-      keys = wave_sum((float)n * (float)(window > 0 ? min(kv, window) : kv)) / (float)r.total;
-    r.most = __builtin_amdgcn_readfirstlane(Rule::most_parts(tiles, keys));
-  }
-  r.places = r.most > 1 ? grid_places : 1;
-  r.item = bid / Hkv / r.places;
-  r.part = bid / Hkv - r.item * r.places;
+  const int tiles = r.total * Hkv;
+  float keys = 0.f;
+  // (the sum is worth 0.5 us; a window below every line needs none)
+  if (grid_places > 1 && tiles > Rule::kFew && tiles <= kPrefillCutTiles &&
+      (window <= 0 || window >= 2 * kPrefillSplitKeys))
+    keys = wave_sum((float)n * (float)(window > 0 ? min(kv, window) : kv)) / (float)r.total;
+  r.set_places<Rule>(tiles, keys, bid, Hkv, grid_places);
   const int s = __builtin_popcountll(__ballot(x <= r.item));
   r.tile = -1;
   if (s > 63) return r;
@@ -223,10 +232,7 @@ __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int3
   __syncthreads();
   TileItem r;
   r.total = __builtin_amdgcn_readfirstlane(tcum[S]);
-  r.most = grid_places > 1 ? __builtin_amdgcn_readfirstlane(Rule::most_parts(r.total * Hkv, ksum / (float)r.total)) : 1;
-  r.places = r.most > 1 ? grid_places : 1;
-  r.item = bid / Hkv / r.places;
-  r.part = bid / Hkv - r.item * r.places;
+  r.set_places<Rule>(r.total * Hkv, ksum / (float)r.total, bid, Hkv, grid_places);
   r.tile = -1;
   if (r.item >= r.total) return r;
   int s = 0;

@@ -26,7 +26,7 @@
 // entering the probability before it is split and sum p * v_bias kept in fp32 (the 128-wide
 // prefill_affine rounds scale * code + bias to fp16 instead).  Keys sit in LDS in the order
 // in which a lane's scores are then eight consecutive keys, those of its value operand.
-// Tiles of many keys are cut into up to nparts parts (the launcher's tile_parts), merged in
+// Tiles of many keys are cut into parts (MfmaRule), merged in
 // part order by the wave that arrives last (as in prefill_affine.hpp).
 //
 // Bound by the matrix and vector units together (the probability parts double the PV
@@ -53,6 +53,7 @@ namespace emx {
 constexpr int kTiles3 = 170;
 static_assert(3 * kTiles3 <= 2 * kPrefillCutTiles, "the workspace holds either");
 struct MfmaRule {
+  static constexpr int kFew = kTiles3;
   static __host__ __device__ constexpr int most_parts(long tiles, float keys) {
     return tiles <= kTiles3 ? 3
            : tiles <= kPrefillFewTiles || (tiles <= kPrefillCutTiles && keys >= kPrefillLongKeys) ? 2
