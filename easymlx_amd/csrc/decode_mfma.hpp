@@ -228,15 +228,30 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   }
   // (the host keeps the number of items below 2^31)
   const int I = Hu * uru(cum[S]);
-  const int NW = min(nblocks, I);
-  if (bid >= NW) return;
+  auto start_of = [&](int kl) { return a.window > 0 ? max(0, kl - a.window) : 0; };
+  // The most items a unit has.  Solo: no unit's keys reach past one wave's tokens, and each takes units of
+  // its own (a unit to a workgroup, with its three idle waves, the combine and the barriers, 3 to 10 us each:
+  // 200 contexts of 3 to 16 tokens, 16 heads: bf16, D 64 27 -> 13 us, D 256 78 -> 41; 4-bit, D 256 135 -> 48).
+  int nmax = 0;
+  bool solo = true;
+  for (int c = 0; c < S; c += 64) {
+    const int si = c + lane;
+    const int n = si < S ? cum[si + 1] - cum[si] : 0;
+    nmax = max(nmax, n);
+    if (n > 0) solo = solo && (kvl[si] - 1) / P::NTW == start_of(kvl[si]) / P::NTW;
+  }
+  nmax = uru((int)wave_max((float)nmax));
+  solo = __all(solo);
+  const int NW = min(solo ? 4 * nblocks : nblocks, I);
+  const int worker = solo ? wv * nblocks + bid : bid;  // (solo: no barrier from here on)
+  if (worker >= NW) return;
   const int per = (unsigned)I / (unsigned)NW, extra = I - per * NW;  // the first `extra` ranges hold one item more
   auto first_of = [&](int w) { return w * per + min(w, extra); };
   auto wg_of = [&](int g) {  // the workgroup whose range holds item g
     const int big = extra * (per + 1);
     return g < big ? (int)((unsigned)g / (unsigned)(per + 1)) : extra + (int)((unsigned)(g - big) / (unsigned)per);
   };
-  // The sequence of item g; the most items a unit has.
+  // The sequence of item g.
   auto seq_of = [&](const int g) {
     int s = 0;
     for (int c = 0; c < S; c += 64) {
@@ -245,12 +260,6 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     }
     return uru(s);
   };
-  int nmax = 0;
-  for (int c = 0; c < S; c += 64) {
-    const int si = c + lane;
-    nmax = max(nmax, si < S ? cum[si + 1] - cum[si] : 0);
-  }
-  nmax = uru((int)wave_max((float)nmax));
   bool cut = nmax > per + kDecodeMfmaMergeItems;  // (some range holds the longest unit)
   if (!cut && nmax > kDecodeMfmaMergeItems) {     // (no range exceeds per + nmax)
     // the longest range of whole units: those whose first item lies in an equal share
@@ -280,7 +289,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     cut = max(max(red[0], red[1]), max(red[2], red[3])) > per + kDecodeMfmaMergeItems;
     cut = uru(cut);
   }
-  int g0 = first_of(bid), g1 = first_of(bid + 1);
+  int g0 = first_of(worker), g1 = first_of(worker + 1);
   if (!cut) {  // whole units: those whose first item lies in the range
     auto unit_ceil = [&](const int g) {
       if (g >= I) return I;
@@ -293,7 +302,6 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     if (g0 >= g1) return;
   }
 
-  auto start_of = [&](int kl) { return a.window > 0 ? max(0, kl - a.window) : 0; };
   // An item: item j of the n of unit y of sequence s; this wave's tokens start at tb.
   // (No bool: the compiler kept the bytes that pad it as arrays in LDS, whose index needs the workgroup's
   // size from the dispatch packet in host memory, 7 us and more before the first product with all compute
@@ -303,7 +311,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
     int s, y, j, n, kl, st, tb;
     int has;  // inside the range
   };
-  auto tb_of = [&](int st, int jx) { return (st / NT + jx) * NT + P::NTW * wv; };
+  auto tb_of = [&](int st, int jx) { return solo ? st / P::NTW * P::NTW : (st / NT + jx) * NT + P::NTW * wv; };
   Item it0;
   {
     it0.s = seq_of(g0);
@@ -749,10 +757,26 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       }
       bool bad = false;
       QT* out = reinterpret_cast<QT*>(a.out) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0) * D;
+      if (solo) {  // this wave has the whole unit: its lanes write what they hold
+        if (col < nh) {
+          QT* o = out + (size_t)col * D;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int b = 0; b < P::SB; b += 4) {
+              if constexpr (C::kAffine)
+                bad |= write4(acc[b + r], l, o + 16 * (b + r) + 4 * jj);
+              else
+                bad |= write4(f32x4{acc[b][r], acc[b + 1][r], acc[b + 2][r], acc[b + 3][r]}, l,
+                              o + (4 * jj + r) * P::SB + b);
+            }
+        }
+      }
       const __amdgpu_buffer_rsrc_t ro =
           uniform_rsrc(a.ws_o + (size_t)slot * (A.hc * D), whole ? 0 : np * A.hc * D * 4);
       const __amdgpu_buffer_rsrc_t rm = uniform_rsrc(a.ws_ml + (size_t)slot * (A.hc * 2), whole ? 0 : np * A.hc * 8);
       const int me = whole ? 0 : uru(bid + u - slot);
+      if (!solo) {
 #pragma unroll
       for (int rd = 0; rd < D / P::RD; ++rd) {
         __syncthreads();  // (the previous combine has been read)
@@ -806,14 +830,16 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
           }
         }
       }
+      }
       // ---- rows that are not finite over this workgroup's keys: again in fp32 (attend_row)
-      if (__syncthreads_or(bad)) {
+      const bool again = solo ? __any(bad) : __syncthreads_or(bad);
+      if (again) {
         __builtin_amdgcn_s_waitcnt(0);  // every wave's stores above come first
-        __syncthreads();
+        if (!solo) __syncthreads();
         const int b0 = start_k / NT - unit_first;  // item g of the unit: tokens from (b0 + g) NT
         // (a piece's sums are of p = 2^(x - m + kPBias), as the others')
         const int k0 = max(start_k, (b0 + seg0) * NT), k1 = min(kv_len, (b0 + g + 1) * NT);
-        for (int h = wv; h < nh; h += 4) {
+        for (int h = solo ? 0 : wv; h < nh; h += solo ? 1 : 4) {
           float mr, lr, x[D / 64];
           const QT* qp = reinterpret_cast<const QT*>(a.q) + ((size_t)qrw[s] * a.Hq + (size_t)kvh * HG + h0 + h) * D;
           attend_row<C, D>(a, s, kvh, qp, k0, k1, mr, lr, x, lane);

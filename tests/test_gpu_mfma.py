@@ -276,6 +276,30 @@ def test_decode_infinities_in_cut_rows(cuda, kind, d, page):
     assert us2 < 8 * us + 50, (us, us2)
 
 
+@pytest.mark.parametrize("kind", ["f16", "bf16", "fp8", "q4", "q8"])
+@pytest.mark.parametrize("d,page,hq,hkv", [(64, 16, 14, 2), (128, 24, 6, 2), (128, 8, 40, 2), (256, 64, 4, 4)])
+@pytest.mark.parametrize("longest", [32, 33, 64, 65])
+def test_decode_contexts_of_one_wave(cuda, kind, d, page, hq, hkv, longest):
+    """Contexts that one wave's tokens hold (32; 64 over 4-bit pages) go a unit to a wave; one longer, none does."""
+    if kind in ("q4", "q8") and page in (8, 24):
+        page = 16
+    print(f"[decode one wave {kind} d{d} page{page} {hq}/{hkv} up to {longest}]", flush=True)
+    kvl = [longest] + [int(x) for x in np.random.default_rng(longest).integers(0, 33, size=150)]
+    b = batch(kind, [1] * len(kvl), kvl, hq, hkv, d, page, seed=d + longest, invalid=[(3, 0), (9, 1)] if page < 32 else [])
+    for window in (0, 7):
+        check(b, run(b, cuda, window), expected(b, window))
+    if kind in ("f16", "bf16"):
+        s = max(range(1, len(kvl)), key=lambda i: kvl[i] % page and kvl[i])
+        exp, blk = expected(b), int(b["tables"][s, (kvl[s] - 1) // page])
+        b["cache"][1][blk, (kvl[s] - 1) % page, 0, 5] = float("inf")
+        if kvl[s] % page:
+            b["cache"][0][blk, kvl[s] % page:] = float("nan")  # stale
+        got, hg = run(b, cuda), hq // hkv
+        assert np.isposinf(got[s, :hg, 5]).all()
+        got[s, :hg, 5] = exp[s, :hg, 5]
+        check(b, got, exp)
+
+
 # chunks around the tile and step edges, over cached prefixes, beside single-token and empty rows
 RAGGED = [(33, 40), (1, 129), (2, 2), (130, 700), (1, 1), (0, 5), (65, 65), (7, 3), (1, 600), (5, 0), (64, 1300)]
 
