@@ -31,9 +31,11 @@
 //
 // Bound by HBM.  Against decode_split and its merge (VALU dot products, single-element
 // loads, two launches), which ran these shapes before: batch 32, contexts of 512 to
-// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 71.3 us, FP8 (136 MB)
-// 330 -> 44 us; one context of 1024, D 64, fp16: 38.4 -> 14.2 us; 8-bit pages, D 256, 13
-// contexts of 200 to 5000 (64 MB): 141 -> 40 us.
+// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 66 us, FP8 (136 MB)
+// 330 -> 34 us; one context of 1024, D 64, fp16: 38.4 -> 11.2 us; 8-bit pages, D 256, 13
+// contexts of 200 to 5000 (64 MB): 141 -> 30 us.  Slower than they: more than 1024 units of a few
+// tokens at D 256 (96 contexts of 3 to 16, 16 heads: bf16 19.5 / 23.9, 4-bit 22.1 / 26.6 us), 4-bit D 256
+// without GQA at 60 to 128 tokens (200 contexts of 16 heads 115 / 135).
 #pragma once
 
 #include "mfma_common.hpp"

@@ -1691,8 +1691,9 @@ int emx_paged_attention_fp8(const void* queries, int num_tokens, int num_q_heads
     hipLaunchKernelGGL(dfn, dim3((unsigned)(nw / 4)), dim3(256), 0, st, a);
     return check_launch("decode_fp8_d128");
   }
-  // (over these pages they beat the kernels below: batch 32 of 512 .. 4096 45.7 against 55.5 us,
-  // the 512-token chunks beside 28 decode rows 91 against 102 us)
+  // (over these pages decode_fp8_d128 and unified_fp8 mostly beat decode_mfma and mixed_mfma below: 8
+  // contexts of 32768 113 against 123 us, the 512-token chunks beside 28 decode rows 87 against 93, a
+  // 1000-token prompt 35 against 36; batch 32 of 512 .. 4096 is the other way, 44 against 41)
   // other GQA ratios: the MFMA prefill kernel over every row (a decode row is a
   // tile of one query token)
   if (pf && query_start_loc) return launch_prefill(1);

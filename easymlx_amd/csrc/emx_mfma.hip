@@ -1,4 +1,4 @@
-// MFMA attention kernels over token-major caches and their launchers.
+// MFMA attention kernels over any cache (token-major and affine pages) and their launchers.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

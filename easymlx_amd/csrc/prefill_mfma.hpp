@@ -696,9 +696,10 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
 
 // Workgroups [0, ndec) decode the single-token rows (decode_mfma.hpp), the rest take the
 // query tiles: as unified.hpp does, the page streams run beside the matrix work.
+// (Two workgroups per compute unit; at D 256, where the decode body alone takes 250 registers and
+// more, the bound spills 7 to 117 of them, at D 128 over 4-bit group 64 34 and 8-bit pages 47 and 9.)
 template <class C, int D, int CT>
-__global__ __launch_bounds__(256, D > 128 && CT == 2 ? 1 : 2) void mixed_mfma(PrefillMfmaArgs p, DecodeMfmaArgs d,
-                                                                             int ndec) {
+__global__ __launch_bounds__(256, 2) void mixed_mfma(PrefillMfmaArgs p, DecodeMfmaArgs d, int ndec) {
   if ((int)blockIdx.x < ndec)
     decode_mfma_body<C, D>(d, blockIdx.x, ndec);
   else

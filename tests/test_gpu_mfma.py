@@ -276,6 +276,20 @@ def test_decode_infinities_in_cut_rows(cuda, kind, d, page):
     assert us2 < 8 * us + 50, (us, us2)
 
 
+@pytest.mark.parametrize("kind", ["f16", "fp8", "q4", "q8"])
+@pytest.mark.parametrize("d,hq,hkv", [(64, 128, 1), (64, 130, 2), (128, 72, 1), (256, 64, 1), (64, 4, 4)])
+def test_item_edges_and_many_heads(cuda, kind, d, hq, hkv):
+    """Contexts at the item edges of 4-bit pages (64 tokens a wave, 256 an item), up to 128 query heads per kv head
+    (one query token a tile, eight head groups in the decode)."""
+    print(f"[item edges {kind} d{d} {hq}/{hkv}]", flush=True)
+    kvl = [63, 64, 65, 255, 256, 257, 511, 513]
+    b = batch(kind, [1] * len(kvl), kvl, hq, hkv, d, 16, seed=d + hq)
+    check(b, run(b, cuda), expected(b))
+    lens = [(1, 257), (3, 65), (66, 256), (1, 1), (2, 64)]
+    b = batch(kind, [q for q, _ in lens], [k for _, k in lens], hq, hkv, d, 16, seed=d + hq)
+    check(b, run(b, cuda, decode=False), expected(b))
+
+
 @pytest.mark.parametrize("kind", ["f16", "bf16", "fp8", "q4", "q8"])
 @pytest.mark.parametrize("d,page,hq,hkv", [(64, 16, 14, 2), (128, 24, 6, 2), (128, 8, 40, 2), (256, 64, 4, 4)])
 @pytest.mark.parametrize("longest", [32, 33, 64, 65])
