@@ -31,8 +31,8 @@
 //
 // Bound by HBM.  Against decode_split and its merge (VALU dot products, single-element
 // loads, two launches), which ran these shapes before: batch 32, contexts of 512 to
-// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 66 us, FP8 (136 MB)
-// 330 -> 34 us; one context of 1024, D 64, fp16: 38.4 -> 11.2 us; 8-bit pages, D 256, 13
+// 4096, 8 kv heads, D 128, pages of 16: bf16 (311 MB) 121.7 -> 67 us, FP8 (136 MB)
+// 330 -> 39 us; one context of 1024, D 64, fp16: 38.4 -> 11.4 us; 8-bit pages, D 256, 13
 // contexts of 200 to 5000 (64 MB): 141 -> 30 us.  Slower than they: more than 1024 units of a few
 // tokens at D 256 (96 contexts of 3 to 16, 16 heads: bf16 19.5 / 23.9, 4-bit 22.1 / 26.6 us), 4-bit D 256
 // without GQA at 60 to 128 tokens (200 contexts of 16 heads 115 / 135).
@@ -308,7 +308,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
   // (No bool: the compiler kept the bytes that pad it as arrays in LDS, whose index needs the workgroup's
   // size from the dispatch packet in host memory, 7 us and more before the first product with all compute
   // units at it: 25 contexts of 8 to 17 tokens, bf16, D 64, 19.1 -> 7.4 us; batch 32 over FP8 pages of 16
-  // 46 -> 34.)
+  // 46.6 -> 38.7.)
   struct Item {
     int s, y, j, n, kl, st, tb;
     int has;  // inside the range

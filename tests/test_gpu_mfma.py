@@ -415,6 +415,26 @@ def test_ragged_many_tiles(cuda, kind, page, seqs, qlen, ctx, hq, hkv):
     assert (np.abs(got - exp) <= affine_bound(b, exp)).all()
 
 
+@pytest.mark.parametrize("kind,page,seqs,qlen,ctx,hq,hkv,rows", [
+    ("f16", 16, 1, 150, 1600, 64, 1, 3),                                    # 75 tiles: three parts
+    ("f16", 16, 1, 400, 1500, 64, 1, 1), ("bf16", 16, 2, 300, 700, 64, 1, 1),  # 200 and 300: two, in two and three places
+    ("f16", 16, 2, 700, 2700, 64, 1, 1), ("q4", 128, 2, 340, 2700, 128, 8, 1),  # 700, 688, long contexts: two
+    ("f16", 16, 3, 150, 1600, 64, 1, 80), ("q4", 128, 3, 150, 1600, 128, 8, 80)])  # the workgroup's scan, cut
+def test_ragged_parts(cuda, kind, page, seqs, qlen, ctx, hq, hkv, rows):
+    """Each number of parts and places a tile can have, beside single-token rows (80: more than 64 sequences)."""
+    print(f"[ragged parts {seqs}x{qlen}/{ctx} beside {rows} {kind} {hq}/{hkv}]", flush=True)
+    d = 128 if kind == "q4" else 64
+    ctxs = [ctx - 37 * i for i in range(seqs)]
+    b = batch(kind, [qlen] * seqs + [1] * rows, ctxs + [77] * rows, hq, hkv, d, page, seed=qlen + rows)
+    exp = expected(b)
+    for _ in range(2):  # the arrival counters are back at zero
+        got = run(b, cuda, decode=False)
+        if kind == "q4":
+            assert (np.abs(got - exp) <= affine_bound(b, exp)).all()
+        else:
+            check(b, got, exp)
+
+
 @pytest.mark.parametrize("kind,page,hq", [("f16", 16, 6), ("q4", 128, 8)])  # prefill_mfma, prefill_affine
 @pytest.mark.parametrize("seqs", [15, 16, 17, 33, 63, 64, 65, 130])
 def test_ragged_sequence_counts(cuda, kind, page, hq, seqs):
