@@ -780,58 +780,58 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeMfmaArgs& A, const 
       const int me = whole ? 0 : uru(bid + u - slot);
       if (!solo) {
 #pragma unroll
-      for (int rd = 0; rd < D / P::RD; ++rd) {
-        __syncthreads();  // (the previous combine has been read)
-        constexpr int BR = P::SB / (D / P::RD);  // sub-tiles of the round
-        float* xw = xo + (wv * 16 + col) * P::XS;
-        if constexpr (C::kAffine) {  // sub-tile b, row 4 jj + r: dim 16 b + 4 jj + r
-          if (col < nh) {
+        for (int rd = 0; rd < D / P::RD; ++rd) {
+          __syncthreads();  // (the previous combine has been read)
+          constexpr int BR = P::SB / (D / P::RD);  // sub-tiles of the round
+          float* xw = xo + (wv * 16 + col) * P::XS;
+          if constexpr (C::kAffine) {  // sub-tile b, row 4 jj + r: dim 16 b + 4 jj + r
+            if (col < nh) {
 #pragma unroll
-            for (int b = 0; b < BR; ++b) *reinterpret_cast<f32x4*>(xw + 16 * b + 4 * jj) = acc[rd * BR + b];
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int b = 0; b < BR; b += 4) {
-              const f32x4 x = {acc[rd * BR + b][r], acc[rd * BR + b + 1][r], acc[rd * BR + b + 2][r],
-                               acc[rd * BR + b + 3][r]};
-              if (col < nh) *reinterpret_cast<f32x4*>(xw + (4 * jj + r) * BR + b) = x;
+              for (int b = 0; b < BR; ++b) *reinterpret_cast<f32x4*>(xw + 16 * b + 4 * jj) = acc[rd * BR + b];
             }
-        }
-        if (rd == 0 && jj == 0 && col < nh) {
-          xml[(wv * 16 + col) * 2] = m_run;
-          xml[(wv * 16 + col) * 2 + 1] = l;
-        }
-        __syncthreads();
-        for (int e = tid; e < nh * (P::RD / 4); e += 256) {
-          const int h = e / (P::RD / 4), c = e % (P::RD / 4);
-          float M = -INFINITY;
-#pragma unroll
-          for (int w = 0; w < 4; ++w) M = fmaxf(M, xml[(w * 16 + h) * 2]);
-          f32x4 O = {0.f, 0.f, 0.f, 0.f};
-          float L = 0.f;
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const float mw = xml[(w * 16 + h) * 2];
-            const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-            O += *reinterpret_cast<const f32x4*>(xo + (w * 16 + h) * P::XS + 4 * c) * f;
-            L = fmaf(xml[(w * 16 + h) * 2 + 1], f, L);
-          }
-          // element 4 c + k of the round is dim SB * row + rd * BR + ..: contiguous in k
-          const int dim = C::kAffine ? rd * P::RD + 4 * c : (4 * c / BR) * P::SB + rd * BR + (4 * c) % BR;
-          if (whole) {
-            bad |= write4(O, L, out + (size_t)h * D + dim);
           } else {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) bad |= not_finite(O[k]);
-            store_f32x4(O, ro, (h * D + dim) * 4, me * A.hc * D * 4);
-            if (rd == 0 && c == 0)
-              __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{M, L}), rm, h * 8, me * A.hc * 8,
-                                                    kCoherent);
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+              for (int b = 0; b < BR; b += 4) {
+                const f32x4 x = {acc[rd * BR + b][r], acc[rd * BR + b + 1][r], acc[rd * BR + b + 2][r],
+                                 acc[rd * BR + b + 3][r]};
+                if (col < nh) *reinterpret_cast<f32x4*>(xw + (4 * jj + r) * BR + b) = x;
+              }
+          }
+          if (rd == 0 && jj == 0 && col < nh) {
+            xml[(wv * 16 + col) * 2] = m_run;
+            xml[(wv * 16 + col) * 2 + 1] = l;
+          }
+          __syncthreads();
+          for (int e = tid; e < nh * (P::RD / 4); e += 256) {
+            const int h = e / (P::RD / 4), c = e % (P::RD / 4);
+            float M = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) M = fmaxf(M, xml[(w * 16 + h) * 2]);
+            f32x4 O = {0.f, 0.f, 0.f, 0.f};
+            float L = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const float mw = xml[(w * 16 + h) * 2];
+              const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+              O += *reinterpret_cast<const f32x4*>(xo + (w * 16 + h) * P::XS + 4 * c) * f;
+              L = fmaf(xml[(w * 16 + h) * 2 + 1], f, L);
+            }
+            // element 4 c + k of the round is dim SB * row + rd * BR + ..: contiguous in k
+            const int dim = C::kAffine ? rd * P::RD + 4 * c : (4 * c / BR) * P::SB + rd * BR + (4 * c) % BR;
+            if (whole) {
+              bad |= write4(O, L, out + (size_t)h * D + dim);
+            } else {
+#pragma unroll
+              for (int k = 0; k < 4; ++k) bad |= not_finite(O[k]);
+              store_f32x4(O, ro, (h * D + dim) * 4, me * A.hc * D * 4);
+              if (rd == 0 && c == 0)
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{M, L}), rm, h * 8, me * A.hc * 8,
+                                                      kCoherent);
+            }
           }
         }
-      }
       }
       // ---- rows that are not finite over this workgroup's keys: again in fp32 (attend_row)
       const bool again = solo ? __any(bad) : __syncthreads_or(bad);
