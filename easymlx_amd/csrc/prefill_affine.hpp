@@ -134,7 +134,8 @@ __device__ __forceinline__ constexpr int pv_slot(int k) { return 8 * ((k & 15) >
 // us, without a prefix 48.4 -> 45.7; sixteen 256-token chunks 57.7 -> 55.7; prefill_mfma, two
 // 700-token chunks at head_dim 64 26.7 -> 24.0.  `rows`: query rows of the call; tiles past the
 // last one are not counted.
-// Places: where most tiles are cut, as many as their parts; else three also for two parts.  Workgroups go
+// Places: one where no context is longer than a part; where most tiles are cut, as many as their
+// parts; else three also for two parts.  Workgroups go
 // round the chip in turn, and tiles that use one place of two leave every other compute unit idle, although
 // the part that works changes place every other tile (bf16, GQA 7, four 514-token prompts 62 us, at three
 // places 44; four 230-token ones 25 / 23; 4-bit pages of 16, five 512-token chunks after up to 3000 tokens
@@ -145,8 +146,9 @@ struct TileItem {
   int total;
 
   template <class Rule>
-  __device__ __forceinline__ void set_places(int tiles, float keys, int bid, int Hkv, int grid_places) {
-    most = grid_places > 1 ? __builtin_amdgcn_readfirstlane(Rule::most_parts(tiles, keys)) : 1;
+  __device__ __forceinline__ void set_places(int tiles, float keys, bool any_long, int bid, int Hkv,
+                                             int grid_places) {
+    most = grid_places > 1 && any_long ? __builtin_amdgcn_readfirstlane(Rule::most_parts(tiles, keys)) : 1;
     const bool mostly_cut = __builtin_amdgcn_readfirstlane(keys >= 2.f * kPrefillSplitKeys);
     places = most == 1 ? 1 : most == 2 && mostly_cut ? 2 : grid_places;
     item = bid / Hkv / places;
@@ -171,11 +173,13 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
   r.total = __builtin_amdgcn_readlane(x, 63);
   const int tiles = r.total * Hkv;
   float keys = 0.f;
+  const int kvw = window > 0 ? min(kv, window) : kv;
+  const bool any_long = __any(n > 0 && kvw > kPrefillSplitKeys);
   // (the sum is worth 0.5 us; a window below every line needs none)
-  if (grid_places > 1 && tiles > Rule::kFew && tiles <= kPrefillCutTiles &&
+  if (grid_places > 1 && any_long && tiles > Rule::kFew && tiles <= kPrefillCutTiles &&
       (window <= 0 || window >= 2 * kPrefillSplitKeys))
-    keys = wave_sum((float)n * (float)(window > 0 ? min(kv, window) : kv)) / (float)r.total;
-  r.set_places<Rule>(tiles, keys, bid, Hkv, grid_places);
+    keys = wave_sum((float)n * (float)kvw) / (float)r.total;
+  r.set_places<Rule>(tiles, keys, any_long, bid, Hkv, grid_places);
   const int s = __builtin_popcountll(__ballot(x <= r.item));
   r.tile = -1;
   if (s > 63) return r;
@@ -187,7 +191,7 @@ __device__ __forceinline__ TileItem tile_item64(const int32_t* qsl, const int32_
   return r;
 }
 
-// The same for any number of sequences, scanned by the workgroup: tcum [S + 1] and wred [8] in LDS.
+// The same for any number of sequences, scanned by the workgroup: tcum [S + 1] and wred [12] in LDS.
 template <class Rule>
 __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int32_t* kv_lens, int S, int min_q, int tokb,
                                                   int window, int bid, int Hkv, int grid_places, int* tcum, int* wred,
@@ -196,12 +200,17 @@ __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int3
   const int ch = (S + 255) / 256, s0 = tid * ch;
   int tsum = 0;
   float ksum = 0.f;
+  bool any_long = false;
   for (int i = 0; i < ch; ++i) {
     const int si = s0 + i;
     if (si >= S) break;
     const int q0 = qsl[si], ql = qsl[si + 1] - q0;
     const int n = ql >= min_q ? (max(min(ql, rows - max(q0, 0)), 0) + tokb - 1) / tokb : 0;
-    if (n > 0) ksum += (float)n * (float)(window > 0 ? min(kv_lens[si], window) : kv_lens[si]);
+    if (n > 0) {
+      const int kvw = window > 0 ? min(kv_lens[si], window) : kv_lens[si];
+      ksum += (float)n * (float)kvw;
+      any_long = any_long || kvw > kPrefillSplitKeys;
+    }
     tcum[si] = n;  // the count for now
     tsum += n;
   }
@@ -212,14 +221,17 @@ __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int3
     if (lane >= o) x += y;
   }
   ksum = wave_sum(ksum);
+  any_long = __any(any_long);
   if (lane == 63) {
     wred[wv] = x;
     wred[4 + wv] = __float_as_int(ksum);
+    wred[8 + wv] = any_long;
   }
   __syncthreads();
   int base = 0;
   for (int w = 0; w < wv; ++w) base += wred[w];
   ksum = __int_as_float(wred[4]) + __int_as_float(wred[5]) + __int_as_float(wred[6]) + __int_as_float(wred[7]);
+  any_long = wred[8] | wred[9] | wred[10] | wred[11];
   int run = base + x - tsum;
   for (int i = 0; i < ch; ++i) {
     const int si = s0 + i;
@@ -232,7 +244,8 @@ __device__ __forceinline__ TileItem tile_item_any(const int32_t* qsl, const int3
   __syncthreads();
   TileItem r;
   r.total = __builtin_amdgcn_readfirstlane(tcum[S]);
-  r.set_places<Rule>(r.total * Hkv, ksum / (float)r.total, bid, Hkv, grid_places);
+  r.set_places<Rule>(r.total * Hkv, ksum / (float)r.total, __builtin_amdgcn_readfirstlane(any_long), bid, Hkv,
+                     grid_places);
   r.tile = -1;
   if (r.item >= r.total) return r;
   int s = 0;
@@ -273,13 +286,13 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int bid
   // ---- per-sequence tile counts, scanned by the whole workgroup (one pass of
   // global loads in parallel, not a serial walk by one thread)
   // LDS, carved from the shared arena
-  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oRawv = lds_next(oWred, 32);
+  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oRawv = lds_next(oWred, 48);
   constexpr int oRaws = lds_next(oRawv, RAWV), oKe = lds_next(oRaws, 2 * 4 * G * NT);
   constexpr int oVe = lds_next(oKe, 2 * NT * P::KSTR), oKsf = lds_next(oVe, 2 * D * P::VSTR);
   constexpr int oKbe = lds_next(oKsf, 4 * G * NT), oEnd = lds_next(oKbe, 16 * NT);
   static_assert(oEnd <= kArenaBytes, "LDS arena too small");
   int(&tcum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oTcum);
-  int(&wred)[8] = lds_at<int[8]>(oWred);
+  int(&wred)[12] = lds_at<int[12]>(oWred);
   const int kvh = bid % a.Hkv;
   const TileItem ti =
       a.S <= 64 ? tile_item64<PrefillRule>(a.qsl, a.kv_lens, a.S, a.min_q, P::TOKB, a.window, bid, a.Hkv, a.places)

@@ -168,13 +168,13 @@ __device__ __forceinline__ void prefill_mfma_body(const PrefillMfmaArgs& A, cons
     if constexpr (C::kAffine) return P::G;
     return 1;
   }();
-  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oKe = lds_next(oWred, 32);
+  constexpr int oTcum = 0, oWred = lds_next(oTcum, 4 * (kMaxSeqs + 1)), oKe = lds_next(oWred, 48);
   constexpr int oVe = lds_next(oKe, 2 * NT * P::KSTR), oKsf = lds_next(oVe, 2 * (AFF ? D : NT) * P::VSTR);
   constexpr int oVsf = lds_next(oKsf, 4 * G * NT), oVbf = lds_next(oVsf, 4 * G * NT);
   constexpr int oKbe = lds_next(oVbf, AFF ? 4 * G * NT : 0), oEnd = lds_next(oKbe, AFF ? 16 * NT : 0);
   static_assert(oEnd <= kArenaBytes, "LDS arena too small");
   int(&tcum)[kMaxSeqs + 1] = lds_at<int[kMaxSeqs + 1]>(oTcum);
-  int(&wred)[8] = lds_at<int[8]>(oWred);
+  int(&wred)[12] = lds_at<int[12]>(oWred);
   uint16_t* ke = &lds_at<uint16_t>(oKe);  // [key][KSTR]
   uint16_t* ve = &lds_at<uint16_t>(oVe);  // [key][VSTR]; affine: [dim][VSTR]
   float* ksf = &lds_at<float>(oKsf);      // key scale of each key; affine: [group][NT], * 2^kCodeExp
